@@ -287,6 +287,24 @@ int swc_plan_export(const swc_plan* p, int which, void* dst);
 /* Byte sizes of the exported structs {Panel, Tile, Task, SolveBlock}. */
 int swc_plan_struct_sizes(int64_t* out);
 
+/* The multifrontal plan the default factorization runs (csrc/fronts.h), host only.
+ * A2 = tril(P A P^T) as in swc_upload, entry e holding value e; rlb as in
+ * swc_set_plan_params.  Fails where the structure has no front tree (the
+ * factorization then runs the left-looking plan).  sizes[13] = {levels, arena
+ * doubles, diagonal scratch doubles, gathers, entries of A, factor tiles, small
+ * fronts, update tiles, byte sizes of the structs Gather, AEntry, FactorTile,
+ * SmallFront, FrontTile}; swc_front_plan_export copies array `which`: 0 gathers, 1
+ * entries of A, 2 factor tiles, 3 level->factor-tile offsets, 4 per level: tiles of
+ * panels of <= 16 columns, 5 small fronts, 6 level->small-front offsets, 7 update
+ * tiles, 8 level->update-tile offsets, 9 per level: deferred tiles. */
+typedef struct swc_front_plan swc_front_plan;
+int swc_front_plan_build(int n, const int* blockSet, int supNo, const size_t* lC, const int* Ls,
+                         const size_t* Li_ptr, const int* prunePtr, const int* pruneSet,
+                         const int* A2p, const int* A2i, int rlb, swc_front_plan** out);
+void swc_front_plan_free(swc_front_plan* p);
+int swc_front_plan_sizes(const swc_front_plan* p, int64_t* sizes);
+int swc_front_plan_export(const swc_front_plan* p, int which, void* dst);
+
 #ifdef __cplusplus
 }
 #endif

@@ -414,3 +414,46 @@ def build_plan(bcsc: BCSC, derive_sets=False, params=None, schedule=None):
         return out
     finally:
         lib.swc_plan_free(h)
+
+
+GATHER_DT = np.dtype([("src", np.int64), ("ld", np.int32), ("pad", np.int32),
+                      ("rmask", np.uint64), ("cmask", np.uint64)])
+AENTRY_DT = np.dtype([("q", np.int32), ("pos", np.int32)])
+FACTOR_TILE_DT = np.dtype([("vbase", np.int64)] + [(k, np.int32) for k in (
+    "r0", "nr", "kind", "slot", "ld", "ncol", "c0", "first", "g0", "g1", "a0", "a1", "dg0", "dg1",
+    "da0", "da1")])
+SMALL_FRONT_DT = np.dtype([("vbase", np.int64), ("ubase", np.int64)] + [(k, np.int32) for k in (
+    "R", "w", "ldu", "c0", "g0", "g1", "a0", "a1")])
+FRONT_TILE_DT = np.dtype([("vbase", np.int64), ("asrc", np.int64), ("bsrc", np.int64)] + [
+    (k, np.int32) for k in ("ld", "sld", "k", "nr", "nc", "diag", "first", "upd", "g0", "g1", "a0",
+                            "a1", "slot", "pad")])
+
+
+def build_fronts(bcsc: BCSC, rlb=8):
+    """The multifrontal plan of a structure (csrc/fronts.h), as numpy record arrays
+    (host only); entries of A count in A2 order."""
+    lib = _lib.lib()
+    h = ctypes.c_void_p()
+    arrs = [np.ascontiguousarray(bcsc.super), np.ascontiguousarray(bcsc.p.astype(np.uint64)),
+            np.ascontiguousarray(bcsc.i_ptr.astype(np.uint64))]
+    check(lib.swc_front_plan_build(bcsc.n, ptr(arrs[0]), bcsc.nsuper, ptr(arrs[1]), ptr(bcsc.s),
+                                   ptr(arrs[2]), ptr(bcsc.prunePtr), ptr(bcsc.pruneSet),
+                                   ptr(bcsc.a2p), ptr(bcsc.a2i), int(rlb), ctypes.byref(h)))
+    try:
+        sz = np.zeros(13, dtype=np.int64)
+        check(lib.swc_front_plan_sizes(h, ptr(sz)))
+        nl, usize, dscr, ng, na, nf, ns, nu = (int(v) for v in sz[:8])
+        dts = [GATHER_DT, AENTRY_DT, FACTOR_TILE_DT, SMALL_FRONT_DT, FRONT_TILE_DT]
+        if [d.itemsize for d in dts] != [int(v) for v in sz[8:]]:
+            raise RuntimeError(f"front plan struct layout mismatch: library {list(sz[8:])}")
+        spec = [("gathers", dts[0], ng), ("aents", dts[1], na), ("ftiles", dts[2], nf),
+                ("lvl_f", np.int32, nl + 1), ("lvl_fn", np.int32, nl), ("small", dts[3], ns),
+                ("lvl_small", np.int32, nl + 1), ("utiles", dts[4], nu), ("lvl_u", np.int32, nl + 1),
+                ("lvl_ud", np.int32, nl)]
+        out = {"nlevel": nl, "usize": usize, "diag_scratch": dscr}
+        for which, (name, dt, cnt) in enumerate(spec):
+            out[name] = np.zeros(cnt, dtype=dt)
+            check(lib.swc_front_plan_export(h, which, ptr(out[name])))
+        return out
+    finally:
+        lib.swc_front_plan_free(h)

@@ -21,6 +21,7 @@
 
 #include "analysis.h"
 #include "capi_common.h"
+#include "fronts.h"
 #include "plan.h"
 
 using swc::Panel;
@@ -370,16 +371,12 @@ __device__ inline double bcast(double v, int src) {
 // waits for another; the diagonal tile stores it and reports info.  Entries
 // above the diagonal of the register copy are never read by lanes on or below
 // it, so they are left unmasked.
-template <int NC>
-__device__ inline void panel_factor_regs_body(double* __restrict__ L, const Tile& tl,
-                                              const double* __restrict__ dscratch,
+template <int NC, class TileT>
+__device__ inline void panel_factor_regs_core(double* __restrict__ L, const TileT& tl,
                                               int* __restrict__ info_out, float* __restrict__ Lf,
-                                              int lane) {
+                                              int lane, double (&y)[NC], double (&x)[NC]) {
+  // y: row `lane` of the diagonal block; x: row `lane` of the tile
   const int nr = tl.nr, nc = tl.ncol;
-  const double* gdiag = dscratch + tl.slot;  // updated diagonal block, ld nc
-  double y[NC];                              // row `lane` of the diagonal block
-#pragma unroll
-  for (int c = 0; c < NC; ++c) y[c] = (lane < nc && c < nc && c <= lane) ? gdiag[c * nc + lane] : 0.0;
   int badcol = 0;
 #pragma unroll
   for (int j = 0; j < NC; ++j) {
@@ -413,9 +410,6 @@ __device__ inline void panel_factor_regs_body(double* __restrict__ L, const Tile
   // rows of this tile below the diagonal block: tile rows [first, nr)
   const int first = tl.kind == 0 ? nc : 0;
   const bool mine = lane >= first && lane < nr;
-  double x[NC];
-#pragma unroll
-  for (int c = 0; c < NC; ++c) x[c] = (mine && c < nc) ? gtile[(int64_t)c * tl.ld + lane] : 0.0;
 #pragma unroll
   for (int j = 0; j < NC; ++j) {
     if (j < nc) {
@@ -431,6 +425,24 @@ __device__ inline void panel_factor_regs_body(double* __restrict__ L, const Tile
       gtile[(int64_t)c * tl.ld + lane] = x[c];
       if (ftile) ftile[(int64_t)c * tl.ld + lane] = (float)x[c];
     }
+}
+
+template <int NC>
+__device__ inline void panel_factor_regs_body(double* __restrict__ L, const Tile& tl,
+                                              const double* __restrict__ dscratch,
+                                              int* __restrict__ info_out, float* __restrict__ Lf,
+                                              int lane) {
+  const int nc = tl.ncol, first = tl.kind == 0 ? nc : 0;
+  const double* gdiag = dscratch + tl.slot;  // updated diagonal block, ld nc
+  const double* gtile = L + tl.vbase + tl.r0;
+  const bool mine = lane >= first && lane < tl.nr;
+  double y[NC], x[NC];
+#pragma unroll
+  for (int c = 0; c < NC; ++c) {
+    y[c] = (lane < nc && c < nc && c <= lane) ? gdiag[c * nc + lane] : 0.0;
+    x[c] = (mine && c < nc) ? gtile[(int64_t)c * tl.ld + lane] : 0.0;
+  }
+  panel_factor_regs_core<NC>(L, tl, info_out, Lf, lane, y, x);
 }
 
 template <int NC>
@@ -631,22 +643,37 @@ __device__ inline d4 lds_block_update(const double* __restrict__ W, d4 acc, int 
 // LDS of k_panel_factor_blk: W, then per sweeping wave column j's multipliers
 constexpr int kBlkLds = swc::PW * kWld + 3 * 16 * 16;
 
-__device__ inline void panel_factor_blk_body(double* __restrict__ L, const Tile& tl,
+struct FrontIn;
+__device__ inline void front_assemble_blk(const double* L, const swc::FactorTile& tl,
+                                          const FrontIn& in, double* W, int first, int nx, int nb,
+                                          int wave, int lane);
+
+// In: nothing for the left-looking tiles (Tile), what a first panel is assembled from
+// for the multifrontal ones (FactorTile).
+template <class TileT, class... In>
+__device__ inline void panel_factor_blk_body(double* __restrict__ L, const TileT& tl,
                                              const double* __restrict__ dscratch,
                                              int* __restrict__ info_out, float* __restrict__ Lf,
-                                             double* lds, int tid) {
-  double* W = lds;
-  double(*lc)[16][16] = reinterpret_cast<double(*)[16][16]>(lds + swc::PW * kWld);
+                                             double* lds, int tid, const In&... in) {
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int nc = tl.ncol;
   const int nb = (nc + 15) >> 4;              // 16-column blocks (2..4)
+  double(*lc)[16][16] = reinterpret_cast<double(*)[16][16]>(lds);
+  double* W = lds + 3 * 16 * 16;              // 16 nb columns
   const int first = tl.kind == 0 ? nc : 0;    // tile rows [first, nr) are solved ...
   const int nx = tl.nr > first ? tl.nr - first : 0;  // ... into W rows 64 .. 64 + nx
   const int nxb = (nx + 15) >> 4;
   const double* gdiag = dscratch + tl.slot;  // updated diagonal block, ld nc
   double* gtile = L + tl.vbase + tl.r0;
   float* ftile = Lf ? Lf + tl.vbase + tl.r0 : nullptr;
-  {
+  bool load = true;
+  if constexpr (sizeof...(In) > 0) {
+    if (tl.first) {
+      front_assemble_blk(L, tl, in..., W, first, nx, nb, wave, lane);
+      load = false;
+    }
+  }
+  if (load) {
     // wave w moves columns 16w..16w+15 of diagonal-block row `lane` and of tile
     // row `lane`; every lane loads from an address inside both buffers and then
     // selects, so all its loads are in flight together
@@ -982,6 +1009,8 @@ k_factor_and_update(double* __restrict__ L, const Tile* __restrict__ ftiles, int
     tile_update_body<MODE>(L, tl, tasks, dscratch, Lf_update, lds, threadIdx.x);
   }
 }
+
+#include "front_kernels.h"
 
 // CSC export of the factor (the layout of the reference's bcsc2csc,
 // common/Util.h:311-338): column j's entries are its supernode's rows from its
@@ -2026,6 +2055,8 @@ struct swc_handle {
   Plan plan;
   swc::PlanParams params;  // shape parameters of the next structure upload
   swc::HLevelSchedule hlevel;  // non-empty: factor levels follow this schedule
+  bool multifrontal = false;   // the factor runs the front plan, else the left-looking one
+  swc::FrontPlan fronts;
   int n = 0, nsuper = 0;
   int64_t nvals = 0;  // number of values swc_factor expects
   std::vector<int> super, Ls;
@@ -2053,6 +2084,11 @@ struct swc_handle {
   int* dOrder = nullptr;
   Tile* dFtiles = nullptr;  // factor-kernel tiles (copies), by level and width class
   swc::FusedPanel* dFused = nullptr;  // fused narrow panels, by level
+  swc::Gather* dGathers = nullptr;    // the front plan's lists (fronts.h)
+  swc::AEntry* dAents = nullptr;
+  swc::FactorTile* dFactorTiles = nullptr;
+  swc::SmallFront* dSmall = nullptr;
+  swc::FrontTile* dFrontTiles = nullptr;
   int* dCounters = nullptr;  // per level: the fused kernel's worklist counter
   int fused_cap[3] = {0, 0, 0};  // per precision mode: fused-kernel workgroups resident at once
   swc::DagItem* dDagItems = nullptr;  // dependency-driven launch: work items, dependencies,
@@ -2132,14 +2168,16 @@ struct swc_handle {
   void release() {
     drop_graphs();
     (void)hipFree(dL); (void)hipFree(dLf); (void)hipFree(dLs); (void)hipFree(dPanels); (void)hipFree(dTiles); (void)hipFree(dTasks);
-    (void)hipFree(dGptr); (void)hipFree(dGidx); (void)hipFree(dGcols); (void)hipFree(dFblk); (void)hipFree(dFblkPtr); (void)hipFree(dV); (void)hipFree(dPb); (void)hipFree(dY); (void)hipFree(dSpanels); (void)hipFree(dSpOrder); (void)hipFree(dOrder); (void)hipFree(dFtiles); (void)hipFree(dFused); (void)hipFree(dCounters); (void)hipFree(dDagItems); (void)hipFree(dDagDeps); (void)hipFree(dDagSync); (void)hipFree(dDiag); (void)hipFree(dAmap); (void)hipFree(dPerm);
+    (void)hipFree(dGptr); (void)hipFree(dGidx); (void)hipFree(dGcols); (void)hipFree(dFblk); (void)hipFree(dFblkPtr); (void)hipFree(dV); (void)hipFree(dPb); (void)hipFree(dY); (void)hipFree(dSpanels); (void)hipFree(dSpOrder); (void)hipFree(dOrder); (void)hipFree(dFtiles); (void)hipFree(dFused);
+    (void)hipFree(dGathers); (void)hipFree(dAents); (void)hipFree(dFactorTiles); (void)hipFree(dSmall); (void)hipFree(dFrontTiles);
+    (void)hipFree(dCounters); (void)hipFree(dDagItems); (void)hipFree(dDagDeps); (void)hipFree(dDagSync); (void)hipFree(dDiag); (void)hipFree(dAmap); (void)hipFree(dPerm);
     (void)hipFree(dVals); (void)hipFree(dWork); (void)hipFree(dInfo);
     (void)hipFree(dRp); (void)hipFree(dCi); (void)hipFree(dVmap); (void)hipFree(dAf); (void)hipFree(dNorm); (void)hipFree(dScal); (void)hipFree(dPart); (void)hipFree(dNormPart);
     (void)hipFree(dRef);
     (void)hipFree(dZ); (void)hipFree(dArena); (void)hipFree(dNodes); (void)hipFree(dCol2sup); (void)hipFree(dSpx);
     (void)hipFree(dSsuper); (void)hipFree(dSpi); (void)hipFree(dDiagPos); (void)hipFree(dQi); (void)hipFree(dQj);
     dL = nullptr; dLf = nullptr; dLs = nullptr; dPanels = nullptr; dTiles = nullptr; dTasks = nullptr;
-    dGptr = nullptr; dGidx = nullptr; dGcols = nullptr; dFblk = nullptr; dFblkPtr = nullptr; dV = nullptr; dPb = nullptr; dY = nullptr; dSpanels = nullptr; dSpOrder = nullptr; dOrder = nullptr; dFtiles = nullptr; dFused = nullptr; dCounters = nullptr; dDagItems = nullptr; dDagDeps = nullptr; dDagSync = nullptr; dDiag = nullptr; dAmap = nullptr; dPerm = nullptr;
+    dGptr = nullptr; dGidx = nullptr; dGcols = nullptr; dFblk = nullptr; dFblkPtr = nullptr; dV = nullptr; dPb = nullptr; dY = nullptr; dSpanels = nullptr; dSpOrder = nullptr; dOrder = nullptr; dFtiles = nullptr; dFused = nullptr; dGathers = nullptr; dAents = nullptr; dFactorTiles = nullptr; dSmall = nullptr; dFrontTiles = nullptr; dCounters = nullptr; dDagItems = nullptr; dDagDeps = nullptr; dDagSync = nullptr; dDiag = nullptr; dAmap = nullptr; dPerm = nullptr;
     dVals = nullptr; dWork = nullptr; dInfo = nullptr;
     dRp = nullptr; dCi = nullptr; dVmap = nullptr; dAf = nullptr; dNorm = nullptr; dScal = nullptr; dPart = nullptr; dNormPart = nullptr;
     lf_cap = 0;
@@ -2169,32 +2207,43 @@ int upload(T** dst, const T* src, size_t count, hipStream_t s) {
 
 int grid_for(int64_t n) { return (int)std::max<int64_t>(1, std::min<int64_t>((n + kThreads - 1) / kThreads, 65536)); }
 
-// Value offset inside L of every entry of tril(P A P^T) given as CSC (a2p, a2i).
-// With src != null, entry e of A2 came from input entry src[e] and the map is
-// indexed by input entries (so swc_factor takes values in the caller's order).
-int build_amap(const swc_handle* h, const int* a2p, const int* a2i, const int64_t* src,
-               int64_t nvals, std::vector<int64_t>& amap) {
+// Position of every entry of tril(P A P^T), given as CSC (a2p, a2i), in the row list of
+// its column's supernode; false for bad pointers or an entry outside the structure.
+bool a2_positions(const swc_handle* h, const int* a2p, const int* a2i, std::vector<int>& pos) {
+  if (!a2p || !a2i || a2p[0] != 0) return false;
+  for (int j = 0; j < h->n; ++j)
+    if (a2p[j + 1] < a2p[j]) return false;
+  pos.resize((size_t)a2p[h->n]);
+  for (int s = 0; s < h->nsuper; ++s) {
+    const int* rows = h->Ls.data() + h->pi[s];
+    const int len = (int)(h->pi[s + 1] - h->pi[s]);
+    for (int j = h->super[s]; j < h->super[s + 1]; ++j)
+      for (int64_t q = a2p[j]; q < a2p[j + 1]; ++q) {
+        const int k = int(std::lower_bound(rows, rows + len, a2i[q]) - rows);
+        if (a2i[q] < j || k >= len || rows[k] != a2i[q]) return false;
+        pos[q] = k;
+      }
+  }
+  return true;
+}
+
+// Value offset inside L of every entry of A2 (at row positions pos).  With src != null,
+// entry e of A2 came from input entry src[e] and the map is indexed by input entries (so
+// swc_factor takes values in the caller's order).
+int build_amap(const swc_handle* h, const int* a2p, const std::vector<int>& pos,
+               const int64_t* src, int64_t nvals, std::vector<int64_t>& amap) {
   const int n = h->n;
   const int64_t nnz = a2p[n];
   amap.assign(src ? nvals : nnz, -1);
-  std::vector<int> col2sup(n);
-  for (int s = 0; s < h->nsuper; ++s)
-    for (int c = h->super[s]; c < h->super[s + 1]; ++c) col2sup[c] = s;
-  for (int j = 0; j < n; ++j) {
-    const int s = col2sup[j];
-    const int* rows = h->Ls.data() + h->pi[s];
-    const int len = (int)(h->pi[s + 1] - h->pi[s]);
-    for (int64_t q = a2p[j]; q < a2p[j + 1]; ++q) {
-      const int r = a2i[q];
-      const int pos = int(std::lower_bound(rows, rows + len, r) - rows);
-      if (r < j || pos >= len || rows[pos] != r)
-        return swc_set_error(SWC_EINVAL, "A2 entry outside the structure of L");
-      const int64_t off = h->px[s] + (int64_t)(j - h->super[s]) * len + pos;
-      const int64_t dst = src ? src[q] : q;
-      if (dst < 0 || dst >= (int64_t)amap.size())
-        return swc_set_error(SWC_EINVAL, "value map index out of range");
-      amap[dst] = off;
-    }
+  for (int s = 0; s < h->nsuper; ++s) {
+    const int64_t len = h->pi[s + 1] - h->pi[s];
+    for (int j = h->super[s]; j < h->super[s + 1]; ++j)
+      for (int64_t q = a2p[j]; q < a2p[j + 1]; ++q) {
+        const int64_t dst = src ? src[q] : q;
+        if (dst < 0 || dst >= (int64_t)amap.size())
+          return swc_set_error(SWC_EINVAL, "value map index out of range");
+        amap[dst] = h->px[s] + (j - h->super[s]) * len + pos[q];
+      }
   }
   for (int64_t v : amap)
     if (v < 0) return swc_set_error(SWC_EINVAL, "value map does not cover every value");
@@ -2227,11 +2276,64 @@ int ensure_work(swc_handle* h, int cols) {
   return SWC_OK;
 }
 
+// The multifrontal factorization's levels (fronts.h): F_l, then U_l.
+template <int MODE>
+void enqueue_fronts(swc_handle* h, bool profile) {
+  hipStream_t st = h->stream;
+  const swc::FrontPlan& F = h->fronts;
+  const FrontIn in{h->dGathers, h->dAents, h->dVals};
+  float* lf = MODE ? h->dLf : nullptr;
+  const swc::SmallFront* sm = h->dSmall;
+  const swc::FactorTile* ft = h->dFactorTiles;
+  const swc::FrontTile* ut = h->dFrontTiles;
+  for (int l = 0; l < F.nlevel; ++l) {
+    hipEvent_t* pe = profile ? &h->pev[(size_t)4 * l] : nullptr;
+    const int s0 = F.lvl_small[l], ns = F.lvl_small[l + 1] - s0;
+    const int f0 = F.lvl_f[l], nf = F.lvl_f[l + 1] - f0, nn = F.lvl_fn[l], nw = nf - nn;
+    const int nd = l > 0 && !profile ? F.lvl_ud[l - 1] : 0;
+    if (pe) (void)hipEventRecord(pe[1], st);
+    // many one-wave items keep their own launch, where more of them fit on a CU
+    const bool lean = nw + nd == 0 || ns + nn > 2048;
+    if (lean && ns + nn > 0)
+      hipLaunchKernelGGL(k_front_narrow<MODE>, dim3(ns + nn), dim3(64), 0, st, h->dL, sm, s0, ns,
+                         ft, f0, in, (const double*)h->dDiag, h->dInfo, lf);
+    if (nw + nd > 0) {
+      const int s1 = lean ? 0 : ns, n1 = lean ? 0 : nn;
+      hipLaunchKernelGGL(k_front_factor<MODE>, dim3((s1 + 3) / 4 + (n1 + 3) / 4 + nw + nd),
+                         dim3(kThreads), front_factor_lds(s1 + n1, F.lvl_widest[l], nd), st, h->dL,
+                         sm, s0, s1, ft, f0 + nn - n1, n1, nw, ut,
+                         F.lvl_u[l] - nd, in, (const double*)h->dDiag, h->dDiag,
+                         h->dInfo, lf, (const float*)h->dLf);
+    }
+    if (pe) (void)hipEventRecord(pe[2], st);
+    const int u0 = F.lvl_u[l], nu = F.lvl_u[l + 1] - u0 - (profile ? 0 : F.lvl_ud[l]);
+    if (nu > 0)
+      hipLaunchKernelGGL(k_front_update<MODE>, dim3(nu), dim3(kThreads), 0, st, h->dL, ut, u0, in,
+                         h->dDiag, (const float*)h->dLf);
+    if (pe) (void)hipEventRecord(pe[3], st);
+  }
+}
+
 // Enqueues the whole numeric factorization of the staged values h->dVals.
 void enqueue_factor(swc_handle* h, bool profile) {
   hipStream_t st = h->stream;
   const Plan& P = h->plan;
   const double* dvals = h->dVals;
+  if (h->multifrontal) {
+    // L needs no clearing: every entry on and below a diagonal block's diagonal is
+    // written by a factor launch, and what lies above is cleared at upload
+    hipLaunchKernelGGL(k_gather, dim3(grid_for(h->nnz_full)), dim3(kThreads), 0, st, h->dAf, dvals,
+                       (const int64_t*)h->dVmap, h->nnz_full);
+    hipLaunchKernelGGL(k_norm_inf, dim3(kRedBlocks), dim3(kThreads), 0, st, (const int*)h->dRp,
+                       (const double*)h->dAf, h->n, h->dNormPart);
+    hipLaunchKernelGGL(k_reduce_final, dim3(1), dim3(kThreads), 0, st,
+                       (const double*)h->dNormPart, 0, h->dNorm);
+    hipLaunchKernelGGL(k_set_int, dim3(1), dim3(1), 0, st, h->dInfo, 0x7fffffff);
+    if (h->precision == 0) enqueue_fronts<0>(h, profile);
+    else if (h->precision == 1) enqueue_fronts<1>(h, profile);
+    else enqueue_fronts<2>(h, profile);
+    return;
+  }
   hipLaunchKernelGGL(k_fill, dim3(grid_for(P.xsize)), dim3(kThreads), 0, st, h->dL, P.xsize, 0.0);
   hipLaunchKernelGGL(k_assemble, dim3(grid_for(h->nvals)), dim3(kThreads), 0, st, h->dL,
                      (const int64_t*)h->dAmap, dvals, h->nvals);
@@ -2333,9 +2435,10 @@ int factor_device(swc_handle* h, const double* dvals) {
   const Plan& P = h->plan;
   if (dvals != h->dVals)
     SWC_HIP(hipMemcpyAsync(h->dVals, dvals, sizeof(double) * h->nvals, hipMemcpyDeviceToDevice, st));
-  if (h->profile && h->pev.size() < (size_t)4 * P.nlevel) {
+  const int nlevel = h->multifrontal ? h->fronts.nlevel : P.nlevel;
+  if (h->profile && h->pev.size() < (size_t)4 * nlevel) {
     for (auto& e : h->pev) (void)hipEventDestroy(e);
-    h->pev.assign((size_t)4 * P.nlevel, nullptr);
+    h->pev.assign((size_t)4 * nlevel, nullptr);
     for (auto& e : h->pev) SWC_HIP(hipEventCreate(&e));
   }
   const bool graph = h->use_graphs && !h->profile;
@@ -2380,13 +2483,16 @@ int factor_device(swc_handle* h, const double* dvals) {
   if (h->profile) {
     h->t_tile_ms = h->t_trsm_ms = 0;
     h->n_tile = h->n_trsm = 0;
-    h->lvl_tile_ms.assign(P.nlevel, 0.0);
-    for (int l = 0; l < P.nlevel; ++l) {
-      const int nt = P.lvl_tiles[l + 1] - P.lvl_tiles[l];
-      const int ns = P.lvl_trsm[l + 1] - P.lvl_trsm[l];
+    h->lvl_tile_ms.assign(nlevel, 0.0);
+    for (int l = 0; l < nlevel; ++l) {
+      // the events around the level's update launch and around its factor launches
+      const swc::FrontPlan& F = h->fronts;
+      const bool mf = h->multifrontal;
+      const int nt = mf ? F.lvl_u[l + 1] - F.lvl_u[l] : P.lvl_tiles[l + 1] - P.lvl_tiles[l];
+      const int ns = mf ? 1 : P.lvl_trsm[l + 1] - P.lvl_trsm[l];
       hipEvent_t* pe = &h->pev[(size_t)4 * l];
       if (nt > 0) {
-        SWC_HIP(hipEventElapsedTime(&ms, pe[0], pe[1]));
+        SWC_HIP(hipEventElapsedTime(&ms, mf ? pe[2] : pe[0], mf ? pe[3] : pe[1]));
         h->t_tile_ms += ms;
         h->lvl_tile_ms[l] = ms;
         h->n_tile++;
@@ -2813,11 +2919,37 @@ int validate_structure(int n, const int* blockSet, int supNo, const size_t* lC, 
   return SWC_OK;
 }
 
-// Structure part of an upload: the plan (solve part only without `factor`), L
-// and its FP32 copy, the row lists and the plan arrays on the device.
+// What a factorization needs of A2: its pattern, and its entries' row positions.
+struct A2Pattern {
+  const int* p;
+  const int* i;
+  const int64_t* src;
+  int64_t nvals;
+  std::vector<int> pos;
+  bool ok = false;  // pos is valid
+};
+
+// Every input value is used once: the condition under which the entry lists of the front
+// plan and the value map agree (build_amap refuses the rest).
+bool covers_values(const A2Pattern& a, int n) {
+  if (!a.src) return true;
+  if (a.nvals != a.p[n]) return false;
+  std::vector<char> seen((size_t)a.nvals, 0);
+  for (int e = 0; e < a.p[n]; ++e) {
+    if (a.src[e] < 0 || a.src[e] >= a.nvals || seen[a.src[e]]) return false;
+    seen[a.src[e]] = 1;
+  }
+  return true;
+}
+
+// Structure part of an upload: the plan (solve part only without A2), L and its FP32
+// copy, the row lists and the plan arrays on the device.  The factorization runs the
+// multifrontal plan (fronts.h) where the structure has one and its arena fits the
+// device, else, and for an H-level schedule, the left-looking one (plan.h).
 int upload_structure(swc_handle* h, int n, const int* blockSet, int supNo, const size_t* lC,
                      const int* Ls, const size_t* Li_ptr, const int* prunePtr,
-                     const int* pruneSet, bool factor) {
+                     const int* pruneSet, A2Pattern* a2) {
+  const bool factor = a2 != nullptr;
   if (int rc = validate_structure(n, blockSet, supNo, lC, Ls, Li_ptr)) return rc;
   // pruneSet may be null when it is empty (no supernode has descendants)
   if (!prunePtr || (!pruneSet && prunePtr[supNo] != 0) || prunePtr[0] != 0)
@@ -2845,19 +2977,55 @@ int upload_structure(swc_handle* h, int n, const int* blockSet, int supNo, const
   h->Ls.assign(Ls, Ls + ssize);
   h->pruneptr.assign(prunePtr, prunePtr + supNo + 1);
   h->pruneset.assign(pruneSet, pruneSet + prunePtr[supNo]);
-  try {
+  h->multifrontal = false;
+  h->fronts = swc::FrontPlan();
+  auto plan = [&](bool left_looking) {
     swc::build_plan(n, supNo, h->super.data(), h->pi.data(), h->px.data(), h->Ls.data(),
-                    prunePtr, pruneSet, h->plan, factor, h->params,
+                    prunePtr, pruneSet, h->plan, left_looking, h->params,
                     h->hlevel.level_ptr.empty() ? nullptr : &h->hlevel);
+  };
+  hipStream_t st = h->stream;
+  int rc = SWC_OK;
+  try {
+    if (factor) a2->ok = a2_positions(h, a2->p, a2->i, a2->pos);
+    int64_t xsize = 0;
+    for (int s = 0; s < supNo; ++s)
+      xsize = std::max(xsize, h->px[s] + (h->pi[s + 1] - h->pi[s]) * (h->super[s + 1] - h->super[s]));
+    h->multifrontal =
+        factor && a2->ok && h->hlevel.level_ptr.empty() && covers_values(*a2, n) &&
+        swc::build_fronts(n, supNo, h->super.data(), h->pi.data(), h->px.data(), xsize,
+                          h->Ls.data(), prunePtr, pruneSet, a2->p, a2->src, a2->pos.data(),
+                          h->params.rlb, h->fronts);
+    plan(factor && !h->multifrontal);
+    if (h->multifrontal) {
+      // the arena follows L in one allocation
+      rc = upload(&h->dL, (const double*)nullptr, (size_t)(h->plan.xsize + h->fronts.usize), st);
+      if (rc && h->fronts.usize > 0) {
+        (void)hipGetLastError();
+        h->multifrontal = false;
+        plan(true);
+      } else if (!rc) {
+        // above the diagonal blocks' diagonals L is never written
+        hipLaunchKernelGGL(k_fill, dim3(grid_for(h->plan.xsize)), dim3(kThreads), 0, st, h->dL,
+                           h->plan.xsize, 0.0);
+      }
+    }
+    if (!h->multifrontal) {
+      h->fronts = swc::FrontPlan();
+      rc = upload(&h->dL, (const double*)nullptr, (size_t)h->plan.xsize, st);
+    }
   } catch (const std::bad_alloc&) {
     return swc_set_error(SWC_ENOMEM, "upload: out of host memory");
   } catch (const std::exception& e) {
     return swc_set_error(SWC_EINVAL, std::string("upload: ") + e.what());
   }
   const Plan& P = h->plan;
-  hipStream_t st = h->stream;
-  int rc = SWC_OK;
-  if (!rc) rc = upload(&h->dL, (const double*)nullptr, (size_t)P.xsize, st);
+  const swc::FrontPlan& F = h->fronts;
+  if (!rc) rc = upload(&h->dGathers, F.gathers.data(), F.gathers.size(), st);
+  if (!rc) rc = upload(&h->dAents, F.aents.data(), F.aents.size(), st);
+  if (!rc) rc = upload(&h->dFactorTiles, F.ftiles.data(), F.ftiles.size(), st);
+  if (!rc) rc = upload(&h->dSmall, F.small.data(), F.small.size(), st);
+  if (!rc) rc = upload(&h->dFrontTiles, F.utiles.data(), F.utiles.size(), st);
   // the FP32 shadow follows the structure's size whatever the current mode: a
   // later switch to a mixed mode finds it sized for this structure
   (void)hipFree(h->dLf);
@@ -2909,7 +3077,9 @@ int upload_structure(swc_handle* h, int n, const int* blockSet, int supNo, const
     else
       for (int m = 0; m < 3; ++m) h->dag_cap[m] = std::max(1, per[m]) * std::max(ncu, 1);
   }
-  if (!rc) rc = upload(&h->dDiag, (const double*)nullptr, (size_t)P.diag_scratch, st);
+  if (!rc)
+    rc = upload(&h->dDiag, (const double*)nullptr,
+                (size_t)std::max(P.diag_scratch, F.diag_scratch), st);
   if (!rc) rc = upload(&h->dNorm, (const double*)nullptr, 8, st);
   if (!rc) rc = upload(&h->dNormPart, (const double*)nullptr, kRedBlocks, st);
   h->zvalid = false;
@@ -2965,14 +3135,16 @@ int swc_upload(swc_handle* h, int n, const int* blockSet, int supNo, const size_
                const int* A2p, const int* A2i, const int64_t* a2src, int64_t nvals) {
   if (int rc = check_handle(h)) return rc;
   if (!A2p || !A2i) return swc_set_error(SWC_EINVAL, "swc_upload: bad argument");
-  if (int rc = upload_structure(h, n, blockSet, supNo, lC, Ls, Li_ptr, prunePtr, pruneSet, true))
+  A2Pattern a2{A2p, A2i, a2src, nvals, {}};
+  if (int rc = upload_structure(h, n, blockSet, supNo, lC, Ls, Li_ptr, prunePtr, pruneSet, &a2))
     return rc;
   if (A2p[0] != 0 || A2p[n] < 0) return swc_set_error(SWC_EINVAL, "swc_upload: bad A2 pointers");
   for (int j = 0; j < n; ++j)
     if (A2p[j + 1] < A2p[j]) return swc_set_error(SWC_EINVAL, "swc_upload: bad A2 pointers");
   h->nvals = a2src ? nvals : (int64_t)A2p[n];
+  if (!a2.ok) return swc_set_error(SWC_EINVAL, "A2 entry outside the structure of L");
   std::vector<int64_t> amap;
-  if (int rc = build_amap(h, A2p, A2i, a2src, nvals, amap)) return rc;
+  if (int rc = build_amap(h, A2p, a2.pos, a2src, nvals, amap)) return rc;
   // full CSR of P A P^T from its lower triangle, each entry mapped to its value
   std::vector<int> frp(n + 1, 0), fci;
   std::vector<int64_t> fvm;
@@ -3414,20 +3586,20 @@ int swc_get_timings(const swc_handle* h, double* out) {
   out[3] = h->n_tile;
   out[4] = h->t_trsm_ms;
   out[5] = h->n_trsm;
-  out[6] = P.tile_kernel_flops;
-  out[7] = P.trsm_kernel_flops;
+  out[6] = h->multifrontal ? h->fronts.update_flops : P.tile_kernel_flops;
+  out[7] = h->multifrontal ? h->fronts.factor_flops : P.trsm_kernel_flops;
   return SWC_OK;
 }
 
 int swc_level_timings(const swc_handle* h, double* out, int cap, int* nlevel) {
   if (int rc = check_handle(h)) return rc;
   if (!nlevel) return swc_set_error(SWC_EINVAL, "swc_level_timings: null argument");
-  const Plan& P = h->plan;
-  *nlevel = P.nlevel;
+  const auto& flops = h->multifrontal ? h->fronts.lvl_flops : h->plan.lvl_tile_flops;
+  *nlevel = h->multifrontal ? h->fronts.nlevel : h->plan.nlevel;
   if (!out) return SWC_OK;
-  for (int l = 0; l < std::min(cap, P.nlevel); ++l) {
+  for (int l = 0; l < std::min(cap, *nlevel); ++l) {
     out[2 * l] = l < (int)h->lvl_tile_ms.size() ? h->lvl_tile_ms[l] : 0.0;
-    out[2 * l + 1] = P.lvl_tile_flops[l];
+    out[2 * l + 1] = flops[l];
   }
   return SWC_OK;
 }
@@ -3448,6 +3620,17 @@ int swc_plan_stats(const swc_handle* h, int64_t* out, double* flops) {
     flops[2] = P.dag_flops;
     flops[3] = P.dag_sim_us;
     flops[4] = P.lvl_sim_us;
+  }
+  if (h->multifrontal) {  // update tiles, and the gathers and products they apply
+    const swc::FrontPlan& F = h->fronts;
+    out[0] = F.npanel;
+    out[1] = (int64_t)F.utiles.size();
+    out[2] = (int64_t)(F.utiles.size() + F.gathers.size());
+    out[3] = out[6] = F.nlevel;
+    if (flops) {
+      flops[0] = F.update_flops;
+      flops[1] = F.factor_flops;
+    }
   }
   return SWC_OK;
 }
@@ -3531,7 +3714,7 @@ int blockedLsolve(int n, size_t* Lp, int* Li, double* Lx, int NNZ, size_t* Li_pt
       swc_set_error(SWC_EINVAL, std::string("blockedLsolve: ") + e.what());
       return 0;
     }
-    if (upload_structure(g_lsolve, n, sup2col, supNo, Lp, Li, Li_ptr, pp.data(), ps.data(), false))
+    if (upload_structure(g_lsolve, n, sup2col, supNo, Lp, Li, Li_ptr, pp.data(), ps.data(), nullptr))
       return 0;
   }
   swc_handle* h = g_lsolve;
