@@ -64,6 +64,7 @@ SIGNATURES = {
                                       c_int, c_vp, c_vp, c_vp, ctypes.POINTER(c_vp)]),
     "swc_plan_free": (None, [c_vp]),
     "swc_plan_sizes": (c_int, [c_vp, c_vp, ctypes.POINTER(c_dbl)]),
+    "swc_plan_sweep_sizes": (c_int, [c_vp, c_vp]),
     "swc_plan_export": (c_int, [c_vp, c_int, c_vp]),
     "swc_plan_struct_sizes": (c_int, [c_vp]),
     "swc_front_plan_build": (c_int, [c_int, c_vp, c_int, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp,

@@ -352,6 +352,10 @@ TASK_DT = np.dtype([("src_base", np.int64), ("ld", np.int32), ("k", np.int32),
                     ("rmask", np.uint64), ("cmask", np.uint64)])
 SBLK_DT = np.dtype([("panel", np.int32), ("r0", np.int32), ("nr", np.int32),
                     ("writer", np.int32)])
+SWEEP_SMALL_DT = np.dtype([("vbase", np.int64), ("voff", np.int64)] + [
+    (k, np.int32) for k in ("R", "w", "c0", "rows_off")])
+SWEEP_ITEM_DT = np.dtype([("vbase", np.int64), ("out", np.int64)] + [(k, np.int32) for k in (
+    "ld", "w", "c0", "kind", "p", "nr", "row0", "row1", "nq", "rows_off", "first", "count")])
 DAG_DT = np.dtype([("tile", np.int32), ("fclass", np.int32), ("prev", np.int32),
                    ("diag", np.int32), ("dep0", np.int32), ("dep1", np.int32)])
 
@@ -408,6 +412,17 @@ def build_plan(bcsc: BCSC, derive_sets=False, params=None, schedule=None):
             a = np.zeros(cnt, dtype=dt)
             check(lib.swc_plan_export(h, which, ptr(a)))
             out[name] = a
+        sw = np.zeros(7, dtype=np.int64)
+        check(lib.swc_plan_sweep_sizes(h, ptr(sw)))
+        if [SWEEP_SMALL_DT.itemsize, SWEEP_ITEM_DT.itemsize] != [int(v) for v in sw[5:]]:
+            raise RuntimeError(f"sweep struct layout mismatch: library {list(sw[5:])}")
+        for which, name, dt, cnt in ((24, "sweep_small", SWEEP_SMALL_DT, sw[0]),
+                                     (25, "sweep_lvl_small", np.int32, sw[1]),
+                                     (26, "sweep_fwd", SWEEP_ITEM_DT, sw[2]),
+                                     (27, "sweep_bwd", SWEEP_ITEM_DT, sw[3])):
+            out[name] = np.zeros(int(cnt), dtype=dt)
+            check(lib.swc_plan_export(h, which, ptr(out[name])))
+        out["sweep_psize"] = int(sw[4])
         out.update(nlevel=nlevel, nslevel=nslevel, xsize=xsize, update_flops=fl[0],
                    factor_flops=fl[1], vsize=vsize, diag_scratch=dscr, dag_level0=dag_level0,
                    dag_flops=fl[2], dag_sim_us=fl[3], lvl_sim_us=fl[4])

@@ -66,8 +66,12 @@ __global__ void k_set_int(int* p, int v) { *p = v; }
 // operations but not for its global loads, which stay in flight across it
 // (__syncthreads() waits for every outstanding memory operation).  Used where no
 // thread reads global data that another thread of the workgroup has written.
+// The wait is explicit: behind a store in a branch of its own the compiler left out
+// the one that the release fence stands for, and waves passed the barrier with the
+// store still on its way.
 __device__ inline void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0), the other counters free
   __builtin_amdgcn_s_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
@@ -1036,613 +1040,7 @@ __global__ void k_factor_csc(const double* __restrict__ L, const int* __restrict
   }
 }
 
-// ---- triangular solves --------------------------------------------------
-// Forward L y = b (blockedLsolve, Triangular_BCSC.h:14-49, restated level by
-// level).  The reference pushes L21(s) x_s into the rows below each supernode
-// s; here every supernode s keeps that product as its contribution vector V_s,
-// and column c takes the contributions of all its descendants in increasing
-// supernode order (the order of the pushes) when its supernode starts.  Each
-// panel then solves its diagonal block; its row blocks push L21 x into the
-// supernode's later columns (in place) or into V_s.  The right-hand sides are
-// accumulated in X and the panel solutions written to Y, so that no launch
-// reads what it writes.  Backward L^T x = y: per panel, L21^T x over the rows
-// below (ancestors, already final in X) and the transposed diagonal solve,
-// written to X.
-
-// x[c] -= V[gidx[e]] for e in [gptr[c], gptr[c+1]), one thread per gathered column.
-__global__ void __launch_bounds__(kThreads)
-k_fwd_gather(const int* __restrict__ gcols, int g0, int ng, const int64_t* __restrict__ gptr,
-             const int64_t* __restrict__ gidx, const double* __restrict__ V, int64_t vld,
-             double* __restrict__ X, int nrhs, int64_t ldx) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  const int r = blockIdx.y;  // right-hand side
-  if (t >= ng || r >= nrhs) return;
-  const int c = gcols[g0 + t];
-  const int64_t e0 = gptr[c], e1 = gptr[c + 1];
-  const double* v = V + (int64_t)r * vld;
-  double acc = X[(int64_t)r * ldx + c];
-#pragma unroll 8
-  for (int64_t e = e0; e < e1; ++e) acc -= v[gidx[e]];
-  X[(int64_t)r * ldx + c] = acc;
-}
-
-// Substitution of one 64-column chunk for RB right-hand sides at once, lane i
-// holding row i of each: x_j = t_j / L_jj, then t_i -= L_ij x_j (forward,
-// row[j] = L_ij, j increasing) or t_i -= L_ji x_j (backward, row[j] = L_ji, the
-// transposed chunk, j decreasing).  row[j] must be zero wherever lane i does
-// not depend on x_j (j >= i forward, j <= i backward, and rows outside the
-// chunk), so every lane applies every step unmasked and its own entry is left
-// as t_i after the steps it depends on: x_i = t_i / L_ii at the end.  The RB
-// chains are independent and interleaved step by step, so their latencies
-// overlap.
-template <bool FORWARD, int RB>
-__device__ inline void substitute64(const double (&row)[64], double rinv, double (&ti)[RB]) {
-#pragma unroll
-  for (int s = 0; s < 64; ++s) {
-    const int j = FORWARD ? s : 63 - s;
-    double xj[RB];
-#pragma unroll
-    for (int q = 0; q < RB; ++q) xj[q] = bcast(ti[q] * rinv, j);  // lane j scales its entry
-#pragma unroll
-    for (int q = 0; q < RB; ++q) ti[q] = fma(-row[j], xj[q], ti[q]);
-  }
-#pragma unroll
-  for (int q = 0; q < RB; ++q) ti[q] *= rinv;
-}
-
-// Forward push of a row block for RB right-hand sides: part[w][q][i] holds wave
-// w's share of (L21 x_q)(row i); the shares are added in wave order and the sum
-// goes to a later column of the supernode (subtracted from x) or to a row of an
-// ancestor (added to the supernode's contribution vector V).
-template <int RB>
-__device__ inline void push_rows(const double (&part)[kThreads / 64][RB][swc::TM],
-                                 const Panel& sp, const swc::SolveBlock& bk, int rb0, int nq,
-                                 double* __restrict__ X, int64_t ldx, double* __restrict__ V,
-                                 int64_t vld) {
-  for (int e = threadIdx.x; e < RB * swc::TM; e += kThreads) {
-    const int q = e / swc::TM, i = e % swc::TM;
-    if (q < nq && i < bk.nr) {
-      const double y = ((part[0][q][i] + part[1][q][i]) + part[2][q][i]) + part[3][q][i];
-      const int p = (sp.c0 - sp.sc0) + bk.r0 + i;  // position in the supernode's rows
-      if (p < sp.sw) X[(int64_t)(rb0 + q) * ldx + sp.sc0 + p] -= y;
-      else V[(int64_t)(rb0 + q) * vld + sp.voff + (p - sp.sw)] += y;
-    }
-  }
-}
-
-// One forward row block of a solve panel (up to SPW = 128 columns of one
-// supernode, two 64-column chunks) for a group of RB right-hand sides
-// (blockIdx.y; the last group may hold fewer, padded with zero chains): solve
-// the panel's diagonal block (every block of the panel, from the same inputs),
-// write the solution if this is the panel's writer block, then push L21 x of
-// the block's rows.  L is read once per group, not once per right-hand side.
-// Each wave loads what its step needs at the start, so all loads are in flight
-// at once: wave 0 the first chunk's triangle (lane = row), wave 1 the second
-// chunk's rows of the first chunk's columns, wave 2 the second chunk's
-// triangle, and every wave its share of the block's rows.  Then wave 0
-// substitutes the first chunk, wave 1 subtracts its products from the second
-// chunk's entries, wave 2 substitutes the second chunk.
-static_assert(swc::SPW == 128, "the solve kernels split a solve panel in two 64-column chunks");
-template <int RB>
-__global__ void __launch_bounds__(kThreads)
-k_fwd_panel(const double* __restrict__ L, const Panel* __restrict__ spanels,
-            const swc::SolveBlock* __restrict__ blocks, int b0, double* __restrict__ V,
-            int64_t vld, double* __restrict__ X, double* __restrict__ Y, int nrhs, int64_t ldx,
-            int64_t ldy) {
-  __shared__ double xs[RB][swc::SPW];
-  __shared__ double part[kThreads / 64][RB][swc::TM];
-  const swc::SolveBlock bk = blocks[b0 + blockIdx.x];
-  const Panel sp = spanels[bk.panel];
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int nc = sp.ncol, na0 = min(64, nc), na1 = nc - 64;  // chunk widths (na1 <= 0: one chunk)
-  const double* D = L + sp.vbase;  // the panel's diagonal block, column j at D + j * ld
-  const int rb0 = blockIdx.y * RB, nq = min(RB, nrhs - rb0);  // this group's right-hand sides
-  // xs[q][c] = x_q of the panel's columns (zero for padded right-hand sides)
-  // The right-hand sides are loaded into registers before the panel's entries
-  // and written to LDS after them: loads complete in issue order, so this way
-  // the write waits only for its own loads, and the panel's entries arrive while
-  // the substitution runs (the barriers below wait for LDS traffic only).
-  constexpr int NX = (RB * swc::SPW + kThreads - 1) / kThreads;
-  double xv[NX];
-#pragma unroll
-  for (int u = 0; u < NX; ++u) {
-    const int e = tid + u * kThreads, q = e / swc::SPW, c = e % swc::SPW;
-    const bool in = e < RB * swc::SPW && c < nc && q < nq;
-    const double v = X[in ? (int64_t)(rb0 + q) * ldx + sp.c0 + c : 0];
-    xv[u] = in ? v : 0.0;
-  }
-  auto stage = [&]() {
-#pragma unroll
-    for (int u = 0; u < NX; ++u) {
-      const int e = tid + u * kThreads, q = e / swc::SPW, c = e % swc::SPW;
-      if (e < RB * swc::SPW && c < nc) xs[q][c] = xv[u];
-    }
-  };
-  auto store = [&]() {
-    for (int e = tid; e < RB * swc::SPW; e += kThreads) {
-      const int q = e / swc::SPW, c = e % swc::SPW;
-      if (q < nq && c < nc) Y[(int64_t)(rb0 + q) * ldy + sp.c0 + c] = xs[q][c];
-    }
-  };
-  if (nc <= 64) {
-    // one chunk: wave 0 substitutes it, then the block's rows are pushed
-    stage();
-    lds_barrier();
-    if (wave == 0) {
-      // row `lane` (clamped into the diagonal block), columns uniform over the wave
-      const int rl = min(lane, nc - 1);
-      const double dval = D[(int64_t)rl * sp.ld + rl];
-      double row[64];
-#pragma unroll
-      for (int c = 0; c < 64; ++c) {
-        const bool in = lane < nc && c < lane;
-        const double val = (D + (int64_t)min(c, nc - 1) * sp.ld)[rl];
-        row[c] = in ? val : 0.0;
-      }
-      const double rinv = lane < nc ? 1.0 / dval : 1.0;
-      double ti[RB];
-#pragma unroll
-      for (int q = 0; q < RB; ++q) ti[q] = lane < nc ? xs[q][lane] : 0.0;
-      substitute64<true, RB>(row, rinv, ti);
-      if (lane < nc) {
-#pragma unroll
-        for (int q = 0; q < RB; ++q) xs[q][lane] = ti[q];
-      }
-    }
-    lds_barrier();
-    if (bk.writer) store();
-    if (bk.nr > 0) {
-      double acc[RB] = {};
-      const int rb = bk.r0 + min(lane, bk.nr - 1);  // row clamped into the block
-#pragma unroll
-      for (int k = 0; k < 16; ++k) {
-        const int j = wave + 4 * k;
-        const bool in = lane < bk.nr && j < nc;
-        const double val = (D + (int64_t)min(j, nc - 1) * sp.ld)[rb];
-        const double lv = in ? val : 0.0;
-#pragma unroll
-        for (int q = 0; q < RB; ++q) acc[q] = fma(lv, j < nc ? xs[q][j] : 0.0, acc[q]);
-      }
-#pragma unroll
-      for (int q = 0; q < RB; ++q) part[wave][q][lane] = acc[q];
-      lds_barrier();
-      push_rows<RB>(part, sp, bk, rb0, nq, X, ldx, V, vld);
-    }
-    return;
-  }
-  // Loads are issued in the order they are needed (they complete in issue
-  // order): this wave's diagonal entry, its step's 64 columns, then its share of
-  // the block's rows, which are used last.
-  // this wave's step: element (row0 + lane, col0 + c), c < 64, where valid
-  // Every load takes a column base that is uniform over the wave (scalar
-  // arithmetic) and a row clamped into the panel once per lane; entries outside
-  // the wanted range are read from a valid address and replaced by zero.
-  const int row0 = wave == 0 ? 0 : 64, col0 = wave == 2 ? 64 : 0;
-  const int nrow = wave == 0 ? na0 : na1, ncol = wave == 2 ? na1 : na0;
-  const int rlast = sp.nrow - 1;  // last row of the panel's columns
-  const bool dg = (wave == 0 || wave == 2) && lane < nrow;
-  const int rs = min(row0 + lane, rlast);  // this lane's row of the step
-  const double dval = D[(int64_t)min(row0 + lane, nc - 1) * sp.ld + rs];
-  double m[64];
-#pragma unroll
-  for (int c = 0; c < 64; ++c) {
-    const bool in = wave < 3 && lane < nrow && c < ncol && (wave == 1 || c < lane);
-    const double val = (D + (int64_t)min(col0 + c, nc - 1) * sp.ld)[rs];
-    m[c] = in ? val : 0.0;
-  }
-  // the block's rows: wave w holds columns j = w, w+4, ... of row `lane`
-  constexpr int NQ = swc::SPW / 4;
-  double bv[NQ];
-  const int rb = min(bk.r0 + lane, rlast);
-#pragma unroll
-  for (int k = 0; k < NQ; ++k) {
-    const int j = wave + 4 * k;
-    const bool in = lane < bk.nr && j < nc;
-    const double val = (D + (int64_t)min(j, nc - 1) * sp.ld)[rb];
-    bv[k] = in ? val : 0.0;
-  }
-  // reciprocal of the diagonal entry; 1 beyond the chunk (padded unknowns stay 0)
-  const double rinv = dg ? 1.0 / dval : 1.0;
-  stage();
-  lds_barrier();
-  if (wave == 0) {
-    double ti[RB];
-#pragma unroll
-    for (int q = 0; q < RB; ++q) ti[q] = lane < na0 ? xs[q][lane] : 0.0;
-    substitute64<true, RB>(m, rinv, ti);
-    if (lane < na0) {
-#pragma unroll
-      for (int q = 0; q < RB; ++q) xs[q][lane] = ti[q];
-    }
-  }
-  lds_barrier();
-  if (na1 > 0) {
-    if (wave == 1 && lane < na1) {
-#pragma unroll
-      for (int q = 0; q < RB; ++q) {  // one right-hand side at a time, as in the push
-        double acc = 0.0;
-#pragma unroll
-        for (int c = 0; c < 64; ++c) acc = fma(m[c], xs[q][c], acc);  // na0 = 64 here
-        xs[q][64 + lane] -= acc;
-        __builtin_amdgcn_sched_barrier(0);
-      }
-    }
-    lds_barrier();
-    if (wave == 2) {
-      double ti[RB];
-#pragma unroll
-      for (int q = 0; q < RB; ++q) ti[q] = lane < na1 ? xs[q][64 + lane] : 0.0;
-      substitute64<true, RB>(m, rinv, ti);
-      if (lane < na1) {
-#pragma unroll
-        for (int q = 0; q < RB; ++q) xs[q][64 + lane] = ti[q];
-      }
-    }
-    lds_barrier();
-  }
-  if (bk.writer) store();
-  if (bk.nr > 0) {
-    // wave w sums columns j = w, w+4, ... for row `lane`, in increasing j
-    // (one right-hand side at a time: the barrier keeps the scheduler from
-    // hoisting every right-hand side's LDS reads at once, which would not fit
-    // the registers)
-#pragma unroll
-    for (int q = 0; q < RB; ++q) {
-      double acc = 0.0;
-#pragma unroll
-      for (int k = 0; k < NQ; ++k) {
-        const int j = wave + 4 * k;
-        acc = fma(bv[k], j < nc ? xs[q][j] : 0.0, acc);
-      }
-      part[wave][q][lane] = acc;
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    lds_barrier();
-    push_rows<RB>(part, sp, bk, rb0, nq, X, ldx, V, vld);
-  }
-}
-
-// Narrow solve panels (at most SPW_NARROW = 16 columns): one wave per row block
-// and per panel, everything in registers.  Forward: substitute the panel's
-// triangle (lane i holds row i), store the solution from the writer block, and
-// push L21 x of the block's rows (lane = row).
-__global__ void __launch_bounds__(64)
-k_fwd_narrow(const double* __restrict__ L, const Panel* __restrict__ spanels,
-             const swc::SolveBlock* __restrict__ blocks, int b0, double* __restrict__ V,
-             int64_t vld, double* __restrict__ X, double* __restrict__ Y, int64_t ldx,
-             int64_t ldy) {
-  constexpr int NW = swc::SPW_NARROW;
-  const swc::SolveBlock bk = blocks[b0 + blockIdx.x];
-  const Panel sp = spanels[bk.panel];
-  const int lane = threadIdx.x, r = blockIdx.y;
-  const int nc = sp.ncol;
-  double* x = X + (int64_t)r * ldx;
-  double* v = V + (int64_t)r * vld;
-  const double* D = L + sp.vbase;
-  const double* blk = D + bk.r0;
-  double row[NW], lv[NW];
-#pragma unroll
-  for (int c = 0; c < NW; ++c) {
-    row[c] = (lane < nc && c < lane) ? D[(int64_t)c * sp.ld + lane] : 0.0;
-    lv[c] = (lane < bk.nr && c < nc) ? blk[(int64_t)c * sp.ld + lane] : 0.0;
-  }
-  const double rinv = lane < nc ? 1.0 / D[(int64_t)lane * sp.ld + lane] : 1.0;
-  double ti = lane < nc ? x[sp.c0 + lane] : 0.0;
-#pragma unroll
-  for (int j = 0; j < NW; ++j)  // row[j] = 0 for j >= lane: unmasked steps
-    ti = fma(-row[j], bcast(ti * rinv, j), ti);  // lane j scales its own entry
-  ti *= rinv;
-  if (bk.writer && lane < nc) Y[(int64_t)r * ldy + sp.c0 + lane] = ti;
-  if (bk.nr > 0) {
-    double acc = 0.0;
-#pragma unroll
-    for (int c = 0; c < NW; ++c) acc = fma(lv[c], bcast(ti, c), acc);
-    if (lane < bk.nr) {
-      const int p = (sp.c0 - sp.sc0) + bk.r0 + lane;  // position in the supernode's rows
-      if (p < sp.sw) x[sp.sc0 + p] -= acc;
-      else v[sp.voff + (p - sp.sw)] += acc;
-    }
-  }
-}
-
-// Backward row block of a narrow panel: partial[j] = sum over the block's rows
-// of L(row, j) x(row).  Lane i forms row i's products and stores them in LDS;
-// lane l then sums column l mod 16 over rows 16g..16g+15 (g = l / 16) in order,
-// and two butterfly steps add the four row groups in a fixed order.
-__global__ void __launch_bounds__(64)
-k_bwd_partial_narrow(const double* __restrict__ L, const int* __restrict__ Ls,
-                     const Panel* __restrict__ spanels,
-                     const swc::SolveBlock* __restrict__ blocks, int b0, int bl,
-                     double* __restrict__ Pb, int64_t pld, const double* __restrict__ X,
-                     int64_t ldx) {
-  constexpr int NW = swc::SPW_NARROW;
-  const swc::SolveBlock bk = blocks[b0 + blockIdx.x];  // nr = 0 writes zeros
-  const Panel sp = spanels[bk.panel];
-  const int lane = threadIdx.x, r = blockIdx.y;
-  const int nc = sp.ncol;
-  const double* blk = L + sp.vbase + bk.r0;
-  const double xr = lane < bk.nr ? X[(int64_t)r * ldx + Ls[sp.rows_off + bk.r0 + lane]] : 0.0;
-  static_assert(NW == 16, "lane l sums column l mod 16 of a quarter of the rows");
-  __shared__ double pr[64][NW + 1];  // pr[row][column] (padded against bank conflicts)
-#pragma unroll
-  for (int c = 0; c < NW; ++c)
-    pr[lane][c] = (lane < bk.nr && c < nc) ? blk[(int64_t)c * sp.ld + lane] * xr : 0.0;
-  lds_barrier();
-  const int cl = lane % NW, g = lane / NW;
-  double sum = 0.0;
-#pragma unroll
-  for (int rr = 0; rr < 16; ++rr) sum += pr[16 * g + rr][cl];
-  sum += __shfl_xor(sum, 16);
-  sum += __shfl_xor(sum, 32);
-  double* out = Pb + (int64_t)r * pld + (int64_t)(b0 + blockIdx.x - bl) * swc::SPW;
-  if (lane < nc) out[lane] = sum;  // lanes 0..15 hold columns 0..15
-}
-
-// Backward narrow panel: t = y_p - (sum of its row blocks' partials, in block
-// order), then the transposed substitution (lane i holds column i of L11).
-__global__ void __launch_bounds__(64)
-k_bwd_diag_narrow(const double* __restrict__ L, const Panel* __restrict__ spanels,
-                  const int* __restrict__ order, int p0, const int* __restrict__ fblk_ptr,
-                  int bl, const double* __restrict__ Pb, int64_t pld,
-                  const double* __restrict__ Y, double* __restrict__ X, int64_t ldx,
-                  int64_t ldy) {
-  constexpr int NW = swc::SPW_NARROW;
-  const int qi = p0 + blockIdx.x;
-  const Panel sp = spanels[order[qi]];
-  const int lane = threadIdx.x, r = blockIdx.y;
-  const int nc = sp.ncol;
-  const int f0 = fblk_ptr[qi], f1 = fblk_ptr[qi + 1];
-  const double* D = L + sp.vbase;
-  double col[NW];
-#pragma unroll
-  for (int j = 0; j < NW; ++j) col[j] = (lane < nc && j > lane && j < nc) ? D[(int64_t)lane * sp.ld + j] : 0.0;
-  const double rinv = lane < nc ? 1.0 / D[(int64_t)lane * sp.ld + lane] : 1.0;
-  double ti = 0.0;
-  if (lane < nc) {
-    const double* pb = Pb + (int64_t)r * pld;
-    double sum = 0.0;
-    for (int b = f0; b < f1; ++b) sum += pb[(int64_t)(b - bl) * swc::SPW + lane];
-    ti = Y[(int64_t)r * ldy + sp.c0 + lane] - sum;
-  }
-#pragma unroll
-  for (int j = NW - 1; j >= 0; --j)  // col[j] = 0 for j <= lane: unmasked steps
-    ti = fma(-col[j], bcast(ti * rinv, j), ti);  // lane j scales its own entry
-  ti *= rinv;
-  if (lane < nc) X[(int64_t)r * ldx + sp.c0 + lane] = ti;
-}
-
-// Backward row block: partial[j] = sum over the block's rows of L(row, j) x(row)
-// for the solve panel's columns j, into Pb at the block's slot in its level
-// (its index minus the level's first block bl), for a group of RB right-hand
-// sides (blockIdx.y), so the block of L is read once per group.
-// Thread t takes column t mod SPW and half t / SPW of the block's rows, reads
-// them (contiguous in memory) all at once, and sums them in row order against
-// x(rows) staged in LDS; the two halves are then added, first half first.
-static_assert(kThreads == 2 * swc::SPW && swc::TM % 2 == 0, "two threads per column");
-template <int RB>
-__global__ void __launch_bounds__(kThreads)
-k_bwd_partial(const double* __restrict__ L, const int* __restrict__ Ls,
-              const Panel* __restrict__ spanels, const swc::SolveBlock* __restrict__ blocks,
-              int b0, int bl, double* __restrict__ Pb, int64_t pld, const double* __restrict__ X,
-              int nrhs, int64_t ldx) {
-  constexpr int H = swc::TM / 2;
-  __shared__ double xr[RB][swc::TM];
-  __shared__ double part[2][RB][swc::SPW];
-  const swc::SolveBlock bk = blocks[b0 + blockIdx.x];  // nr = 0 writes zeros
-  const Panel sp = spanels[bk.panel];
-  const int tid = threadIdx.x, c = tid % swc::SPW, h = tid / swc::SPW;
-  const int nc = sp.ncol, nr = bk.nr;
-  const int rb0 = blockIdx.y * RB, nq = min(RB, nrhs - rb0);  // this group's right-hand sides
-  // column c, rows [H h, H h + H) of the block (entries outside it read the
-  // panel's first diagonal entry, which always exists, and are replaced by zero)
-  // (the column clamped into the panel; a full block reads its 32 rows from one
-  // base address, a partial one clamps each row into the block)
-  const double* colp = L + sp.vbase + (int64_t)min(c, nc - 1) * sp.ld + bk.r0;
-  double lv[H];
-  if (nr == swc::TM) {
-#pragma unroll
-    for (int i = 0; i < H; ++i) {
-      const double val = colp[H * h + i];
-      lv[i] = c < nc ? val : 0.0;
-    }
-  } else if (nr > 0) {
-#pragma unroll
-    for (int i = 0; i < H; ++i) {
-      const bool in = c < nc && H * h + i < nr;
-      const double val = colp[min(H * h + i, nr - 1)];
-      lv[i] = in ? val : 0.0;
-    }
-  } else {
-#pragma unroll
-    for (int i = 0; i < H; ++i) lv[i] = 0.0;
-  }
-  for (int e = tid; e < RB * swc::TM; e += kThreads) {
-    const int q = e / swc::TM, i = e % swc::TM;
-    if (i < nr)
-      xr[q][i] = q < nq ? X[(int64_t)(rb0 + q) * ldx + Ls[sp.rows_off + bk.r0 + i]] : 0.0;
-  }
-  lds_barrier();
-  // one right-hand side at a time (the barrier bounds the LDS reads in flight
-  // to what the registers hold)
-#pragma unroll
-  for (int q = 0; q < RB; ++q) {
-    double acc = 0.0;
-#pragma unroll
-    for (int i = 0; i < H; ++i) acc = fma(lv[i], H * h + i < nr ? xr[q][H * h + i] : 0.0, acc);
-    part[h][q][c] = acc;
-    __builtin_amdgcn_sched_barrier(0);
-  }
-  lds_barrier();
-  const int64_t slot = (int64_t)(b0 + blockIdx.x - bl) * swc::SPW;
-  for (int e = tid; e < RB * swc::SPW; e += kThreads) {
-    const int q = e / swc::SPW, cc = e % swc::SPW;
-    if (q < nq && cc < nc) Pb[(int64_t)(rb0 + q) * pld + slot + cc] = part[0][q][cc] + part[1][q][cc];
-  }
-}
-
-// t = y - (sum of the panel's row-block partials) for RB right-hand sides, into
-// ts: thread t sums half t / SPW of the blocks for column t mod SPW, in block
-// order, kGather loads in flight per step; the halves are added first half first.
-// Every column of ts is written (zero past nc and for padded right-hand sides).
-constexpr int kGather = 32;
-template <int RB>
-__device__ inline void gather_partials(double (&ts)[RB][swc::SPW], const Panel& sp, int f0,
-                                       int f1, int b0, const double* __restrict__ Pb, int64_t pld,
-                                       const double* __restrict__ Y, int64_t ldy, int rb0,
-                                       int nq) {
-  const int tid = threadIdx.x, c = tid % swc::SPW, h = tid / swc::SPW, nc = sp.ncol;
-  const int fm = f0 + (f1 - f0 + 1) / 2, fa = h == 0 ? f0 : fm, fb = h == 0 ? fm : f1;
-  double sum[RB] = {};
-  if (c < nc) {
-    for (int b = fa; b < fb; b += kGather) {
-#pragma unroll
-      for (int q = 0; q < RB; ++q) {
-        if (q < nq) {  // uniform
-          const double* pb = Pb + (int64_t)(rb0 + q) * pld + c;
-          double pv[kGather];
-#pragma unroll
-          for (int u = 0; u < kGather; ++u) {
-            // clamped to the last block, so every load is inside the partials
-            const double val = pb[(int64_t)(min(b + u, fb - 1) - b0) * swc::SPW];
-            pv[u] = b + u < fb ? val : 0.0;
-          }
-#pragma unroll
-          for (int u = 0; u < kGather; ++u) sum[q] += pv[u];
-        }
-        __builtin_amdgcn_sched_barrier(0);  // kGather loads in flight, not kGather RB
-      }
-    }
-  }
-  if (h == 1) {
-#pragma unroll
-    for (int q = 0; q < RB; ++q) ts[q][c] = sum[q];
-  }
-  lds_barrier();
-  if (h == 0 && c < nc) {
-#pragma unroll
-    for (int q = 0; q < RB; ++q)
-      ts[q][c] = q < nq ? Y[(int64_t)(rb0 + q) * ldy + sp.c0 + c] - (sum[q] + ts[q][c]) : 0.0;
-  }
-}
-
-// Backward solve panel: t = y_p - (sum of its row blocks' partials, in block
-// order), then L11^T x_p = t chunk by chunk from the last, for a group of RB
-// right-hand sides (blockIdx.y).  As in the forward
-// kernel each wave loads its step's operands first: wave 0 the second
-// chunk's transposed triangle (lane = column), wave 1 the second chunk's rows
-// of the first chunk's columns (lane = column), wave 2 the first chunk's
-// transposed triangle.  Wave 0 substitutes the second chunk, wave 1 subtracts
-// its products from the first chunk's entries, wave 2 substitutes the first.
-template <int RB>
-__global__ void __launch_bounds__(kThreads)
-k_bwd_diag(const double* __restrict__ L, const Panel* __restrict__ spanels,
-           const int* __restrict__ order, int p0, const int* __restrict__ fblk_ptr, int b0,
-           const double* __restrict__ Pb, int64_t pld, const double* __restrict__ Y,
-           double* __restrict__ X, int nrhs, int64_t ldx, int64_t ldy) {
-  __shared__ double ts[RB][swc::SPW];
-  const int qi = p0 + blockIdx.x;
-  const Panel sp = spanels[order[qi]];
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int nc = sp.ncol, na0 = min(64, nc), na1 = nc - 64;  // chunk widths (na1 <= 0: one chunk)
-  const int f0 = fblk_ptr[qi], f1 = fblk_ptr[qi + 1];
-  const double* D = L + sp.vbase;
-  const int rb0 = blockIdx.y * RB, nq = min(RB, nrhs - rb0);  // this group's right-hand sides
-  auto store = [&]() {
-    for (int e = tid; e < RB * swc::SPW; e += kThreads) {
-      const int q = e / swc::SPW, c = e % swc::SPW;
-      if (q < nq && c < nc) X[(int64_t)(rb0 + q) * ldx + sp.c0 + c] = ts[q][c];
-    }
-  };
-  if (nc <= 64) {
-    // one chunk: wave 0 loads its transposed triangle while the partials are
-    // summed, then substitutes it
-    double col[64];
-    double rinv = 1.0;
-    if (wave == 0) {
-      // column `lane` (clamped into the panel), rows uniform over the wave
-      const double* colp = D + (int64_t)min(lane, nc - 1) * sp.ld;
-      const double dval = colp[min(lane, nc - 1)];
-#pragma unroll
-      for (int j = 0; j < 64; ++j) {
-        const bool in = lane < nc && j > lane && j < nc;
-        const double val = colp[min(j, nc - 1)];
-        col[j] = in ? val : 0.0;
-      }
-      rinv = lane < nc ? 1.0 / dval : 1.0;
-    }
-    gather_partials<RB>(ts, sp, f0, f1, b0, Pb, pld, Y, ldy, rb0, nq);
-    lds_barrier();
-    if (wave == 0) {
-      double ti[RB];
-#pragma unroll
-      for (int q = 0; q < RB; ++q) ti[q] = lane < nc ? ts[q][lane] : 0.0;
-      substitute64<false, RB>(col, rinv, ti);
-      if (lane < nc) {
-#pragma unroll
-        for (int q = 0; q < RB; ++q) ts[q][lane] = ti[q];
-      }
-    }
-    lds_barrier();
-    store();
-    return;
-  }
-  // this wave's step: m[j] = L(rowc + j, colc + lane) where valid
-  const int colc = wave == 0 ? 64 : 0, rowc = wave == 2 ? 0 : 64;
-  const int ncl = wave == 0 ? na1 : na0, nrw = wave == 2 ? na0 : na1;
-  // column colc + lane (clamped into the panel), rows uniform over the wave;
-  // the diagonal entry first, as loads complete in issue order
-  const double* colp = D + (int64_t)min(colc + lane, nc - 1) * sp.ld;
-  const bool dg = (wave == 0 || wave == 2) && lane < ncl;
-  const double dval = colp[min(colc + lane, nc - 1)];
-  double m[64];
-#pragma unroll
-  for (int j = 0; j < 64; ++j) {
-    const bool in = wave < 3 && lane < ncl && j < nrw && (wave == 1 || j > lane);
-    const double val = colp[min(rowc + j, nc - 1)];
-    m[j] = in ? val : 0.0;
-  }
-  const double rinv = dg ? 1.0 / dval : 1.0;
-  gather_partials<RB>(ts, sp, f0, f1, b0, Pb, pld, Y, ldy, rb0, nq);
-  lds_barrier();
-  if (na1 > 0) {
-    if (wave == 0) {
-      double ti[RB];
-#pragma unroll
-      for (int q = 0; q < RB; ++q) ti[q] = lane < na1 ? ts[q][64 + lane] : 0.0;
-      substitute64<false, RB>(m, rinv, ti);
-      if (lane < na1) {
-#pragma unroll
-        for (int q = 0; q < RB; ++q) ts[q][64 + lane] = ti[q];
-      }
-    }
-    lds_barrier();
-    // first-chunk entries: t_i -= sum_j L(64 + j, i) x_(64 + j); ts is zero
-    // past nc (gather_partials writes every column), so no read is masked
-    if (wave == 1) {
-#pragma unroll
-      for (int q = 0; q < RB; ++q) {  // one right-hand side at a time (register bound)
-        double acc = 0.0;
-#pragma unroll
-        for (int j = 0; j < 64; ++j) acc = fma(m[j], ts[q][64 + j], acc);
-        ts[q][lane] -= acc;  // na0 = 64 here
-        __builtin_amdgcn_sched_barrier(0);
-      }
-    }
-    lds_barrier();
-  }
-  if (wave == 2) {
-    double ti[RB];
-#pragma unroll
-    for (int q = 0; q < RB; ++q) ti[q] = lane < na0 ? ts[q][lane] : 0.0;
-    substitute64<false, RB>(m, rinv, ti);
-    if (lane < na0) {
-#pragma unroll
-      for (int q = 0; q < RB; ++q) ts[q][lane] = ti[q];
-    }
-  }
-  lds_barrier();
-  store();
-}
+#include "sweep_kernels.h"
 
 // y[k] = b[perm[k]] (to the factor's ordering) or x[perm[k]] = y[k] (back).
 __global__ void k_permute(const double* __restrict__ in, double* __restrict__ out,
@@ -1670,6 +1068,32 @@ constexpr int kRedBlocks = 512;
 // device's copy once (scratch_ptr) and everything else uses that pointer.
 constexpr int64_t kScratchDoubles = (int64_t)16 << 20;  // 128 MiB
 static __device__ __align__(256) double scratch[kScratchDoubles];
+
+// Pinned host words that a sweep sets when one of its waits runs out, one per handle: taken
+// in swc_create and given back in swc_destroy, in blocks that are kept for later handles.
+std::mutex g_abort_mu;
+std::vector<int*> g_abort_free;
+
+int* take_abort_word() {
+  std::lock_guard<std::mutex> lock(g_abort_mu);
+  if (g_abort_free.empty()) {
+    constexpr int kWords = 1024;
+    int* block = nullptr;
+    if (hipHostMalloc((void**)&block, kWords * sizeof(int), hipHostMallocPortable) != hipSuccess)
+      return nullptr;
+    for (int i = 0; i < kWords; ++i) g_abort_free.push_back(block + i);
+  }
+  int* w = g_abort_free.back();
+  g_abort_free.pop_back();
+  *w = 0;
+  return w;
+}
+
+void give_abort_word(int* w) {
+  if (!w) return;
+  std::lock_guard<std::mutex> lock(g_abort_mu);
+  g_abort_free.push_back(w);
+}
 
 // Per-device address of `scratch`, looked up once per device with that device
 // current (hipGetSymbolAddress); null until then.
@@ -2068,20 +1492,18 @@ struct swc_handle {
   float* dLf = nullptr;  // FP32 shadow of L, written with it when FP32 updates are on
   int64_t lf_cap = 0;    // elements allocated at dLf
   int* dLs = nullptr;
-  Panel* dPanels = nullptr;
   Tile* dTiles = nullptr;
   Task* dTasks = nullptr;
   int64_t* dGptr = nullptr;  // forward gathers: per column, offsets into dGidx
   int64_t* dGidx = nullptr;
-  int* dGcols = nullptr;     // gathered columns by level
-  swc::SolveBlock* dFblk = nullptr;
-  int* dFblkPtr = nullptr;  // per panel (level order): its forward/backward row blocks
+  swc::SweepSmall* dSweepSmall = nullptr;  // the solves' work lists (sweeps.h)
+  swc::SweepItem* dSweepFwd = nullptr;
+  swc::SweepItem* dSweepBwd = nullptr;
+  int* dSweepSync = nullptr;  // tickets of the two sweeps, abort flag
+  int* abort_host = nullptr;  // pinned: a sweep's wait ran out (a slot of the abort pool)
   double* dV = nullptr;   // contribution vectors, vsize * work_cols
   double* dPb = nullptr;  // backward partial sums, max_lvl_fblk * SPW * work_cols
-  Panel* dSpanels = nullptr;  // solve panels
-  int* dSpOrder = nullptr;    // solve panels by level
   double* dY = nullptr;   // forward solutions, n * work_cols
-  int* dOrder = nullptr;
   Tile* dFtiles = nullptr;  // factor-kernel tiles (copies), by level and width class
   swc::FusedPanel* dFused = nullptr;  // fused narrow panels, by level
   swc::Gather* dGathers = nullptr;    // the front plan's lists (fronts.h)
@@ -2157,7 +1579,12 @@ struct swc_handle {
   std::vector<double> lvl_tile_ms;  // per level, when profiling
   int n_tile = 0, n_trsm = 0;
 
-  ~swc_handle() { release(); }
+  int sweep_cap = 0;  // workgroups of a sweep's persistent launch
+
+  ~swc_handle() {
+    release();
+    give_abort_word(abort_host);
+  }
   void drop_graphs() {
     for (auto& g : fgraph)
       if (g) (void)hipGraphExecDestroy(g);
@@ -2167,8 +1594,8 @@ struct swc_handle {
   }
   void release() {
     drop_graphs();
-    (void)hipFree(dL); (void)hipFree(dLf); (void)hipFree(dLs); (void)hipFree(dPanels); (void)hipFree(dTiles); (void)hipFree(dTasks);
-    (void)hipFree(dGptr); (void)hipFree(dGidx); (void)hipFree(dGcols); (void)hipFree(dFblk); (void)hipFree(dFblkPtr); (void)hipFree(dV); (void)hipFree(dPb); (void)hipFree(dY); (void)hipFree(dSpanels); (void)hipFree(dSpOrder); (void)hipFree(dOrder); (void)hipFree(dFtiles); (void)hipFree(dFused);
+    (void)hipFree(dL); (void)hipFree(dLf); (void)hipFree(dLs); (void)hipFree(dTiles); (void)hipFree(dTasks);
+    (void)hipFree(dGptr); (void)hipFree(dGidx); (void)hipFree(dSweepSmall); (void)hipFree(dSweepFwd); (void)hipFree(dSweepBwd); (void)hipFree(dSweepSync); (void)hipFree(dV); (void)hipFree(dPb); (void)hipFree(dY); (void)hipFree(dFtiles); (void)hipFree(dFused);
     (void)hipFree(dGathers); (void)hipFree(dAents); (void)hipFree(dFactorTiles); (void)hipFree(dSmall); (void)hipFree(dFrontTiles);
     (void)hipFree(dCounters); (void)hipFree(dDagItems); (void)hipFree(dDagDeps); (void)hipFree(dDagSync); (void)hipFree(dDiag); (void)hipFree(dAmap); (void)hipFree(dPerm);
     (void)hipFree(dVals); (void)hipFree(dWork); (void)hipFree(dInfo);
@@ -2176,8 +1603,8 @@ struct swc_handle {
     (void)hipFree(dRef);
     (void)hipFree(dZ); (void)hipFree(dArena); (void)hipFree(dNodes); (void)hipFree(dCol2sup); (void)hipFree(dSpx);
     (void)hipFree(dSsuper); (void)hipFree(dSpi); (void)hipFree(dDiagPos); (void)hipFree(dQi); (void)hipFree(dQj);
-    dL = nullptr; dLf = nullptr; dLs = nullptr; dPanels = nullptr; dTiles = nullptr; dTasks = nullptr;
-    dGptr = nullptr; dGidx = nullptr; dGcols = nullptr; dFblk = nullptr; dFblkPtr = nullptr; dV = nullptr; dPb = nullptr; dY = nullptr; dSpanels = nullptr; dSpOrder = nullptr; dOrder = nullptr; dFtiles = nullptr; dFused = nullptr; dGathers = nullptr; dAents = nullptr; dFactorTiles = nullptr; dSmall = nullptr; dFrontTiles = nullptr; dCounters = nullptr; dDagItems = nullptr; dDagDeps = nullptr; dDagSync = nullptr; dDiag = nullptr; dAmap = nullptr; dPerm = nullptr;
+    dL = nullptr; dLf = nullptr; dLs = nullptr; dTiles = nullptr; dTasks = nullptr;
+    dGptr = nullptr; dGidx = nullptr; dSweepSmall = nullptr; dSweepFwd = nullptr; dSweepBwd = nullptr; dSweepSync = nullptr; dV = nullptr; dPb = nullptr; dY = nullptr; dFtiles = nullptr; dFused = nullptr; dGathers = nullptr; dAents = nullptr; dFactorTiles = nullptr; dSmall = nullptr; dFrontTiles = nullptr; dCounters = nullptr; dDagItems = nullptr; dDagDeps = nullptr; dDagSync = nullptr; dDiag = nullptr; dAmap = nullptr; dPerm = nullptr;
     dVals = nullptr; dWork = nullptr; dInfo = nullptr;
     dRp = nullptr; dCi = nullptr; dVmap = nullptr; dAf = nullptr; dNorm = nullptr; dScal = nullptr; dPart = nullptr; dNormPart = nullptr;
     lf_cap = 0;
@@ -2511,89 +1938,101 @@ int factor_device(swc_handle* h, const double* dvals) {
   return SWC_OK;
 }
 
-// Enqueues the forward and backward sweeps on device columns X (factor
-// ordering); the panel kernels take the right-hand sides in groups: RF for the
-// forward kernel, RP for the backward partials, RD for the backward diagonal.
-// Forward sweep L Y = X: X is consumed (it accumulates the pushes), the
-// solution goes to Y (ld n), V holds the contribution vectors (ld vsize).
-template <int RF>
-void enqueue_forward(swc_handle* h, double* dX, int nrhs, int64_t ldx, double* dY, double* dV) {
-  const int ngf = (nrhs + RF - 1) / RF;
-  hipStream_t st = h->stream;
-  const Plan& P = h->plan;
-  const int64_t vld = std::max<int64_t>(P.vsize, 1);
-  const int64_t ldy = h->n;
-  const Panel* sps = (const Panel*)h->dSpanels;
-  const swc::SolveBlock* fbl = (const swc::SolveBlock*)h->dFblk;
-  hipLaunchKernelGGL(k_fill, dim3(grid_for(vld * nrhs)), dim3(kThreads), 0, st, dV, vld * nrhs, 0.0);
-  for (int l = 0; l < P.nslevel; ++l) {
-    const int g0 = P.lvl_gcol[l], ng = P.lvl_gcol[l + 1] - g0;
-    const int b0 = P.lvl_fblk[l], nb = P.lvl_fblk[l + 1] - b0, nbn = P.lvl_fblk_narrow[l];
-    if (ng > 0)
-      hipLaunchKernelGGL(k_fwd_gather, dim3((ng + kThreads - 1) / kThreads, nrhs), dim3(kThreads), 0, st,
-                         (const int*)h->dGcols, g0, ng, (const int64_t*)h->dGptr,
-                         (const int64_t*)h->dGidx, (const double*)dV, vld, dX, nrhs, ldx);
-    if (nbn > 0)
-      hipLaunchKernelGGL(k_fwd_narrow, dim3(nbn, nrhs), dim3(64), 0, st, (const double*)h->dL, sps,
-                         fbl, b0, dV, vld, dX, dY, ldx, ldy);
-    if (nb > nbn)
-      hipLaunchKernelGGL(k_fwd_panel<RF>, dim3(nb - nbn, ngf), dim3(kThreads), 0, st, (const double*)h->dL,
-                         sps, fbl, b0 + nbn, dV, vld, dX, dY, nrhs, ldx, ldy);
+// Right-hand sides from which the sweeps take them 16 to an item (MFMA) instead of one.
+constexpr int kSweepGroupMin = 2;
+
+// One persistent launch of a sweep; the ticket was cleared before.
+template <bool FORWARD, int GROUP>
+void launch_sweep(swc_handle* h, const SweepRun& a) {
+  if (a.nitems == 0) return;
+  const int ngroups = (a.nrhs + GROUP - 1) / GROUP;
+  // tickets are ints: very many right-hand sides go in several launches
+  const int step = (int)std::max<int64_t>(1, std::min<int64_t>(ngroups, (1 << 30) / a.nitems));
+  for (int g0 = 0; g0 < ngroups; g0 += step) {
+    const int ng = std::min(step, ngroups - g0);
+    if (g0 > 0)
+      hipLaunchKernelGGL(k_set_int, dim3(1), dim3(1), 0, h->stream, a.ticket, 0);
+    const int64_t total = (int64_t)a.nitems * ng;
+    hipLaunchKernelGGL((k_sweep<FORWARD, GROUP>), dim3((unsigned)std::min<int64_t>(total, h->sweep_cap)),
+                       dim3(kThreads), 0, h->stream, a, g0, ng);
   }
 }
 
-// Backward sweep L^T X = Y (Y ld n), into X; Pb holds the row blocks' partials.
-template <int RP, int RD>
-void enqueue_backward(swc_handle* h, double* dX, int nrhs, int64_t ldx, const double* dY,
-                      double* dPb) {
-  const int ngp = (nrhs + RP - 1) / RP, ngd = (nrhs + RD - 1) / RD;
-  hipStream_t st = h->stream;
+template <bool FORWARD>
+void launch_small(swc_handle* h, const SweepRun& a, int level) {
+  const std::vector<int>& ls = h->plan.sweeps.lvl_small;
+  const int s0 = ls[level], ns = ls[level + 1] - s0;
+  if (a.nrhs == 1)
+    hipLaunchKernelGGL((k_sweep_small<FORWARD, 1>), dim3((ns + 3) / 4, 1), dim3(kThreads), 0,
+                       h->stream, a, s0, ns);
+  else
+    hipLaunchKernelGGL((k_sweep_small<FORWARD, 4>), dim3((ns + 3) / 4, (a.nrhs + 3) / 4),
+                       dim3(kThreads), 0, h->stream, a, s0, ns);
+}
+
+SweepRun sweep_run(swc_handle* h, double* dX, int nrhs, int64_t ldx, double* dY, double* dV,
+                   double* dPb) {
   const Plan& P = h->plan;
-  const int64_t ldy = h->n;
-  const Panel* sps = (const Panel*)h->dSpanels;
-  const swc::SolveBlock* fbl = (const swc::SolveBlock*)h->dFblk;
-  const int64_t pld = (int64_t)std::max(P.max_lvl_fblk, 1) * swc::SPW;
-  for (int l = P.nslevel - 1; l >= 0; --l) {
-    const int p0 = P.lvl_sp[l], np = P.lvl_sp[l + 1] - p0, npn = P.lvl_sp_narrow[l];
-    const int b0 = P.lvl_fblk[l], nb = P.lvl_fblk[l + 1] - b0, nbn = P.lvl_fblk_narrow[l];
-    if (nbn > 0)
-      hipLaunchKernelGGL(k_bwd_partial_narrow, dim3(nbn, nrhs), dim3(64), 0, st, (const double*)h->dL,
-                         (const int*)h->dLs, sps, fbl, b0, b0, dPb, pld, (const double*)dX, ldx);
-    if (nb > nbn)
-      hipLaunchKernelGGL(k_bwd_partial<RP>, dim3(nb - nbn, ngp), dim3(kThreads), 0, st, (const double*)h->dL,
-                         (const int*)h->dLs, sps, fbl, b0 + nbn, b0, dPb, pld, (const double*)dX,
-                         nrhs, ldx);
-    if (npn > 0)
-      hipLaunchKernelGGL(k_bwd_diag_narrow, dim3(npn, nrhs), dim3(64), 0, st, (const double*)h->dL, sps,
-                         (const int*)h->dSpOrder, p0, (const int*)h->dFblkPtr, b0,
-                         (const double*)dPb, pld, dY, dX, ldx, ldy);
-    if (np > npn)
-      hipLaunchKernelGGL(k_bwd_diag<RD>, dim3(np - npn, ngd), dim3(kThreads), 0, st, (const double*)h->dL, sps,
-                         (const int*)h->dSpOrder, p0 + npn, (const int*)h->dFblkPtr, b0,
-                         (const double*)dPb, pld, dY, dX, nrhs, ldx, ldy);
-  }
+  SweepRun a{};
+  a.L = h->dL;
+  a.Ls = h->dLs;
+  a.gptr = h->dGptr;
+  a.gidx = h->dGidx;
+  a.small = h->dSweepSmall;
+  a.abort_flag = h->dSweepSync + 2;
+  a.abort_host = h->abort_host;
+  a.X = dX;
+  a.Y = dY;
+  a.V = dV;
+  a.P = dPb;
+  a.ldx = ldx;
+  a.ldy = h->n;
+  a.ldv = std::max<int64_t>(P.vsize, 1);
+  a.ldp = std::max<int64_t>(P.sweeps.psize, 1);
+  a.nrhs = nrhs;
+  return a;
 }
 
-template <int RF, int RP, int RD>
-void enqueue_solve_rb(swc_handle* h, double* dX, int nrhs, int64_t ldx, double* dY, double* dV,
-                      double* dPb) {
-  enqueue_forward<RF>(h, dX, nrhs, ldx, dY, dV);
-  enqueue_backward<RP, RD>(h, dX, nrhs, ldx, dY, dPb);
+// Forward sweep L Y = X (X is left marked for the backward sweep).
+void enqueue_forward(swc_handle* h, SweepRun a) {
+  const swc::SweepPlan& W = h->plan.sweeps;
+  const int64_t ny = a.ldy * a.nrhs, nv = a.ldv * a.nrhs, np = a.ldp * a.nrhs;
+  hipLaunchKernelGGL(k_sweep_init, dim3(std::min(grid_for(std::max(ny, nv)), 4096)), dim3(kThreads),
+                     0, h->stream, a.Y, ny, a.V, nv, a.P, np, h->dSweepSync);
+  for (int l = 0; l + 1 < (int)W.lvl_small.size(); ++l) launch_small<true>(h, a, l);
+  a.items = h->dSweepFwd;
+  a.nitems = (int)W.fwd.size();
+  a.ticket = h->dSweepSync;
+  if (a.nrhs < kSweepGroupMin) launch_sweep<true, 1>(h, a);
+  else launch_sweep<true, 16>(h, a);
 }
 
-// Groups of right-hand sides: each block of L is read once per group, while
-// the substitution chains of a group run one after another in one wave.  The
-// forward kernel takes 4 (at 8 it needs more than 256 registers per lane, one
-// wave per SIMD); the backward partials, which have no chain, take 8, or 16
-// from 16 right-hand sides on; the backward diagonal, mostly chain, takes one
-// per workgroup (measured on the vector 48^3 operator at 8 and 32 RHS).
-// dY (n x nrhs), dV (max(vsize, 1) x nrhs) and dPb (max(max_lvl_fblk, 1) SPW x
-// nrhs) are the sweeps' workspace.
+// Backward sweep L^T X = Y.
+void enqueue_backward(swc_handle* h, SweepRun a) {
+  const swc::SweepPlan& W = h->plan.sweeps;
+  a.items = h->dSweepBwd;
+  a.nitems = (int)W.bwd.size();
+  a.ticket = h->dSweepSync + 1;
+  if (a.nrhs < kSweepGroupMin) launch_sweep<false, 1>(h, a);
+  else launch_sweep<false, 16>(h, a);
+  for (int l = (int)W.lvl_small.size() - 2; l >= 0; --l) launch_small<false>(h, a, l);
+}
+
+// dY (n x nrhs), dV (max(vsize, 1) x nrhs) and dPb (max(max_lvl_fblk, 1) SPW x nrhs, which
+// holds the backward partials) are the sweeps' workspace.
 void enqueue_solve_bufs(swc_handle* h, double* dX, int nrhs, int64_t ldx, double* dY, double* dV,
                         double* dPb) {
-  if (nrhs >= 16) enqueue_solve_rb<4, 16, 1>(h, dX, nrhs, ldx, dY, dV, dPb);
-  else if (nrhs >= 2) enqueue_solve_rb<4, 8, 1>(h, dX, nrhs, ldx, dY, dV, dPb);
-  else enqueue_solve_rb<1, 1, 1>(h, dX, nrhs, ldx, dY, dV, dPb);
+  const SweepRun a = sweep_run(h, dX, nrhs, ldx, dY, dV, dPb);
+  enqueue_forward(h, a);
+  enqueue_backward(h, a);
+}
+
+// Waits for the handle's stream; an error where a sweep's wait ran out.
+int sync_stream(swc_handle* h) {
+  SWC_HIP(hipStreamSynchronize(h->stream));
+  if (__atomic_exchange_n(h->abort_host, 0, __ATOMIC_RELAXED) != 0)
+    return swc_set_error(SWC_EDEVICE, "solve: a wait inside a sweep ran out of time");
+  return SWC_OK;
 }
 
 void enqueue_solve(swc_handle* h, double* dX, int nrhs, int64_t ldx) {
@@ -2669,8 +2108,7 @@ int from_factor(swc_handle* h, const double* dIn, double* X, int on_device, int6
   if (!on_device)
     SWC_HIP(hipMemcpy2DAsync(X, sizeof(double) * ldx, h->dWork, sizeof(double) * n,
                              sizeof(double) * n, nrhs, hipMemcpyDeviceToHost, st));
-  SWC_HIP(hipStreamSynchronize(st));
-  return SWC_OK;
+  return sync_stream(h);
 }
 
 // ---- refinement -------------------------------------------------------------
@@ -2683,8 +2121,7 @@ int reduce_cols(swc_handle* h, const double* X, const double* Y, int ncol, int o
   hipLaunchKernelGGL(k_reduce_final, dim3(ncol), dim3(kThreads), 0, st, (const double*)h->dPart, op,
                      h->dScal + 64);
   SWC_HIP(hipMemcpyAsync(out, h->dScal + 64, sizeof(double) * ncol, hipMemcpyDeviceToHost, st));
-  SWC_HIP(hipStreamSynchronize(st));
-  return SWC_OK;
+  return sync_stream(h);
 }
 
 // Y = A X, or R = B - A X when B is given, on n x nrhs device columns of
@@ -3036,20 +2473,26 @@ int upload_structure(swc_handle* h, int n, const int* blockSet, int supNo, const
     if (!rc) h->lf_cap = P.xsize;
   }
   if (!rc) rc = upload(&h->dLs, h->Ls.data(), h->Ls.size(), st);
-  if (!rc) rc = upload(&h->dPanels, P.panels.data(), P.panels.size(), st);
   if (!rc) rc = upload(&h->dTiles, P.tiles.data(), P.tiles.size(), st);
   if (!rc) rc = upload(&h->dTasks, P.tasks.data(), P.tasks.size(), st);
   if (!rc) rc = upload(&h->dGptr, P.gptr.data(), P.gptr.size(), st);
   if (!rc) rc = upload(&h->dGidx, P.gidx.data(), P.gidx.size(), st);
-  if (!rc) rc = upload(&h->dGcols, P.gcols.data(), P.gcols.size(), st);
-  if (!rc) rc = upload(&h->dFblk, P.fblocks.data(), P.fblocks.size(), st);
-  if (!rc) rc = upload(&h->dFblkPtr, P.fblk_ptr.data(), P.fblk_ptr.size(), st);
-  if (!rc) rc = upload(&h->dSpanels, P.spanels.data(), P.spanels.size(), st);
-  if (!rc) rc = upload(&h->dSpOrder, P.sp_order.data(), P.sp_order.size(), st);
-  if (!rc) rc = upload(&h->dOrder, P.panel_order.data(), P.panel_order.size(), st);
+  if (!rc) rc = upload(&h->dSweepSmall, P.sweeps.small.data(), P.sweeps.small.size(), st);
+  if (!rc) rc = upload(&h->dSweepFwd, P.sweeps.fwd.data(), P.sweeps.fwd.size(), st);
+  if (!rc) rc = upload(&h->dSweepBwd, P.sweeps.bwd.data(), P.sweeps.bwd.size(), st);
+  if (!rc) rc = upload(&h->dSweepSync, (const int*)nullptr, 4, st);
   if (!rc) rc = upload(&h->dFtiles, P.ftiles.data(), P.ftiles.size(), st);
   if (!rc) rc = upload(&h->dFused, P.fused.data(), P.fused.size(), st);
   if (!rc) rc = upload(&h->dCounters, (const int*)nullptr, (size_t)std::max(P.nlevel, 1), st);
+  if (!rc && h->sweep_cap == 0) {
+    // two workgroups to a CU (what the sweeps' registers allow); any number is safe
+    int ncu = 0;
+    const hipError_t e = hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, h->device);
+    if (e != hipSuccess)
+      rc = swc_set_error(SWC_EDEVICE, std::string("upload: device query: ") + hipGetErrorString(e));
+    else
+      h->sweep_cap = 2 * std::max(ncu, 1);
+  }
   if (!rc && h->fused_cap[0] == 0) {
     // a persistent grid: as many workgroups as the device holds at once
     int ncu = 0, per[3] = {0, 0, 0};
@@ -3113,6 +2556,7 @@ int swc_create(swc_handle** out) {
     delete h;
     return SWC_EDEVICE;  // bind_scratch recorded why
   }
+  if (e == hipSuccess && !(h->abort_host = take_abort_word())) e = hipErrorOutOfMemory;
   if (e == hipSuccess) e = hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking);
   if (e == hipSuccess) e = hipMalloc((void**)&h->dInfo, sizeof(int));
   for (auto& ev : h->ev)
@@ -3725,18 +3169,17 @@ int blockedLsolve(int n, size_t* Lp, int* Li, double* Lx, int NNZ, size_t* Li_pt
   if (e == hipSuccess)
     e = hipMemcpyAsync(h->dWork, x, sizeof(double) * (size_t)n, hipMemcpyHostToDevice, st);
   if (e == hipSuccess) {
-    enqueue_forward<1>(h, h->dWork, 1, n, h->dY, h->dV);
+    enqueue_forward(h, sweep_run(h, h->dWork, 1, n, h->dY, h->dV, h->dPb));
     e = hipGetLastError();
   }
   if (e == hipSuccess)
     e = hipMemcpyAsync(x, h->dY, sizeof(double) * (size_t)n, hipMemcpyDeviceToHost, st);
-  const hipError_t se = hipStreamSynchronize(st);
-  if (e == hipSuccess) e = se;
+  const int rc = sync_stream(h);
   if (e != hipSuccess) {
     swc_set_error(SWC_EDEVICE, std::string("blockedLsolve: ") + hipGetErrorString(e));
     return 0;
   }
-  return 1;
+  return rc == SWC_OK ? 1 : 0;
 }
 
 }  // extern "C"

@@ -609,6 +609,11 @@ void build_plan(int n, int nsuper, const int* super, const int64_t* pi, const in
     }
   }
 
+  // the backward partials take the place (and at most the room) that the row blocks'
+  // partial sums of one solve level would
+  build_sweeps(nsuper, super, pi, px, voff.data(), prunePtr, pruneSet,
+               (int64_t)std::max(P.max_lvl_fblk, 1) * SPW, P.sweeps);
+
   // ---- flatten: tiles by level (stable), tasks, TRSM lists ----
   // Within a level the most expensive tiles go first (longest-processing-time
   // order), so that the level does not end on a long tile started last.  The
@@ -949,6 +954,19 @@ int swc_plan_sizes(const swc_plan* p, int64_t* out, double* flops) {
   return SWC_OK;
 }
 
+int swc_plan_sweep_sizes(const swc_plan* p, int64_t* out) {
+  if (!p || !out) return swc_set_error(SWC_EINVAL, "swc_plan_sweep_sizes: null argument");
+  const swc::SweepPlan& W = p->P.sweeps;
+  out[0] = (int64_t)W.small.size();
+  out[1] = (int64_t)W.lvl_small.size();
+  out[2] = (int64_t)W.fwd.size();
+  out[3] = (int64_t)W.bwd.size();
+  out[4] = W.psize;
+  out[5] = sizeof(swc::SweepSmall);
+  out[6] = sizeof(swc::SweepItem);
+  return SWC_OK;
+}
+
 int swc_plan_export(const swc_plan* p, int which, void* dst) {
   if (!p || !dst) return swc_set_error(SWC_EINVAL, "swc_plan_export: null argument");
   const swc::Plan& P = p->P;
@@ -981,6 +999,10 @@ int swc_plan_export(const swc_plan* p, int which, void* dst) {
     case 14: return cp(P.spanels);
     case 15: return cp(P.sp_order);
     case 16: return cp(P.lvl_sp);
+    case 24: return cp(P.sweeps.small);
+    case 25: return cp(P.sweeps.lvl_small);
+    case 26: return cp(P.sweeps.fwd);
+    case 27: return cp(P.sweeps.bwd);
     default: return swc_set_error(SWC_EINVAL, "swc_plan_export: unknown array id");
   }
 }

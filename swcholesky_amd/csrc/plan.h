@@ -16,6 +16,8 @@
 #include <cstdint>
 #include <vector>
 
+#include "sweeps.h"
+
 namespace swc {
 
 constexpr int PW = 64;  // panel width (columns)
@@ -170,6 +172,7 @@ struct Plan {
   std::vector<int> lvl_fblk;        // nslevel+1
   std::vector<int> fblk_ptr;        // nsp+1: blocks of sp_order[i]
   int max_lvl_fblk = 0;             // most row blocks in one level
+  SweepPlan sweeps;                 // the solves' work lists
   int64_t diag_scratch = 0;         // doubles of diagonal-block copies one level needs (the
                                     // levels of the dependency-driven launch hold theirs together)
   // dependency-driven factor launch over levels dag_level0 .. nlevel-1 (none when

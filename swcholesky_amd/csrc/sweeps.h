@@ -1,0 +1,72 @@
+// Work lists of the triangular solves, built once per symbolic structure.
+//
+// Each sweep is one persistent launch whose workgroups claim items from a ticket counter
+// in list order and pass each other only vector entries: an entry not yet computed holds
+// a reserved bit pattern, and whoever needs it reads it again until it does not.  L is
+// only read, so no cache is written back or invalidated inside the launch, and there are
+// no launches per level.  Bound: the chain of 64-column panels (about 3 us each: an entry's
+// way through memory, 64 substitution steps), above that HBM.  Per-level launches -> this
+// (ms): 64^3, one right-hand side 4.58 (382 launches) -> 1.55, vector 48^3 with 32 28.4 ->
+// 10.4, a 2D 100^2 solve alone 0.35 -> 0.08.
+//
+// List order is a topological order of the waits: an item waits only for entries that
+// items before it produce.  An item in work has every earlier item claimed by a running
+// workgroup, and the earliest unfinished one never waits for an unfinished one, so the
+// launch cannot deadlock, whatever share of it is resident.
+//
+// A supernode of w columns and m rows below is cut into blocks of 64: column panels and
+// row blocks [64 p, 64 p + 64) of its own rows ("own"), row blocks from row w ("below").
+// Narrow supernodes (w <= 16, m <= kSmallRows) are one wave's work from start to finish.
+#pragma once
+#include <cstdint>
+#include <vector>
+
+namespace swc {
+
+constexpr int kSmallRows = 1024;
+
+// A narrow supernode.
+struct SweepSmall {
+  int64_t vbase;  // value offset of (row 0, column 0)
+  int64_t voff;   // offset of its contribution vector
+  int R, w, c0;   // rows, columns, first global column
+  int rows_off;   // offset into Ls of its row 0
+};
+
+enum SweepKind {
+  kSweepOwn = 0,    // forward: an own row block; backward: a column panel
+  kSweepBelow = 1,  // forward: a row block below; backward: part of a panel's rows below
+  kSweepSmall = 2   // narrow supernodes [first, first + count) of the small list
+};
+
+// Forward: rows [row0, row0 + nr) of the supernode, x of its panels 0 .. nq - 1 applied.
+// Backward: columns [col0, col0 + nr) of panel p, over rows [row0, row1) below (by list)
+// and, for a panel, own row blocks p + 1 .. np - 1; `parts` earlier-made partial sums.
+struct SweepItem {
+  int64_t vbase;  // value offset of the supernode's (row 0, column 0)
+  int64_t out;    // forward below: V offset of row0; backward below: slot in the partials;
+                  // backward own: first slot of its partials
+  int ld, w, c0;  // the supernode's rows, width, first global column
+  int kind;
+  int p;          // own block / panel index
+  int nr;
+  int row0, row1;
+  int nq;         // forward: panels to apply; backward own: number of partials
+  int rows_off;   // offset into Ls of the supernode's row 0
+  int first, count;  // small ones
+};
+
+struct SweepPlan {
+  std::vector<SweepSmall> small;   // by level, ascending
+  std::vector<int> lvl_small;      // small ones of the launches before the persistent one:
+                                   // level l holds [lvl_small[l], lvl_small[l + 1])
+  std::vector<SweepItem> fwd, bwd;
+  int64_t psize = 0;               // doubles of backward partials per right-hand side
+};
+
+// voff[s]: offset of the contribution vector of s.  maxpart: most doubles of partials.
+void build_sweeps(int nsuper, const int* super, const int64_t* pi, const int64_t* px,
+                  const int64_t* voff, const int* prunePtr, const int* pruneSet, int64_t maxpart,
+                  SweepPlan& W);
+
+}  // namespace swc
