@@ -23,6 +23,7 @@
 #include "capi_common.h"
 #include "fronts.h"
 #include "plan.h"
+#include "selinv.h"
 
 using swc::Panel;
 using swc::Plan;
@@ -1246,194 +1247,10 @@ __global__ void k_xpby_cols(double* __restrict__ P, const double* __restrict__ Z
 }
 
 // ---- adjoint: selected inverse on the pattern of L ------------------------
-// Z = A^{-1} restricted to the pattern of L (in L's BCSC layout), by the
-// supernodal Takahashi recurrences, one level of supernodes at a time (four
-// launches), root level first.  For supernode J with L = [L11; L21] (rows R
-// below):
-//   T   = L11^{-1}
-//   U   = L21 T                       (recomputed from L, not stored by the factor)
-//   Z21 = -Z(R,R) U                   (Z(R,R) gathered from the ancestors' Z)
-//   Z11 = T^T T - U^T Z21
-// This is the reverse sweep of the blocked Cholesky adjoint for
-// d logdet(A) / dA = A^{-1} (no reference counterpart).
-
-struct SelinvNode {
-  int64_t vbase;    // value offset of the supernode (row 0, column 0)
-  int64_t scratch;  // offset of its Tt | Ut | Zrr scratch
-  int w, nrow;      // width, rows
-  int c0;           // first column
-  int rows_off;     // offset into Ls
-};
-
-__device__ inline int lower_pos(const int* a, int len, int v) {
-  int lo = 0, hi = len;
-  while (lo < hi) {
-    const int mid = (lo + hi) >> 1;
-    if (a[mid] < v) lo = mid + 1;
-    else hi = mid;
-  }
-  return lo;
-}
-
-// The sweep of one level runs in four launches, each spread over blockIdx.y
-// workgroups per supernode (a level near the root holds one or a few large
-// supernodes).  Scratch per supernode: Tt (W x W, Tt[k W + x] = T(k, x), row
-// major), Ut (m x W, Ut[j W + x] = U(j, x), row major) and Zrr (m x m), so that
-// the threads of a wave (consecutive x or i) read consecutive addresses, and
-// the operand shared by the wave is one broadcast load.  Every entry is
-// accumulated in the same order as a one-thread-per-entry loop would.
-
-// T = L11^{-1}, column j per lane, one wave per workgroup (64 columns from
-// j0): T(i, j) = 0 above the diagonal, T(j, j) = 1 / L(j, j), and below it
-// T(i, j) = -(sum_{k=j}^{i-1} L(i, k) T(k, j)) / L(i, i), the sum taken in
-// increasing k (the wave's columns start it at j0; the terms k < j are zero).
-// Rows go in blocks of 64: a lane keeps its column's sums for the block's rows
-// in registers (x[r]); the finished rows above the block (k < i0) are applied
-// 64 columns of L at a time from LDS (each load of T(k, j) serves 64 rows),
-// then the block's own triangle, row by row, turns x[r] into T(i0 + r, j).
-__global__ void __launch_bounds__(64)
-k_selinv_T(const double* __restrict__ L, const SelinvNode* __restrict__ nodes, int node0,
-           double* __restrict__ arena) {
-  __shared__ double lb[64][64];  // lb[q][r] = L(i0 + r, k0 + q)
-  __shared__ double tl[64][64];  // tl[q][lane] = T(k0 + q, j)
-  const SelinvNode nd = nodes[node0 + blockIdx.x];
-  const int W = nd.w, R = nd.nrow;
-  const int lane = (int)threadIdx.x;
-  const int j0 = blockIdx.y * 64, j = j0 + lane;
-  if (j0 >= W) return;  // the whole workgroup
-  const double* L11 = L + nd.vbase;  // ld R
-  double* Tt = arena + nd.scratch;   // Tt[k W + j] = T(k, j)
-  const bool mine = j < W;
-  for (int i0 = j0; i0 < W; i0 += 64) {
-    const int nb = min(64, W - i0);
-    double x[64];
-#pragma unroll
-    for (int r = 0; r < 64; ++r) x[r] = 0.0;
-    for (int k0 = j0; k0 < i0; k0 += 64) {  // k0 + 63 < i0: whole chunks
-      __syncthreads();  // the previous chunk has been read
-#pragma unroll 16
-      for (int q = 0; q < 64; ++q) {
-        lb[q][lane] = lane < nb ? L11[(int64_t)(k0 + q) * R + i0 + lane] : 0.0;
-        tl[q][lane] = mine ? Tt[(int64_t)(k0 + q) * W + j] : 0.0;
-      }
-      __syncthreads();
-#pragma unroll 1
-      for (int q = 0; q < 64; ++q) {
-        const double t = tl[q][lane];
-#pragma unroll
-        for (int r = 0; r < 64; ++r) {
-          x[r] = fma(lb[q][r], t, x[r]);
-          if (r % 16 == 15) __builtin_amdgcn_sched_barrier(0);  // 16 LDS reads in flight
-        }
-      }
-    }
-    // the block's triangle: lb[c][r] = L(i0 + r, i0 + c)
-    __syncthreads();
-#pragma unroll 8
-    for (int q = 0; q < 64; ++q)
-      lb[q][lane] = lane < nb && i0 + q < W ? L11[(int64_t)(i0 + q) * R + i0 + lane] : 0.0;
-    __syncthreads();
-#pragma unroll
-    for (int r = 0; r < 64; ++r) {
-      const int i = i0 + r;
-      double sum = x[r];
-#pragma unroll
-      for (int c = 0; c < r; ++c) {
-        sum = fma(lb[c][r], x[c], sum);
-        if (c % 16 == 15) __builtin_amdgcn_sched_barrier(0);  // 16 LDS reads in flight
-      }
-      __builtin_amdgcn_sched_barrier(0);
-      const double d = lb[r][r];  // L(i, i) (0 past the block's rows)
-      x[r] = i < j ? 0.0 : (i == j ? 1.0 / d : -sum / d);
-    }
-    if (mine) {
-#pragma unroll
-      for (int r = 0; r < 64; ++r)
-        if (r < nb) Tt[(int64_t)(i0 + r) * W + j] = x[r];
-    }
-  }
-}
-
-// U = L21 T (entry (i, c): sum over k >= c of L21(i, k) T(k, c)), and Zrr = Z(R, R),
-// both triangles, gathered from the ancestors' selected inverse.
-__global__ void __launch_bounds__(kThreads)
-k_selinv_UZ(const double* __restrict__ L, const double* __restrict__ Z,
-            const int* __restrict__ Ls, const int* __restrict__ col2sup,
-            const int64_t* __restrict__ spx, const int* __restrict__ ssuper,
-            const int64_t* __restrict__ spi, const SelinvNode* __restrict__ nodes, int node0,
-            double* __restrict__ arena) {
-  const SelinvNode nd = nodes[node0 + blockIdx.x];
-  const int W = nd.w, R = nd.nrow, m = R - W;
-  const double* L21 = L + nd.vbase + W;  // ld R
-  const double* Tt = arena + nd.scratch;
-  double* Ut = arena + nd.scratch + (int64_t)W * W;
-  double* Zrr = Ut + (int64_t)m * W;
-  const int* rows = Ls + nd.rows_off;
-  const int64_t nU = (int64_t)m * W, nZ = (int64_t)m * m;
-  for (int64_t e = (int64_t)blockIdx.y * kThreads + threadIdx.x; e < nU + nZ;
-       e += (int64_t)gridDim.y * kThreads) {
-    if (e < nU) {
-      const int i = (int)(e % m), c = (int)(e / m);
-      double sum = 0.0;
-      for (int k = c; k < W; ++k) sum = fma(L21[(int64_t)k * R + i], Tt[(int64_t)k * W + c], sum);
-      Ut[(int64_t)i * W + c] = sum;
-    } else {
-      const int64_t f = e - nU;
-      const int i = (int)(f % m), j = (int)(f / m);
-      if (i < j) continue;
-      const int ri = rows[W + i], rj = rows[W + j];
-      const int K = col2sup[rj];
-      const int rk0 = (int)spi[K];
-      const int lenK = (int)(spi[K + 1] - spi[K]);
-      const int pos = lower_pos(Ls + rk0, lenK, ri);
-      const double z = Z[spx[K] + (int64_t)(rj - ssuper[K]) * lenK + pos];
-      Zrr[(int64_t)j * m + i] = z;
-      Zrr[(int64_t)i * m + j] = z;
-    }
-  }
-}
-
-// Z21 = -Zrr U, written into Z (rows W.. of the supernode).
-__global__ void __launch_bounds__(kThreads)
-k_selinv_Z21(double* __restrict__ Z, const SelinvNode* __restrict__ nodes, int node0,
-             const double* __restrict__ arena) {
-  const SelinvNode nd = nodes[node0 + blockIdx.x];
-  const int W = nd.w, R = nd.nrow, m = R - W;
-  const double* Ut = arena + nd.scratch + (int64_t)W * W;
-  const double* Zrr = Ut + (int64_t)m * W;
-  double* Zs = Z + nd.vbase;
-  for (int64_t e = (int64_t)blockIdx.y * kThreads + threadIdx.x; e < (int64_t)m * W;
-       e += (int64_t)gridDim.y * kThreads) {
-    const int i = (int)(e % m), c = (int)(e / m);
-    double sum = 0.0;
-    for (int j = 0; j < m; ++j) sum = fma(Zrr[(int64_t)j * m + i], Ut[(int64_t)j * W + c], sum);
-    Zs[(int64_t)c * R + W + i] = -sum;
-  }
-}
-
-// Z11 = T^T T - U^T Z21 (lower triangle; the strict upper part stays zero).
-__global__ void __launch_bounds__(kThreads)
-k_selinv_Z11(double* __restrict__ Z, const SelinvNode* __restrict__ nodes, int node0,
-             const double* __restrict__ arena) {
-  const SelinvNode nd = nodes[node0 + blockIdx.x];
-  const int W = nd.w, R = nd.nrow, m = R - W;
-  const double* Tt = arena + nd.scratch;
-  const double* Ut = Tt + (int64_t)W * W;
-  double* Zs = Z + nd.vbase;
-  for (int64_t e = (int64_t)blockIdx.y * kThreads + threadIdx.x; e < (int64_t)W * W;
-       e += (int64_t)gridDim.y * kThreads) {
-    const int i = (int)(e % W), c = (int)(e / W);
-    if (i < c) {
-      Zs[(int64_t)c * R + i] = 0.0;
-      continue;
-    }
-    double sum = 0.0;
-    for (int k = i; k < W; ++k) sum = fma(Tt[(int64_t)k * W + i], Tt[(int64_t)k * W + c], sum);
-    double sub = 0.0;
-    for (int j = 0; j < m; ++j) sub = fma(Ut[(int64_t)j * W + i], Zs[(int64_t)c * R + W + j], sub);
-    Zs[(int64_t)c * R + i] = sum - sub;
-  }
-}
+// Z = A^{-1} restricted to the pattern of L (in L's BCSC layout): the reverse sweep of
+// the blocked Cholesky adjoint for d logdet(A) / dA = A^{-1} (no reference counterpart).
+#include "selinv_kernels.h"
+constexpr int kSelLists = 8;
 
 // logdet partials: sum of log L_jj over the diagonal entries (fixed grid).
 __global__ void k_logdet_partial(const double* __restrict__ L, const int64_t* __restrict__ diag,
@@ -1541,18 +1358,18 @@ struct swc_handle {
   double normA = 0;
   // adjoint (selected inverse) state, built on first use
   double* dZ = nullptr;          // selected inverse, xsize
-  double* dArena = nullptr;      // per-level T | U | Zrr scratch
-  SelinvNode* dNodes = nullptr;
-  int* dCol2sup = nullptr;
-  int64_t* dSpx = nullptr;
-  int* dSsuper = nullptr;
-  int64_t* dSpi = nullptr;
+  double* dArena = nullptr;      // Z(R,R) of a level's supernodes
+  double* dSelM = nullptr;       // [T; U] of a chunk of levels
+  swc::SelNode* dNodes = nullptr;
+  swc::SelRun* dSelRuns = nullptr;
+  int* dSelJrun = nullptr;
+  int* dSelRel = nullptr;
+  swc::SelItem* dSelItems = nullptr;  // the plan's item lists
+  size_t sel_items[kSelLists] = {};   // and where each begins
+  swc::SelPlan sel;                   // offsets per chunk and level
   int64_t* dDiagPos = nullptr;   // offset of L(j,j), j in factor order
   int* dQi = nullptr;            // factor-order row / column of every input value
   int* dQj = nullptr;
-  std::vector<int> sel_lvl;      // level -> node offsets (root level first)
-  std::vector<int> sel_wmax;     // per level: widest supernode
-  std::vector<int64_t> sel_emax; // per level: most scratch entries of one supernode
   bool zvalid = false;
   int precision = 0;  // 0 FP64; 1 FP32 descendant updates; 2 FP32 for every update
   int fp32_mask = 0;  // bit k: tasks of kind k use FP32 MFMA
@@ -1601,16 +1418,16 @@ struct swc_handle {
     (void)hipFree(dVals); (void)hipFree(dWork); (void)hipFree(dInfo);
     (void)hipFree(dRp); (void)hipFree(dCi); (void)hipFree(dVmap); (void)hipFree(dAf); (void)hipFree(dNorm); (void)hipFree(dScal); (void)hipFree(dPart); (void)hipFree(dNormPart);
     (void)hipFree(dRef);
-    (void)hipFree(dZ); (void)hipFree(dArena); (void)hipFree(dNodes); (void)hipFree(dCol2sup); (void)hipFree(dSpx);
-    (void)hipFree(dSsuper); (void)hipFree(dSpi); (void)hipFree(dDiagPos); (void)hipFree(dQi); (void)hipFree(dQj);
+    (void)hipFree(dZ); (void)hipFree(dArena); (void)hipFree(dNodes); (void)hipFree(dSelM); (void)hipFree(dSelRuns);
+    (void)hipFree(dSelJrun); (void)hipFree(dSelRel); (void)hipFree(dSelItems); (void)hipFree(dDiagPos); (void)hipFree(dQi); (void)hipFree(dQj);
     dL = nullptr; dLf = nullptr; dLs = nullptr; dTiles = nullptr; dTasks = nullptr;
     dGptr = nullptr; dGidx = nullptr; dSweepSmall = nullptr; dSweepFwd = nullptr; dSweepBwd = nullptr; dSweepSync = nullptr; dV = nullptr; dPb = nullptr; dY = nullptr; dFtiles = nullptr; dFused = nullptr; dGathers = nullptr; dAents = nullptr; dFactorTiles = nullptr; dSmall = nullptr; dFrontTiles = nullptr; dCounters = nullptr; dDagItems = nullptr; dDagDeps = nullptr; dDagSync = nullptr; dDiag = nullptr; dAmap = nullptr; dPerm = nullptr;
     dVals = nullptr; dWork = nullptr; dInfo = nullptr;
     dRp = nullptr; dCi = nullptr; dVmap = nullptr; dAf = nullptr; dNorm = nullptr; dScal = nullptr; dPart = nullptr; dNormPart = nullptr;
     lf_cap = 0;
     dRef = nullptr;
-    dZ = nullptr; dArena = nullptr; dNodes = nullptr; dCol2sup = nullptr; dSpx = nullptr;
-    dSsuper = nullptr; dSpi = nullptr; dDiagPos = nullptr; dQi = nullptr; dQj = nullptr;
+    dZ = nullptr; dArena = nullptr; dNodes = nullptr; dSelM = nullptr; dSelRuns = nullptr;
+    dSelJrun = nullptr; dSelRel = nullptr; dSelItems = nullptr; dDiagPos = nullptr; dQi = nullptr; dQj = nullptr;
     for (auto& e : ev)
       if (e) (void)hipEventDestroy(e);
     for (auto& e : pev) (void)hipEventDestroy(e);
@@ -2239,59 +2056,55 @@ int refine_device(swc_handle* h, const double* Bt, double* Xt, int nrhs, double 
 
 int selinv_setup(swc_handle* h) {
   if (h->dNodes) return SWC_OK;
-  const int ns = h->nsuper;
   hipStream_t st = h->stream;
-  // supernode levels of the descendant DAG; the sweep runs them top-down
-  std::vector<int> lev(ns, 0), col2sup(h->n);
-  int nlev = 0;
-  std::vector<int> pp(h->pruneptr), ps(h->pruneset);
-  for (int s = 0; s < ns; ++s) {
-    for (int t = pp[s]; t < pp[s + 1]; ++t) lev[s] = std::max(lev[s], lev[ps[t]] + 1);
-    nlev = std::max(nlev, lev[s] + 1);
-    for (int c = h->super[s]; c < h->super[s + 1]; ++c) col2sup[c] = s;
-  }
-  std::vector<SelinvNode> nodes;
-  h->sel_lvl.assign(nlev + 1, 0);
-  h->sel_wmax.clear();
-  h->sel_emax.clear();
-  int64_t arena = 0;
-  for (int l = nlev - 1, k = 0; l >= 0; --l, ++k) {
-    int64_t off = 0;
-    for (int s = 0; s < ns; ++s) {
-      if (lev[s] != l) continue;
-      SelinvNode nd;
-      nd.vbase = h->px[s];
-      nd.w = h->super[s + 1] - h->super[s];
-      nd.nrow = (int)(h->pi[s + 1] - h->pi[s]);
-      nd.c0 = h->super[s];
-      nd.rows_off = (int)h->pi[s];
-      nd.scratch = off;
-      const int64_t m = nd.nrow - nd.w;
-      off += (int64_t)nd.w * nd.w + m * nd.w + m * m;
-      nodes.push_back(nd);
-    }
-    h->sel_lvl[k + 1] = (int)nodes.size();
-    arena = std::max(arena, off);
-    int wmax = 0;
-    int64_t emax = 0;
-    for (int q = h->sel_lvl[k]; q < h->sel_lvl[k + 1]; ++q) {
-      const int64_t w = nodes[q].w, m = nodes[q].nrow - nodes[q].w;
-      wmax = std::max<int>(wmax, (int)w);
-      emax = std::max(emax, std::max(w * w, m * w + m * m));
-    }
-    h->sel_wmax.push_back(wmax);
-    h->sel_emax.push_back(emax);
-  }
+  h->sel = swc::build_selinv(h->n, h->nsuper, h->super.data(), h->pi.data(), h->px.data(), h->Ls.data(),
+                             h->pruneptr.data(), h->pruneset.data());
+  swc::SelPlan& S = h->sel;
   int rc = SWC_OK;
-  if (!rc) rc = upload(&h->dNodes, nodes.data(), nodes.size(), st);
-  if (!rc) rc = upload(&h->dCol2sup, col2sup.data(), col2sup.size(), st);
-  if (!rc) rc = upload(&h->dSpx, h->px.data(), h->px.size(), st);
-  if (!rc) rc = upload(&h->dSsuper, h->super.data(), h->super.size(), st);
-  if (!rc) rc = upload(&h->dSpi, h->pi.data(), h->pi.size(), st);
-  if (!rc) rc = upload(&h->dArena, (const double*)nullptr, (size_t)std::max<int64_t>(arena, 1), st);
+  if (!rc) rc = upload(&h->dSelRuns, S.runs.data(), S.runs.size(), st);
+  if (!rc) rc = upload(&h->dSelJrun, S.jrun.data(), S.jrun.size(), st);
+  if (!rc) rc = upload(&h->dSelRel, (const int*)nullptr, (size_t)S.nrel, st);
+  // the item lists, one after the other
+  std::vector<swc::SelItem> items;
+  const std::vector<swc::SelItem>* lists[kSelLists] = {&S.diag,   &S.cols,  &S.u,   &S.gather,
+                                                        &S.small, &S.z21, &S.z11, &S.diag16};
+  size_t total = 0;
+  for (int q = 0; q < kSelLists; ++q) total += lists[q]->size();
+  items.reserve(total);
+  for (int q = 0; q < kSelLists; ++q) {
+    h->sel_items[q] = items.size();
+    items.insert(items.end(), lists[q]->begin(), lists[q]->end());
+  }
+  if (!rc) rc = upload(&h->dSelItems, items.data(), items.size(), st);
+  if (!rc) rc = upload(&h->dSelM, (const double*)nullptr, (size_t)S.msize, st);
+  if (!rc) rc = upload(&h->dArena, (const double*)nullptr, (size_t)S.zsize, st);
   if (!rc) rc = upload(&h->dZ, (const double*)nullptr, (size_t)h->plan.xsize, st);
-  if (rc) return rc;
-  SWC_HIP(hipStreamSynchronize(st));
+  if (!rc) rc = upload(&h->dNodes, S.nodes.data(), S.nodes.size(), st);
+  if (rc) {
+    (void)hipStreamSynchronize(st);  // the uploads read vectors of this frame
+    return rc;
+  }
+  // the strict upper triangles of the diagonal blocks are not written
+  hipError_t e = hipMemsetAsync(h->dZ, 0, sizeof(double) * (size_t)h->plan.xsize, st);
+  if (e == hipSuccess && !S.runs.empty()) {
+    hipLaunchKernelGGL(k_selinv_rel, dim3((unsigned)S.runs.size()), dim3(kThreads), 0, st,
+                       (const int*)h->dLs, (const swc::SelNode*)h->dNodes,
+                       (const swc::SelRun*)h->dSelRuns, h->dSelRel);
+    e = hipGetLastError();
+  }
+  const hipError_t es = hipStreamSynchronize(st);
+  if (e == hipSuccess) e = es;
+  if (e != hipSuccess) {  // the next call starts over
+    (void)hipFree(h->dNodes);
+    h->dNodes = nullptr;
+    SWC_HIP(e);
+  }
+  // the lists are on the device: only the offsets stay
+  for (auto* v : {&S.diag, &S.cols, &S.u, &S.gather, &S.small, &S.z21, &S.z11, &S.diag16})
+    std::vector<swc::SelItem>().swap(*v);
+  std::vector<swc::SelNode>().swap(S.nodes);
+  std::vector<swc::SelRun>().swap(S.runs);
+  std::vector<int>().swap(S.jrun);
   return SWC_OK;
 }
 
@@ -2299,25 +2112,38 @@ int selinv_device(swc_handle* h) {
   if (h->zvalid) return SWC_OK;
   if (int rc = selinv_setup(h)) return rc;
   hipStream_t st = h->stream;
-  const int nl = (int)h->sel_lvl.size() - 1;
-  for (int k = 0; k < nl; ++k) {
-    const int n0 = h->sel_lvl[k], nn = h->sel_lvl[k + 1] - n0;
-    if (nn <= 0) continue;
-    const SelinvNode* nd = (const SelinvNode*)h->dNodes;
-    // workgroups per supernode: one wave per 64 columns of T; for the other
-    // steps about 8 entries per thread of the level's largest supernode
-    const int gt = (h->sel_wmax[k] + 63) / 64;
-    const int ge = (int)std::min<int64_t>(std::max<int64_t>((h->sel_emax[k] + 8 * kThreads - 1) / (8 * kThreads), 1), 1024);
-    hipLaunchKernelGGL(k_selinv_T, dim3(nn, gt), dim3(64), 0, st, (const double*)h->dL, nd, n0,
-                       h->dArena);
-    hipLaunchKernelGGL(k_selinv_UZ, dim3(nn, ge), dim3(kThreads), 0, st, (const double*)h->dL,
-                       (const double*)h->dZ, (const int*)h->dLs, (const int*)h->dCol2sup,
-                       (const int64_t*)h->dSpx, (const int*)h->dSsuper, (const int64_t*)h->dSpi, nd,
-                       n0, h->dArena);
-    hipLaunchKernelGGL(k_selinv_Z21, dim3(nn, ge), dim3(kThreads), 0, st, h->dZ, nd, n0,
-                       (const double*)h->dArena);
-    hipLaunchKernelGGL(k_selinv_Z11, dim3(nn, ge), dim3(kThreads), 0, st, h->dZ, nd, n0,
-                       (const double*)h->dArena);
+  const swc::SelPlan& S = h->sel;
+  const swc::SelNode* nd = h->dNodes;
+  const double* L = h->dL;
+  double* M = h->dSelM;
+  auto list = [&](int q, int first) { return (const swc::SelItem*)h->dSelItems + h->sel_items[q] + first; };
+  for (size_t c = 0; c + 1 < S.chunk_lvl.size(); ++c) {
+    const int d0 = S.chunk_diag[c], nd0 = S.chunk_diag[c + 1] - d0;
+    const int h0 = S.chunk_diag16[c], nh = S.chunk_diag16[c + 1] - h0;
+    const int t0 = S.chunk_cols[c], nt = S.chunk_cols[c + 1] - t0;
+    const int u0 = S.chunk_u[c], nu = S.chunk_u[c + 1] - u0;
+    if (nd0) hipLaunchKernelGGL(k_selinv_diag, dim3(nd0), dim3(64), 0, st, L, nd, list(0, d0), M);
+    if (nh)
+      hipLaunchKernelGGL(k_selinv_diag16, dim3((nh + 15) / 16), dim3(kThreads), 0, st, L, nd, list(7, h0), nh, M);
+    if (nt) hipLaunchKernelGGL(k_selinv_cols, dim3(nt), dim3(kThreads), 0, st, L, nd, list(1, t0), M);
+    if (nu) hipLaunchKernelGGL(k_selinv_U, dim3(nu), dim3(kThreads), 0, st, L, nd, list(2, u0), M);
+    for (int l = S.chunk_lvl[c]; l < S.chunk_lvl[c + 1]; ++l) {
+      const int g0 = S.lvl_gather[l], ng = S.lvl_gather[l + 1] - g0;
+      const int s0 = S.lvl_small[l], nsm = S.lvl_small[l + 1] - s0;
+      const int z0 = S.lvl_z21[l], nz = S.lvl_z21[l + 1] - z0;
+      const int y0 = S.lvl_z11[l], ny = S.lvl_z11[l + 1] - y0;
+      const int ldz = S.lvl_m[l] | 1;
+      const size_t lds = nsm ? sizeof(double) * (size_t)ldz * (2 * 17 + S.lvl_m[l]) : 0;
+      if (nsm + ng)
+        hipLaunchKernelGGL(k_selinv_gather, dim3(nsm + ng), dim3(kThreads), lds, st, h->dZ, (const double*)M,
+                           (const int*)h->dLs, nd, (const swc::SelRun*)h->dSelRuns, (const int*)h->dSelJrun,
+                           (const int*)h->dSelRel, list(4, s0), nsm, ldz, list(3, g0), h->dArena);
+      if (nz)
+        hipLaunchKernelGGL(k_selinv_Z21, dim3(nz), dim3(kThreads), 0, st, h->dZ, (const double*)M,
+                           (const double*)h->dArena, nd, list(5, z0));
+      if (ny)
+        hipLaunchKernelGGL(k_selinv_Z11, dim3(ny), dim3(kThreads), 0, st, h->dZ, (const double*)M, nd, list(6, y0));
+    }
   }
   SWC_HIP(hipGetLastError());
   SWC_HIP(hipStreamSynchronize(st));
