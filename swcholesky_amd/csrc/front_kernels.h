@@ -408,23 +408,7 @@ __device__ inline void small_front_nb(double* __restrict__ L, const swc::SmallFr
   wave_lds_sync();
 #pragma unroll
   for (int c = 0; c < NC; ++c) y[c] += T[lane * (NC + 1) + c];
-  int badcol = 0;
-#pragma unroll
-  for (int j = 0; j < NC; ++j) {
-    if (j < w) {
-      const double d = bcast(y[j], j);
-      const bool ok = d > 0.0;
-      if (!ok && badcol == 0) badcol = j + 1;
-      double r = rsqrt(d);
-      asm volatile("" : "+v"(r));  // a select, not a branch (panel_factor_regs_core)
-      const double rs = ok ? r : 1.0;
-      if (lane == j) y[j] = ok ? d * rs : 1.0;
-      else if (lane > j) y[j] *= rs;
-#pragma unroll
-      for (int c = j + 1; c < NC; ++c)
-        if (c < w) y[c] -= y[j] * bcast(y[j], c);
-    }
-  }
+  const int badcol = factor_rows<NC, false>(y, y, w, lane);
   if (badcol && lane == 0) atomicMin(info_out, f.c0 + badcol);
   double* gl = L + f.vbase;
   float* fl = Lf ? Lf + f.vbase : nullptr;
@@ -595,7 +579,7 @@ k_front_factor(double* __restrict__ L, const swc::SmallFront* __restrict__ small
 inline size_t front_factor_lds(int nwave_items, int widest, int ndefer) {
   size_t d = 0;
   if (nwave_items) d = 4 * kSmallLds;
-  if (widest) d = std::max(d, (size_t)((widest + 15) / 16 * 16 * kWld + 3 * 16 * 16));
+  if (widest) d = std::max(d, (size_t)((widest + 15) / 16 * 16 * kWld));
   if (ndefer) d = std::max(d, (size_t)swc::PW * kTileLd);
   return d * sizeof(double);
 }

@@ -362,6 +362,77 @@ __device__ inline double bcast(double v, int src) {
   return __hiloint2double(hi, lo);
 }
 
+// Lane C of every 16 lanes' own group, in all of them (v_mov_b64_dpp, row_newbcast): half
+// the instructions of bcast, and the value stays in vector registers.
+extern "C" __device__ __attribute__((const)) double swc_update_dpp(double, double, int, int, int,
+                                                                   bool) __asm("llvm.amdgcn.update.dpp.f64");
+template <int C>
+__device__ inline double group_bcast(double v) {
+  return swc_update_dpp(0.0, v, 0x150 + C, 0xf, 0xf, true);
+}
+
+template <int N>
+struct Index {
+  static constexpr int value = N;
+};
+// f(Index<LO>) ... f(Index<HI - 1>): loops whose index is a template argument inside
+template <int LO, int HI, class F>
+__device__ inline void unrolled(F&& f) {
+  if constexpr (LO < HI) {
+    f(Index<LO>{});
+    unrolled<LO + 1, HI>(f);
+  }
+}
+
+// POTRF of a block of nc <= NC columns held by one wave, lane = row (y[c]: column c),
+// and the same column operations on the rows of x (X): x <- x L11^{-T}.  Bound: the chain
+// of nc pivots.  Pivot j + 1 is formed from column j's raw entries, read from their lanes
+// while the reciprocal square root of pivot j runs, so the chain is reciprocal square
+// root, product, fma; the same operations on the same values give the lanes' own copies,
+// bitwise.  Reading it from the updated lane instead puts two lane reads and a select on
+// the chain.  Columns past nc are checked four at a time: what their entries become is
+// not used.  Returns 1 + the first column with a non-positive pivot, else 0; such a
+// pivot continues as 1, so no NaNs spread.
+template <int NC, bool X>
+__device__ inline int factor_rows(double (&y)[NC], double (&x)[NC], int nc, int lane) {
+  int badcol = 0;
+  double d = bcast(y[0], 0);
+#pragma unroll
+  for (int j = 0; j < NC; ++j) {
+    if (j < nc) {
+      const double b1 = j + 1 < NC ? bcast(y[j], j + 1) : 0.0;
+      const double c1 = j + 1 < NC ? bcast(y[j + 1 < NC ? j + 1 : j], j + 1) : 0.0;
+      // 1/sqrt(d) once, then a multiply per entry (dpotf2 scales the column by 1/ajj)
+      double r = rsqrt(d);
+      asm volatile("" : "+v"(r));  // computed whatever d is: a select, not a branch
+      const bool ok = d > 0.0;
+      badcol = ok || badcol != 0 ? badcol : j + 1;
+      const double rs = ok ? r : 1.0;
+      const double m1 = b1 * rs;  // entry (j+1, j)
+      y[j] = ok ? y[j] * rs : (lane == j ? 1.0 : y[j]);
+      if constexpr (X) x[j] *= rs;
+      if (j + 1 < NC) {
+        d = fma(-m1, m1, c1);
+        y[j + 1] = fma(-y[j], m1, y[j + 1]);
+        if constexpr (X) x[j + 1] = fma(-x[j], m1, x[j + 1]);
+      }
+#pragma unroll
+      for (int g = (j + 2) & ~3; g < NC; g += 4) {
+        if (g <= j + 2 || g < nc) {
+#pragma unroll
+          for (int c = g; c < g + 4; ++c) {
+            if (c < j + 2) continue;
+            const double m = bcast(y[j], c);
+            y[c] = fma(-y[j], m, y[c]);
+            if constexpr (X) x[c] = fma(-x[j], m, x[c]);
+          }
+        }
+      }
+    }
+  }
+  return badcol;
+}
+
 // Panel factorization for panels of at most 16 columns (NC), one wave per tile
 // and registers only, for levels with many narrow panels (the leaves, batched
 // instances), where how many workgroups fit on a CU matters more than one
@@ -380,27 +451,9 @@ template <int NC, class TileT>
 __device__ inline void panel_factor_regs_core(double* __restrict__ L, const TileT& tl,
                                               int* __restrict__ info_out, float* __restrict__ Lf,
                                               int lane, double (&y)[NC], double (&x)[NC]) {
-  // y: row `lane` of the diagonal block; x: row `lane` of the tile
+  // y: row `lane` of the diagonal block, 0 past it; x: row `lane` of the tile
   const int nr = tl.nr, nc = tl.ncol;
-  int badcol = 0;
-#pragma unroll
-  for (int j = 0; j < NC; ++j) {
-    if (j < nc) {
-      const double d = bcast(y[j], j);
-      const bool ok = d > 0.0;
-      if (!ok && badcol == 0) badcol = j + 1;
-      // 1/sqrt(d) once, then a multiply per entry (dpotf2 scales the column by
-      // 1/ajj); a non-positive pivot continues with 1 so no NaNs spread
-      double r = rsqrt(d);
-      asm volatile("" : "+v"(r));  // computed whatever d is: a select, not a branch
-      const double rs = ok ? r : 1.0;
-      if (lane == j) y[j] = ok ? d * rs : 1.0;
-      else if (lane > j) y[j] *= rs;
-#pragma unroll
-      for (int c = j + 1; c < NC; ++c)
-        if (c < nc) y[c] -= y[j] * bcast(y[j], c);
-    }
-  }
+  const int badcol = factor_rows<NC, true>(y, x, nc, lane);
   double* gtile = L + tl.vbase + tl.r0;
   float* ftile = Lf ? Lf + tl.vbase + tl.r0 : nullptr;
   if (tl.kind == 0) {
@@ -415,15 +468,6 @@ __device__ inline void panel_factor_regs_core(double* __restrict__ L, const Tile
   // rows of this tile below the diagonal block: tile rows [first, nr)
   const int first = tl.kind == 0 ? nc : 0;
   const bool mine = lane >= first && lane < nr;
-#pragma unroll
-  for (int j = 0; j < NC; ++j) {
-    if (j < nc) {
-      x[j] *= 1.0 / bcast(y[j], j);
-#pragma unroll
-      for (int c = j + 1; c < NC; ++c)
-        if (c < nc) x[c] -= x[j] * bcast(y[j], c);
-    }
-  }
 #pragma unroll
   for (int c = 0; c < NC; ++c)
     if (mine && c < nc) {
@@ -618,6 +662,81 @@ __device__ inline d4 lds_block_update(const double* __restrict__ W, d4 acc, int 
   return acc;
 }
 
+// One sweep over 16 columns: the 16x16 pivot block is factored, z holding its rows in
+// every group of 16 lanes, and each lane's row x solved with it (x <- x L11^{-T}).  Every
+// entry takes its updates in increasing column order.  A wave alone on its SIMD issues an
+// instruction every 4 to 5 cycles, so the sweep costs its instructions, about 36 a
+// column: a multiplier is one move within the lane group (group_bcast) for two fmas, the
+// pivot of column j + 1 is formed from column j's raw entries beside the others' updates,
+// and nothing is selected: a pivot that is not a positive finite number is noticed at the
+// end and the sweep done again with a test in every column (SAFE).  Cycles a column, the
+// kernel's own: multipliers through LDS and selects 328, by readlane 377, this 200.
+// Returns 1 + the first column whose pivot is not positive, else 0; such a pivot
+// continues as 1, so no NaNs spread.
+template <bool SAFE>
+__device__ inline int sweep_columns_as(double (&x)[16], double (&z)[16], int lane, int self, bool* redo) {
+  double d = group_bcast<0>(z[0]);
+  uint64_t ok = ~0ull;
+  int bad = 0;
+  unrolled<0, 16>([&](auto J) {
+    constexpr int j = decltype(J)::value, jn = j < 15 ? j + 1 : 15;
+    const double b1 = group_bcast<jn>(z[j]), c1 = group_bcast<jn>(z[jn]);  // (j+1, j), (j+1, j+1)
+    double r;
+    if constexpr (SAFE) {
+      // 1/sqrt(d) once, then a multiply per entry (dpotf2 scales the column by 1/ajj)
+      r = rsqrt(d);
+      if (!(d > 0.0)) {
+        r = 1.0;
+        if (bad == 0) bad = j + 1;
+        if (self == j) x[j] = 1.0;
+        if ((lane & 15) == j) z[j] = 1.0;
+      }
+    } else {
+      // 1/sqrt(d) = y / sqrt(1 - e), y within 2^-25 of it and e = 1 - d y^2, by the
+      // first terms of the binomial series
+      const double y = __builtin_amdgcn_rsq(d), e = fma(-d * y, y, 1.0);
+      r = fma(y * e, fma(e, 0.375, 0.5), y);
+      ok &= __ballot(__builtin_amdgcn_class(d, 0x180));  // positive, finite
+    }
+    const double m1 = b1 * r;
+    d = fma(-m1, m1, c1);
+    z[j] *= r;
+    x[j] *= r;
+    unrolled<j + 1, 16>([&](auto C) {
+      constexpr int c = decltype(C)::value;
+      const double m = group_bcast<c>(z[j]);
+      z[c] = fma(-z[j], m, z[c]);
+      x[c] = fma(-x[j], m, x[c]);
+    });
+    __builtin_amdgcn_sched_barrier(0);  // the columns' moves hoisted together spill
+  });
+  *redo = ok != ~0ull;
+  return bad;
+}
+// self: the pivot row that this lane's x is, if any
+__device__ inline int sweep_columns(double (&x)[16], double (&z)[16], int lane, int self) {
+  double x0[16], z0[16];
+#pragma unroll
+  for (int c = 0; c < 16; ++c) {
+    x0[c] = x[c];
+    z0[c] = z[c];
+  }
+  bool redo;
+  sweep_columns_as<false>(x, z, lane, self, &redo);
+  // used here: not to be computed behind the branch, with every multiplier kept for it
+#pragma unroll
+  for (int c = 0; c < 16; ++c) asm volatile("" : "+v"(x[c]));
+  if (!redo) return 0;
+#pragma unroll
+  for (int c = 0; c < 16; ++c) {
+    x[c] = x0[c];
+    z[c] = z0[c];
+    // opaque: the first pass's values are not kept for this one
+    asm volatile("" : "+v"(x[c]), "+v"(z[c]));
+  }
+  return sweep_columns_as<true>(x, z, lane, self, &redo);
+}
+
 // Panel factorization of the panels completed at this level for panels of
 // 17..64 columns, one workgroup of four waves per tile: POTRF of the panel's
 // nc x nc diagonal block (dpotrf 'L', sw_parallel_PB_Cholesky_05.c:430) and
@@ -627,26 +746,25 @@ __device__ inline d4 lds_block_update(const double* __restrict__ W, d4 acc, int 
 // The diagonal block (from the launch-invariant copy, identity past nc) and the
 // tile rows sit in LDS (W) from the first load to the final store.  Per block
 // column J:
-//  (1) one sweep over the 16 columns factors the 16x16 diagonal block and
-//      solves every row below it at once, lane = row: wave 0 takes the diagonal
-//      block's rows, waves 1 and 2 the tile rows, each of them also carrying
-//      the 16 pivot rows in lanes 0..15 (the same operations on the same
-//      values, so all three compute the same pivots bitwise).  Each pivot's
-//      reciprocal square root scales its column; the next pivot is read from
-//      its lane (readlane) and the later columns' multipliers from LDS, so the
-//      pivot chain does not wait for LDS;
-//  (2) the later block columns of the diagonal block (blocks on or below its
-//      diagonal) and of the tile rows take the rank-16 update on FP64 MFMA,
-//      the 16x16 output blocks spread over the four waves;
-//  (3) while waves 0-2 sweep block column J, wave 3 stores block column J-1,
-//      which is final, to L, so that only the last block column is stored
-//      after the loop.
+//  (1) one sweep over the 16 columns (sweep_columns) factors the 16x16 diagonal block
+//      and solves every row below it at once, lane = row: wave 0 takes the diagonal
+//      block's rows, wave 1 the tile rows, each with its own copy of the pivot rows
+//      (the same operations on the same values, so both have the same pivots bitwise);
+//  (2) block column J+1 of the diagonal block (blocks on or below its diagonal) and of
+//      the tile rows takes the rank-16 update on FP64 MFMA, the 16x16 output blocks
+//      spread over the four waves;
+//  (3) while waves 0 and 1 sweep block column J, waves 2 and 3 give block column J+1
+//      the updates of the block columns before J, and wave 3 stores block column J-1,
+//      which is final, to L, so that only the last block column is stored after the loop.
+// Bound: latency, of the four sweeps above all (15,200 of a tile's 28,200 cycles at 64
+// columns, loads 4,400; 20,800 of 34,500 with the multipliers through LDS and every
+// block's update between two sweeps).
 // Both apply each entry's updates in increasing column order, so the result is
 // bitwise the one of a column-by-column right-looking factorization.  Every
 // tile of a panel computes the same L11, so no tile waits for another; the
 // diagonal tile stores it and reports info.
-// LDS of k_panel_factor_blk: W, then per sweeping wave column j's multipliers
-constexpr int kBlkLds = swc::PW * kWld + 3 * 16 * 16;
+// LDS of k_panel_factor_blk: W
+constexpr int kBlkLds = swc::PW * kWld;
 
 struct FrontIn;
 __device__ inline void front_assemble_blk(const double* L, const swc::FactorTile& tl,
@@ -663,8 +781,7 @@ __device__ inline void panel_factor_blk_body(double* __restrict__ L, const TileT
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int nc = tl.ncol;
   const int nb = (nc + 15) >> 4;              // 16-column blocks (2..4)
-  double(*lc)[16][16] = reinterpret_cast<double(*)[16][16]>(lds);
-  double* W = lds + 3 * 16 * 16;              // 16 nb columns
+  double* W = lds;                            // 16 nb columns
   const int first = tl.kind == 0 ? nc : 0;    // tile rows [first, nr) are solved ...
   const int nx = tl.nr > first ? tl.nr - first : 0;  // ... into W rows 64 .. 64 + nx
   const int nxb = (nx + 15) >> 4;
@@ -731,95 +848,62 @@ __device__ inline void panel_factor_blk_body(double* __restrict__ L, const TileT
   };
   lds_barrier();
   int badcol = 0;
-  // (1) this lane's W row in block column jb/16 (wave 3 only reads one); the
-  // lane holding pivot row jb + j is pbase + j.  Every wave has read its rows
-  // before any is written back (waves 1 and 2 read the pivot rows that wave 0
-  // rewrites): a barrier follows every read.
-  auto sweep_row = [&](int jb) {
-    return wave == 0 ? lane
-                     : (wave == 3 || lane < 16 || (wave == 2 && lane >= 32)
-                            ? jb + (lane & 15)
-                            : 64 + 48 * (wave - 1) + (lane - 16));
-  };
-  double x[16];
+  // Every wave has read its rows before any is written back (wave 1 reads the pivot rows
+  // that wave 0 rewrites): a barrier follows every read.
+  double x[16], z[16];
   auto read_row = [&](int jb) {
-    const int row = sweep_row(jb);
+    if (wave >= 2) return;
 #pragma unroll
-    for (int c = 0; c < 16; ++c) x[c] = W[(jb + c) * kWld + row];
+    for (int c = 0; c < 16; ++c) {
+      z[c] = W[(jb + c) * kWld + jb + (lane & 15)];
+      x[c] = W[(jb + c) * kWld + 64 * wave + lane];
+    }
   };
   read_row(0);
   lds_barrier();
   for (int J = 0; J < nb; ++J) {
     const int jb = 16 * J;
-    const int row = sweep_row(jb);
-    if (wave < 3) {
-      const int pbase = wave == 0 ? jb : 0;
-      const bool store = wave == 0 ? (lane >= jb && lane < 16 * nb)
-                                   : (lane >= 16 && row - 64 < nx && (wave == 1 || lane < 32));
-      double(*mult)[16] = lc[wave];
-      double d = bcast(x[0], pbase);
-      // Software-pipelined over the columns: column j's multiplier for column
-      // j + 1 (the entry (j+1, j), needed by the next pivot) comes by readlane;
-      // its multipliers for the columns after that go through LDS and are
-      // applied one column later, so no LDS round trip sits on the pivot chain.
-      // Every entry still takes its updates in increasing column order.
-      double pm[16];  // column j-1's multipliers, read from LDS during column j-1
-#pragma unroll
-      for (int c = 0; c < 16; ++c) pm[c] = 0.0;
-#pragma unroll
-      for (int j = 0; j < 16; ++j) {
-        // x[j] has every update from the columns before j
-        // 1/sqrt(d) once, then a multiply per entry (dpotf2 scales the column
-        // by 1/ajj).  A non-positive pivot is reported and continues as 1, so
-        // no NaNs spread.  Selects rather than a branch: the test on d runs
-        // beside the reciprocal square root instead of before it.
-        double r = rsqrt(d);
-        asm volatile("" : "+v"(r));  // computed whatever d is, not under a branch
-        const bool pos = d > 0.0;
-        badcol = pos || badcol != 0 ? badcol : jb + j + 1;
-        x[j] = pos ? x[j] * r : (lane == pbase + j ? 1.0 : x[j]);
-        if (j < 15) {
-          const double m1 = bcast(x[j], pbase + j + 1);  // entry (j+1, j)
-          if (j >= 1) x[j + 1] -= x[j - 1] * pm[j + 1];
-          x[j + 1] -= x[j] * m1;
-          // the next pivot: its lane's x[j+1], now updated by every earlier column
-          d = bcast(x[j + 1], pbase + j + 1);
-          if (lane >= pbase && lane < pbase + 16) mult[j][lane - pbase] = x[j];
-          if (j >= 1) {
-#pragma unroll
-            for (int c = j + 2; c < 16; ++c) x[c] -= x[j - 1] * pm[c];
-          }
-#pragma unroll
-          for (int c = j + 2; c < 16; ++c) pm[c] = mult[j][c];
-        }
-      }
+    if (wave < 2) {
+      const bool store = wave == 0 ? (lane >= jb && lane < 16 * nb) : lane < nx;
+      const int bad = sweep_columns(x, z, lane, wave == 0 ? lane - jb : -1);
+      badcol = badcol != 0 || bad == 0 ? badcol : jb + bad;
       if (store) {
 #pragma unroll
-        for (int c = 0; c < 16; ++c) W[(jb + c) * kWld + row] = x[c];
+        for (int c = 0; c < 16; ++c) W[(jb + c) * kWld + 64 * wave + lane] = x[c];
       }
     } else if (J > 0) {
-      // block column J - 1 is final (the updates after its sweep touch later
-      // columns only): wave 3 writes it back while the others sweep
-      write_back(jb - 16, 1, 16);
-    }
-    lds_barrier();
-    if (J + 1 < nb) {
-      // (2) block columns C > J: rows of the diagonal block from C on, then the
-      // tile rows (W row blocks 4 .. 4 + nxb)
-      int idx = 0;
-      for (int C = J + 1; C < nb; ++C) {
-        const int nrb = (nb - C) + nxb;
-        for (int q = 0; q < nrb; ++q, ++idx) {
-          if ((idx & 3) != wave) continue;
+      // beside the sweep, waves 2 and 3: the updates of block column J + 1 from the
+      // block columns before J; then wave 3 writes block column J - 1, which is final,
+      // to L
+      if (J + 1 < nb) {
+        const int C = J + 1, nrb = (nb - C) + nxb;
+        for (int q = wave - 2; q < nrb; q += 2) {
           const int R = q < nb - C ? C + q : 4 + (q - (nb - C));
           double* out = W + (16 * C + (lane & 15)) * kWld + 16 * R + (lane >> 4);
           d4 acc = d4{out[0], out[4], out[8], out[12]};
-          acc = lds_block_update(W, acc, R, C, jb, lane);
+          for (int kb = 0; kb < jb; kb += 16) acc = lds_block_update(W, acc, R, C, kb, lane);
           out[0] = acc[0];
           out[4] = acc[1];
           out[8] = acc[2];
           out[12] = acc[3];
         }
+      }
+      if (wave == 3) write_back(jb - 16, 1, 16);
+    }
+    lds_barrier();
+    if (J + 1 < nb) {
+      // (2) block column C = J + 1: rows of the diagonal block from C on, then the
+      // tile rows (W row blocks 4 .. 4 + nxb)
+      const int C = J + 1, nrb = (nb - C) + nxb;
+      for (int q = wave; q < nrb; q += 4) {
+        const int R = q < nb - C ? C + q : 4 + (q - (nb - C));
+        double* out = W + (16 * C + (lane & 15)) * kWld + 16 * R + (lane >> 4);
+        d4 acc = d4{out[0], out[4], out[8], out[12]};
+        acc = lds_block_update(W, acc, R, C, jb, lane);
+        out[0] = acc[0];
+        out[4] = acc[1];
+        out[8] = acc[2];
+        out[12] = acc[3];
       }
       lds_barrier();
       read_row(jb + 16);
