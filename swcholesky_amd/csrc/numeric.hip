@@ -1146,6 +1146,7 @@ __global__ void k_permute(const double* __restrict__ in, double* __restrict__ ou
 // ---- residual, norms and vector updates (FP64) ---------------------------
 
 constexpr int kRedBlocks = 512;
+constexpr int kSetupBlocks = 2048;
 
 // Workspace of swc_solve_noalloc, the entry point that allocates nothing: one
 // copy of this array per GPU, held from the library's load until the process
@@ -1154,30 +1155,39 @@ constexpr int kRedBlocks = 512;
 constexpr int64_t kScratchDoubles = (int64_t)16 << 20;  // 128 MiB
 static __device__ __align__(256) double scratch[kScratchDoubles];
 
-// Pinned host words that a sweep sets when one of its waits runs out, one per handle: taken
-// in swc_create and given back in swc_destroy, in blocks that are kept for later handles.
-std::mutex g_abort_mu;
-std::vector<int*> g_abort_free;
+// What kernels report to the host, in pinned memory (a kernel's store is on the host when
+// the stream is, without a copy command and its gap, 14 to 45 us each): one per handle,
+// taken in swc_create and given back in swc_destroy, in blocks that are kept for later
+// handles.
+struct HostRecord {
+  int abort;      // set when one of a sweep's waits ran out
+  int info;       // of the factor
+  double norm;    // ||A||_inf
+  double logdet;  // sum of log L_jj
+  double pad;
+};
+std::mutex g_record_mu;
+std::vector<HostRecord*> g_record_free;
 
-int* take_abort_word() {
-  std::lock_guard<std::mutex> lock(g_abort_mu);
-  if (g_abort_free.empty()) {
-    constexpr int kWords = 1024;
-    int* block = nullptr;
-    if (hipHostMalloc((void**)&block, kWords * sizeof(int), hipHostMallocPortable) != hipSuccess)
+HostRecord* take_record() {
+  std::lock_guard<std::mutex> lock(g_record_mu);
+  if (g_record_free.empty()) {
+    constexpr int kRecords = 256;
+    HostRecord* block = nullptr;
+    if (hipHostMalloc((void**)&block, kRecords * sizeof(HostRecord), hipHostMallocPortable) != hipSuccess)
       return nullptr;
-    for (int i = 0; i < kWords; ++i) g_abort_free.push_back(block + i);
+    for (int i = 0; i < kRecords; ++i) g_record_free.push_back(block + i);
   }
-  int* w = g_abort_free.back();
-  g_abort_free.pop_back();
-  *w = 0;
-  return w;
+  HostRecord* r = g_record_free.back();
+  g_record_free.pop_back();
+  *r = HostRecord{};
+  return r;
 }
 
-void give_abort_word(int* w) {
-  if (!w) return;
-  std::lock_guard<std::mutex> lock(g_abort_mu);
-  g_abort_free.push_back(w);
+void give_record(HostRecord* r) {
+  if (!r) return;
+  std::lock_guard<std::mutex> lock(g_record_mu);
+  g_record_free.push_back(r);
 }
 
 // Per-device address of `scratch`, looked up once per device with that device
@@ -1201,14 +1211,6 @@ int bind_scratch(int device) {
 double* scratch_ptr(int device) {
   std::lock_guard<std::mutex> lock(g_scratch_mu);
   return device < (int)g_scratch_ptr.size() ? g_scratch_ptr[device] : nullptr;
-}
-
-// Af[e] = vals[vmap[e]]: the full P A P^T values in CSR order, from the caller's values.
-__global__ void k_gather(double* __restrict__ out, const double* __restrict__ vals,
-                         const int64_t* __restrict__ vmap, int64_t nnz) {
-  for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < nnz;
-       e += (int64_t)gridDim.x * blockDim.x)
-    out[e] = vals[vmap[e]];
 }
 
 // Y = A X, or R = B - A X when B is given, for all nrhs columns (CSR): a group
@@ -1252,23 +1254,59 @@ k_csr_mv(const int* __restrict__ rp, const int* __restrict__ ci, const double* _
   }
 }
 
-// Partial maxima of the row sums of |A| (||A||_inf), one per block of a fixed grid.
-__global__ void k_norm_inf(const int* __restrict__ rp, const double* __restrict__ av, int n,
-                           double* __restrict__ part) {
-  __shared__ double red[kThreads];
+// First launch of a factorization: the values into the handle's copy (keep, unless they
+// are there already), the full symmetric matrix in CSR for the residuals (both triangles,
+// entry e from value vmap[e]) and its row sums' maxima, part[block] (||A||_inf), and a
+// clean info word.  G lanes a row, as its length asks (setup_group).  Bound: HBM and the
+// latency of vmap -> value.  A 1100-row dense matrix took 222 us for the norm alone with a
+// thread per row; the whole launch is 15 us.
+template <int G>
+__global__ void __launch_bounds__(kThreads)
+k_factor_setup(const double* __restrict__ vals, double* __restrict__ keep, int64_t nvals,
+               const int* __restrict__ rp, const int64_t* __restrict__ vmap, int n,
+               double* __restrict__ af, double* __restrict__ part, int* __restrict__ info) {
+  __shared__ double red[kThreads / 64];
+  const int64_t t0 = (int64_t)blockIdx.x * kThreads + threadIdx.x, nt = (int64_t)gridDim.x * kThreads;
+  if (t0 == 0) *info = 0x7fffffff;
+  if (keep)
+    for (int64_t q = t0; q < nvals; q += nt) keep[q] = vals[q];
+  const int k = (int)(t0 % G);
   double m = 0.0;
-  for (int i = blockIdx.x * kThreads + threadIdx.x; i < n; i += kRedBlocks * kThreads) {
+  for (int64_t i0 = t0 / G; i0 < n; i0 += nt / G) {
+    const int e1 = rp[i0 + 1];
     double t = 0.0;
-    for (int e = rp[i]; e < rp[i + 1]; ++e) t += fabs(av[e]);
+#pragma unroll 4
+    for (int e = rp[i0] + k; e < e1; e += G) {
+      const double v = vals[vmap[e]];
+      af[e] = v;
+      t += fabs(v);
+    }
+#pragma unroll
+    for (int w = G / 2; w > 0; w >>= 1) t += __shfl_xor(t, w, G);
     m = fmax(m, t);
   }
-  red[threadIdx.x] = m;
+#pragma unroll
+  for (int w = 32; w > 0; w >>= 1) m = fmax(m, __shfl_xor(m, w, 64));
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
   __syncthreads();
-  for (int w = kThreads / 2; w > 0; w >>= 1) {
-    if (threadIdx.x < w) red[threadIdx.x] = fmax(red[threadIdx.x], red[threadIdx.x + w]);
-    __syncthreads();
+  if (threadIdx.x == 0) part[blockIdx.x] = fmax(fmax(red[0], red[1]), fmax(red[2], red[3]));
+}
+
+// Last launch of a factorization: its info and ||A||_inf to the host's record.
+__global__ void __launch_bounds__(kThreads)
+k_factor_report(const double* __restrict__ part, int npart, const int* __restrict__ info,
+                HostRecord* __restrict__ rec) {
+  __shared__ double red[kThreads / 64];
+  double m = 0.0;
+  for (int i = threadIdx.x; i < npart; i += kThreads) m = fmax(m, part[i]);
+#pragma unroll
+  for (int w = 32; w > 0; w >>= 1) m = fmax(m, __shfl_xor(m, w, 64));
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    rec->norm = fmax(fmax(red[0], red[1]), fmax(red[2], red[3]));
+    rec->info = *info;
   }
-  if (threadIdx.x == 0) part[blockIdx.x] = red[0];
 }
 
 // Per-column partial reductions over a fixed grid (deterministic): op 0 max|x|,
@@ -1401,7 +1439,7 @@ struct swc_handle {
   swc::SweepItem* dSweepFwd = nullptr;
   swc::SweepItem* dSweepBwd = nullptr;
   int* dSweepSync = nullptr;  // tickets of the two sweeps, abort flag
-  int* abort_host = nullptr;  // pinned: a sweep's wait ran out (a slot of the abort pool)
+  HostRecord* rec = nullptr;  // pinned
   double* dV = nullptr;   // contribution vectors, vsize * work_cols
   double* dPb = nullptr;  // backward partial sums, max_lvl_fblk * SPW * work_cols
   double* dY = nullptr;   // forward solutions, n * work_cols
@@ -1434,7 +1472,6 @@ struct swc_handle {
   // small device scalars written by captured launch sequences ([0] ||A||_inf,
   // [1] logdet): allocated with the structure and never moved while a graph
   // that writes them exists
-  double* dNorm = nullptr;
   double* dScal = nullptr;   // refinement scalars, sized by ensure_work (eager launches only)
   double* dNormPart = nullptr;  // kRedBlocks partial maxima of ||A||_inf
   double* dPart = nullptr;   // reduction partials, kRedBlocks * work_cols
@@ -1469,6 +1506,7 @@ struct swc_handle {
     const double* x;
     int nrhs;
     int64_t ld;
+    bool marked;
     hipGraphExec_t exec;
   };
   std::vector<SolveGraph> sgraphs;
@@ -1484,7 +1522,7 @@ struct swc_handle {
 
   ~swc_handle() {
     release();
-    give_abort_word(abort_host);
+    give_record(rec);
   }
   void drop_graphs() {
     for (auto& g : fgraph)
@@ -1500,14 +1538,14 @@ struct swc_handle {
     (void)hipFree(dGathers); (void)hipFree(dAents); (void)hipFree(dFactorTiles); (void)hipFree(dSmall); (void)hipFree(dFrontTiles);
     (void)hipFree(dCounters); (void)hipFree(dDagItems); (void)hipFree(dDagDeps); (void)hipFree(dDagSync); (void)hipFree(dDiag); (void)hipFree(dAmap); (void)hipFree(dPerm);
     (void)hipFree(dVals); (void)hipFree(dWork); (void)hipFree(dInfo);
-    (void)hipFree(dRp); (void)hipFree(dCi); (void)hipFree(dVmap); (void)hipFree(dAf); (void)hipFree(dNorm); (void)hipFree(dScal); (void)hipFree(dPart); (void)hipFree(dNormPart);
+    (void)hipFree(dRp); (void)hipFree(dCi); (void)hipFree(dVmap); (void)hipFree(dAf); (void)hipFree(dScal); (void)hipFree(dPart); (void)hipFree(dNormPart);
     (void)hipFree(dRef);
     (void)hipFree(dZ); (void)hipFree(dArena); (void)hipFree(dNodes); (void)hipFree(dSelM); (void)hipFree(dSelRuns);
     (void)hipFree(dSelJrun); (void)hipFree(dSelRel); (void)hipFree(dSelItems); (void)hipFree(dDiagPos); (void)hipFree(dQi); (void)hipFree(dQj);
     dL = nullptr; dLf = nullptr; dLs = nullptr; dTiles = nullptr; dTasks = nullptr;
     dGptr = nullptr; dGidx = nullptr; dSweepSmall = nullptr; dSweepFwd = nullptr; dSweepBwd = nullptr; dSweepSync = nullptr; dV = nullptr; dPb = nullptr; dY = nullptr; dFtiles = nullptr; dFused = nullptr; dGathers = nullptr; dAents = nullptr; dFactorTiles = nullptr; dSmall = nullptr; dFrontTiles = nullptr; dCounters = nullptr; dDagItems = nullptr; dDagDeps = nullptr; dDagSync = nullptr; dDiag = nullptr; dAmap = nullptr; dPerm = nullptr;
     dVals = nullptr; dWork = nullptr; dInfo = nullptr;
-    dRp = nullptr; dCi = nullptr; dVmap = nullptr; dAf = nullptr; dNorm = nullptr; dScal = nullptr; dPart = nullptr; dNormPart = nullptr;
+    dRp = nullptr; dCi = nullptr; dVmap = nullptr; dAf = nullptr; dScal = nullptr; dPart = nullptr; dNormPart = nullptr;
     lf_cap = 0;
     dRef = nullptr;
     dZ = nullptr; dArena = nullptr; dNodes = nullptr; dSelM = nullptr; dSelRuns = nullptr;
@@ -1642,6 +1680,28 @@ void enqueue_fronts(swc_handle* h, bool profile) {
   }
 }
 
+// Lanes per row of k_factor_setup, and its workgroups.  8 lanes take rows of a grid or a
+// mesh (5 to 30 entries, vector operators up to 81) in a few steps; a row of more than 64
+// on average gets a wave.  8 against 64 lanes: 100^2 grid 3.2 us against 5.4, 32^3 4.4
+// against 10.5, vector 20^3 6.4 against 9.3, a 1100-row dense matrix 46 against 15.
+int setup_group(const swc_handle* h) { return h->nnz_full > (int64_t)64 * h->n ? 64 : 8; }
+int setup_blocks(const swc_handle* h) {
+  return (int)std::min<int64_t>(((int64_t)h->n * setup_group(h) + kThreads - 1) / kThreads, kSetupBlocks);
+}
+
+// The launch before the factor's graph: it reads the caller's values, whose address the
+// graph does not know.
+void launch_setup(swc_handle* h, const double* dvals) {
+  auto kern = setup_group(h) == 64 ? k_factor_setup<64> : k_factor_setup<8>;
+  hipLaunchKernelGGL(kern, dim3(setup_blocks(h)), dim3(kThreads), 0, h->stream, dvals,
+                     dvals != h->dVals ? h->dVals : nullptr, h->nvals, (const int*)h->dRp,
+                     (const int64_t*)h->dVmap, h->n, h->dAf, h->dNormPart, h->dInfo);
+}
+void launch_report(swc_handle* h) {
+  hipLaunchKernelGGL(k_factor_report, dim3(1), dim3(kThreads), 0, h->stream, (const double*)h->dNormPart,
+                     setup_blocks(h), (const int*)h->dInfo, h->rec);
+}
+
 // Enqueues the whole numeric factorization of the staged values h->dVals.
 void enqueue_factor(swc_handle* h, bool profile) {
   hipStream_t st = h->stream;
@@ -1650,28 +1710,15 @@ void enqueue_factor(swc_handle* h, bool profile) {
   if (h->multifrontal) {
     // L needs no clearing: every entry on and below a diagonal block's diagonal is
     // written by a factor launch, and what lies above is cleared at upload
-    hipLaunchKernelGGL(k_gather, dim3(grid_for(h->nnz_full)), dim3(kThreads), 0, st, h->dAf, dvals,
-                       (const int64_t*)h->dVmap, h->nnz_full);
-    hipLaunchKernelGGL(k_norm_inf, dim3(kRedBlocks), dim3(kThreads), 0, st, (const int*)h->dRp,
-                       (const double*)h->dAf, h->n, h->dNormPart);
-    hipLaunchKernelGGL(k_reduce_final, dim3(1), dim3(kThreads), 0, st,
-                       (const double*)h->dNormPart, 0, h->dNorm);
-    hipLaunchKernelGGL(k_set_int, dim3(1), dim3(1), 0, st, h->dInfo, 0x7fffffff);
     if (h->precision == 0) enqueue_fronts<0>(h, profile);
     else if (h->precision == 1) enqueue_fronts<1>(h, profile);
     else enqueue_fronts<2>(h, profile);
+    launch_report(h);
     return;
   }
   hipLaunchKernelGGL(k_fill, dim3(grid_for(P.xsize)), dim3(kThreads), 0, st, h->dL, P.xsize, 0.0);
   hipLaunchKernelGGL(k_assemble, dim3(grid_for(h->nvals)), dim3(kThreads), 0, st, h->dL,
                      (const int64_t*)h->dAmap, dvals, h->nvals);
-  hipLaunchKernelGGL(k_gather, dim3(grid_for(h->nnz_full)), dim3(kThreads), 0, st, h->dAf, dvals,
-                     (const int64_t*)h->dVmap, h->nnz_full);
-  hipLaunchKernelGGL(k_norm_inf, dim3(kRedBlocks), dim3(kThreads), 0, st, (const int*)h->dRp,
-                     (const double*)h->dAf, h->n, h->dNormPart);
-  hipLaunchKernelGGL(k_reduce_final, dim3(1), dim3(kThreads), 0, st, (const double*)h->dNormPart, 0,
-                     h->dNorm);
-  hipLaunchKernelGGL(k_set_int, dim3(1), dim3(1), 0, st, h->dInfo, 0x7fffffff);
   hipLaunchKernelGGL(k_fill_int, dim3((std::max(P.nlevel, 1) + kThreads - 1) / kThreads),
                      dim3(kThreads), 0, st, h->dCounters, std::max(P.nlevel, 1), 0);
   // the levels from dag_level0 on run as one dependency-driven launch (per-level
@@ -1755,14 +1802,13 @@ void enqueue_factor(swc_handle* h, bool profile) {
                        (const swc::DagDep*)h->dDagDeps, h->dDagSync, h->dDiag, h->dInfo, h->dLf,
                        h->fp32_mask ? 1 : 0);
   }
+  launch_report(h);
 }
 
 // Numeric factorization from values on the device (in upload order).
 int factor_device(swc_handle* h, const double* dvals) {
   hipStream_t st = h->stream;
   const Plan& P = h->plan;
-  if (dvals != h->dVals)
-    SWC_HIP(hipMemcpyAsync(h->dVals, dvals, sizeof(double) * h->nvals, hipMemcpyDeviceToDevice, st));
   const int nlevel = h->multifrontal ? h->fronts.nlevel : P.nlevel;
   if (h->profile && h->pev.size() < (size_t)4 * nlevel) {
     for (auto& e : h->pev) (void)hipEventDestroy(e);
@@ -1784,23 +1830,21 @@ int factor_device(swc_handle* h, const double* dvals) {
     }
   }
   SWC_HIP(hipEventRecord(h->ev[0], st));
+  launch_setup(h, dvals);
   if (graph) SWC_HIP(hipGraphLaunch(gx, st));
   else enqueue_factor(h, h->profile);
   SWC_HIP(hipEventRecord(h->ev[1], st));
   SWC_HIP(hipGetLastError());
   const int big = 0x7fffffff;
-  int info = 0;
-  // both copies target host memory of this frame and the handle: the stream is
-  // synchronized before any return, also when a copy fails to enqueue
-  hipError_t ce = hipMemcpyAsync(&info, h->dInfo, sizeof(int), hipMemcpyDeviceToHost, st);
-  if (ce == hipSuccess)
-    ce = hipMemcpyAsync(&h->normA, h->dNorm, sizeof(double), hipMemcpyDeviceToHost, st);
+  hipError_t ce = hipSuccess;
   int dag_abort = 0;
   const bool dag = !h->profile && !P.dag_items.empty();
   if (ce == hipSuccess && dag)
     ce = hipMemcpyAsync(&dag_abort, h->dDagSync + 1, sizeof(int), hipMemcpyDeviceToHost, st);
   SWC_HIP(hipStreamSynchronize(st));
   SWC_HIP(ce);
+  const int info = h->rec->info;
+  h->normA = h->rec->norm;
   if (dag_abort) {
     h->factored = false;
     return swc_set_error(SWC_EDEVICE, "factor: a dependency wait of the factor launch timed out");
@@ -1881,7 +1925,7 @@ SweepRun sweep_run(swc_handle* h, double* dX, int nrhs, int64_t ldx, double* dY,
   a.gidx = h->dGidx;
   a.small = h->dSweepSmall;
   a.abort_flag = h->dSweepSync + 2;
-  a.abort_host = h->abort_host;
+  a.abort_host = &h->rec->abort;
   a.X = dX;
   a.Y = dY;
   a.V = dV;
@@ -1894,12 +1938,19 @@ SweepRun sweep_run(swc_handle* h, double* dX, int nrhs, int64_t ldx, double* dY,
   return a;
 }
 
-// Forward sweep L Y = X (X is left marked for the backward sweep).
-void enqueue_forward(swc_handle* h, SweepRun a) {
-  const swc::SweepPlan& W = h->plan.sweeps;
+// The marks that the sweeps of `a` start from; X = P in on the way when `in` is given.
+void enqueue_marks(swc_handle* h, const SweepRun& a, const double* in, int64_t ldin) {
   const int64_t ny = a.ldy * a.nrhs, nv = a.ldv * a.nrhs, np = a.ldp * a.nrhs;
   hipLaunchKernelGGL(k_sweep_init, dim3(std::min(grid_for(std::max(ny, nv)), 4096)), dim3(kThreads),
-                     0, h->stream, a.Y, ny, a.V, nv, a.P, np, h->dSweepSync);
+                     0, h->stream, a.Y, ny, a.V, nv, a.P, np, h->dSweepSync, in, ldin, a.X, a.ldx,
+                     (const int*)h->dPerm, h->n, a.nrhs);
+}
+
+// Forward sweep L Y = X (X is left marked for the backward sweep); marked: its
+// enqueue_marks has been launched.
+void enqueue_forward(swc_handle* h, SweepRun a, bool marked = false) {
+  const swc::SweepPlan& W = h->plan.sweeps;
+  if (!marked) enqueue_marks(h, a, nullptr, 0);
   for (int l = 0; l + 1 < (int)W.lvl_small.size(); ++l) launch_small<true>(h, a, l);
   a.items = h->dSweepFwd;
   a.nitems = (int)W.fwd.size();
@@ -1922,32 +1973,32 @@ void enqueue_backward(swc_handle* h, SweepRun a) {
 // dY (n x nrhs), dV (max(vsize, 1) x nrhs) and dPb (max(max_lvl_fblk, 1) SPW x nrhs, which
 // holds the backward partials) are the sweeps' workspace.
 void enqueue_solve_bufs(swc_handle* h, double* dX, int nrhs, int64_t ldx, double* dY, double* dV,
-                        double* dPb) {
+                        double* dPb, bool marked = false) {
   const SweepRun a = sweep_run(h, dX, nrhs, ldx, dY, dV, dPb);
-  enqueue_forward(h, a);
+  enqueue_forward(h, a, marked);
   enqueue_backward(h, a);
 }
 
 // Waits for the handle's stream; an error where a sweep's wait ran out.
 int sync_stream(swc_handle* h) {
   SWC_HIP(hipStreamSynchronize(h->stream));
-  if (__atomic_exchange_n(h->abort_host, 0, __ATOMIC_RELAXED) != 0)
+  if (__atomic_exchange_n(&h->rec->abort, 0, __ATOMIC_RELAXED) != 0)
     return swc_set_error(SWC_EDEVICE, "solve: a wait inside a sweep ran out of time");
   return SWC_OK;
 }
 
-void enqueue_solve(swc_handle* h, double* dX, int nrhs, int64_t ldx) {
-  enqueue_solve_bufs(h, dX, nrhs, ldx, h->dY, h->dV, h->dPb);
+void enqueue_solve(swc_handle* h, double* dX, int nrhs, int64_t ldx, bool marked) {
+  enqueue_solve_bufs(h, dX, nrhs, ldx, h->dY, h->dV, h->dPb, marked);
 }
 
 // In-place solve of L L^T X = B on device columns X (factor ordering); needs
 // ensure_work(h, nrhs).
-int solve_device(swc_handle* h, double* dX, int nrhs, int64_t ldx) {
+int solve_device(swc_handle* h, double* dX, int nrhs, int64_t ldx, bool marked) {
   hipStream_t st = h->stream;
   hipGraphExec_t gx = nullptr;
   if (h->use_graphs) {
     for (auto& g : h->sgraphs)
-      if (g.x == dX && g.nrhs == nrhs && g.ld == ldx) gx = g.exec;
+      if (g.x == dX && g.nrhs == nrhs && g.ld == ldx && g.marked == marked) gx = g.exec;
     if (!gx) {
       if (h->sgraphs.size() >= 8) {
         (void)hipGraphExecDestroy(h->sgraphs.front().exec);
@@ -1955,17 +2006,17 @@ int solve_device(swc_handle* h, double* dX, int nrhs, int64_t ldx) {
       }
       hipGraph_t g = nullptr;
       SWC_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-      enqueue_solve(h, dX, nrhs, ldx);
+      enqueue_solve(h, dX, nrhs, ldx, marked);
       SWC_HIP(hipStreamEndCapture(st, &g));
       hipError_t e = hipGraphInstantiate(&gx, g, nullptr, nullptr, 0);
       (void)hipGraphDestroy(g);
       if (e != hipSuccess) return swc_set_error(SWC_EDEVICE, std::string("solve graph: ") + hipGetErrorString(e));
-      h->sgraphs.push_back({dX, nrhs, ldx, gx});
+      h->sgraphs.push_back({dX, nrhs, ldx, marked, gx});
     }
   }
   SWC_HIP(hipEventRecord(h->ev[2], st));
   if (gx) SWC_HIP(hipGraphLaunch(gx, st));
-  else enqueue_solve(h, dX, nrhs, ldx);
+  else enqueue_solve(h, dX, nrhs, ldx, marked);
   SWC_HIP(hipEventRecord(h->ev[3], st));
   SWC_HIP(hipGetLastError());
   return SWC_OK;
@@ -2014,15 +2065,22 @@ int from_factor(swc_handle* h, const double* dIn, double* X, int on_device, int6
 
 // ---- refinement -------------------------------------------------------------
 
-// Per-column reduction (op 0 max|x|, op 1 x.y) of n x ncol device columns.
-int reduce_cols(swc_handle* h, const double* X, const double* Y, int ncol, int op, double* out) {
+// Column reductions (op 0 max|x|, 1 dot(x, y)) into slot `slot` of dScal, and slots
+// [0, nslots) to the host: what one decision needs is waited for once.
+void launch_reduce(swc_handle* h, const double* X, const double* Y, int ncol, int op, int slot) {
   hipStream_t st = h->stream;
   hipLaunchKernelGGL(k_reduce_partial, dim3(kRedBlocks, ncol), dim3(kThreads), 0, st, X, Y, h->n,
                      (int64_t)h->n, op, h->dPart);
   hipLaunchKernelGGL(k_reduce_final, dim3(ncol), dim3(kThreads), 0, st, (const double*)h->dPart, op,
-                     h->dScal + 64);
-  SWC_HIP(hipMemcpyAsync(out, h->dScal + 64, sizeof(double) * ncol, hipMemcpyDeviceToHost, st));
+                     h->dScal + 64 + (int64_t)slot * ncol);
+}
+int fetch_reduced(swc_handle* h, int ncol, int nslots, double* out) {
+  SWC_HIP(hipMemcpyAsync(out, h->dScal + 64, sizeof(double) * ncol * nslots, hipMemcpyDeviceToHost, h->stream));
   return sync_stream(h);
+}
+int reduce_cols(swc_handle* h, const double* X, const double* Y, int ncol, int op, double* out) {
+  launch_reduce(h, X, Y, ncol, op, 0);
+  return fetch_reduced(h, ncol, 1, out);
 }
 
 // Y = A X, or R = B - A X when B is given, on n x nrhs device columns of
@@ -2042,7 +2100,7 @@ int put_coeffs(swc_handle* h, const std::vector<double>& c) {
   return SWC_OK;
 }
 
-int solve_device(swc_handle* h, double* dX, int nrhs, int64_t ldx);
+int solve_device(swc_handle* h, double* dX, int nrhs, int64_t ldx, bool marked = false);
 
 // Refines X for A X = B (both n x nrhs, factor ordering, ld n) until every
 // column's eta = ||b - A x||_inf / (||A||_inf ||x||_inf + ||b||_inf) <= tol.
@@ -2057,25 +2115,28 @@ int refine_device(swc_handle* h, const double* Bt, double* Xt, int nrhs, double 
   double* Z = h->dRef + (int64_t)3 * n * nrhs;
   double* Pv = h->dRef + (int64_t)4 * n * nrhs;
   const dim3 g(std::min(grid_for(n), 2048), nrhs);
-  std::vector<double> bn(nrhs), xn(nrhs), rn(nrhs), rz(nrhs), pq(nrhs), co(nrhs);
+  std::vector<double> bn, red(3 * (size_t)nrhs), rz(nrhs), pq(nrhs), co(nrhs);
   std::vector<char> conv(nrhs, 0);
   auto copy = [&](double* dst, const double* src) {
     return hipMemcpyAsync(dst, src, sizeof(double) * n * nrhs, hipMemcpyDeviceToDevice, st);
   };
   auto evaluate = [&](double* Rbuf, bool& done) -> int {
     launch_csr_mv(h, (const double*)Xt, Bt, Rbuf, n, ld, nrhs);
-    if (int rc = reduce_cols(h, Rbuf, nullptr, nrhs, 0, rn.data())) return rc;
-    if (int rc = reduce_cols(h, Xt, nullptr, nrhs, 0, xn.data())) return rc;
+    launch_reduce(h, Rbuf, nullptr, nrhs, 0, 0);
+    launch_reduce(h, Xt, nullptr, nrhs, 0, 1);
+    // the first evaluation fetches max|b| too (slot 2, which put_coeffs uses later)
+    if (int rc = fetch_reduced(h, nrhs, bn.empty() ? 3 : 2, red.data())) return rc;
+    if (bn.empty()) bn.assign(red.begin() + 2 * nrhs, red.end());
     done = true;
     for (int c = 0; c < nrhs; ++c) {
-      const double den = h->normA * xn[c] + bn[c];
-      eta[c] = den > 0 ? rn[c] / den : 0.0;
+      const double den = h->normA * red[nrhs + c] + bn[c];
+      eta[c] = den > 0 ? red[c] / den : 0.0;
       conv[c] = eta[c] <= tol;
       done = done && conv[c];
     }
     return SWC_OK;
   };
-  if (int rc = reduce_cols(h, Bt, nullptr, nrhs, 0, bn.data())) return rc;
+  launch_reduce(h, Bt, nullptr, nrhs, 0, 2);
   SWC_HIP(copy(Xt, Bt));
   if (int rc = solve_device(h, Xt, nrhs, ld)) return rc;
   int it = 0;
@@ -2433,8 +2494,7 @@ int upload_structure(swc_handle* h, int n, const int* blockSet, int supNo, const
   if (!rc)
     rc = upload(&h->dDiag, (const double*)nullptr,
                 (size_t)std::max(P.diag_scratch, F.diag_scratch), st);
-  if (!rc) rc = upload(&h->dNorm, (const double*)nullptr, 8, st);
-  if (!rc) rc = upload(&h->dNormPart, (const double*)nullptr, kRedBlocks, st);
+  if (!rc) rc = upload(&h->dNormPart, (const double*)nullptr, kSetupBlocks, st);
   h->zvalid = false;
   (void)hipFree(h->dZ);
   (void)hipFree(h->dArena);
@@ -2466,7 +2526,7 @@ int swc_create(swc_handle** out) {
     delete h;
     return SWC_EDEVICE;  // bind_scratch recorded why
   }
-  if (e == hipSuccess && !(h->abort_host = take_abort_word())) e = hipErrorOutOfMemory;
+  if (e == hipSuccess && !(h->rec = take_record())) e = hipErrorOutOfMemory;
   if (e == hipSuccess) e = hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking);
   if (e == hipSuccess) e = hipMalloc((void**)&h->dInfo, sizeof(int));
   for (auto& ev : h->ev)
@@ -2644,8 +2704,20 @@ int swc_solve(swc_handle* h, double* B, int nrhs, int64_t ldb, int on_device) {
     return swc_set_error(SWC_EINVAL, "swc_solve: bad argument");
   if (int rc = ensure_work(h, nrhs)) return rc;
   double* dY = h->dRef;
-  if (int rc = to_factor(h, B, on_device, ldb, dY, nrhs)) return rc;
-  if (int rc = solve_device(h, dY, nrhs, h->n)) return rc;
+  // with an ordering, B goes into factor order in the launch that marks the vectors
+  const bool marked = !h->perm.empty();
+  if (marked) {
+    const double* src = B;
+    if (!on_device) {
+      SWC_HIP(hipMemcpy2DAsync(h->dWork, sizeof(double) * h->n, B, sizeof(double) * ldb,
+                               sizeof(double) * h->n, nrhs, hipMemcpyHostToDevice, h->stream));
+      src = h->dWork;
+    }
+    enqueue_marks(h, sweep_run(h, dY, nrhs, h->n, h->dY, h->dV, h->dPb), src, on_device ? ldb : h->n);
+  } else if (int rc = to_factor(h, B, on_device, ldb, dY, nrhs)) {
+    return rc;
+  }
+  if (int rc = solve_device(h, dY, nrhs, h->n, marked)) return rc;
   if (int rc = from_factor(h, dY, B, on_device, ldb, nrhs)) return rc;
   float ms = 0;
   SWC_HIP(hipEventElapsedTime(&ms, h->ev[2], h->ev[3]));
@@ -2724,13 +2796,14 @@ int swc_residual(swc_handle* h, const double* B, const double* X, int nrhs, int6
   if (int rc = to_factor(h, B, on_device, ld, Bt, nrhs)) return rc;
   if (int rc = to_factor(h, X, on_device, ld, Xt, nrhs)) return rc;
   launch_csr_mv(h, (const double*)Xt, (const double*)Bt, R, n, (int64_t)n, nrhs);
-  std::vector<double> rn(nrhs), xn(nrhs), bn(nrhs);
-  if (int rc = reduce_cols(h, R, nullptr, nrhs, 0, rn.data())) return rc;
-  if (int rc = reduce_cols(h, Xt, nullptr, nrhs, 0, xn.data())) return rc;
-  if (int rc = reduce_cols(h, Bt, nullptr, nrhs, 0, bn.data())) return rc;
+  std::vector<double> red(3 * (size_t)nrhs);
+  launch_reduce(h, R, nullptr, nrhs, 0, 0);
+  launch_reduce(h, Xt, nullptr, nrhs, 0, 1);
+  launch_reduce(h, Bt, nullptr, nrhs, 0, 2);
+  if (int rc = fetch_reduced(h, nrhs, 3, red.data())) return rc;
   for (int c = 0; c < nrhs; ++c) {
-    const double den = h->normA * xn[c] + bn[c];
-    eta[c] = den > 0 ? rn[c] / den : 0.0;
+    const double den = h->normA * red[nrhs + c] + red[2 * nrhs + c];
+    eta[c] = den > 0 ? red[c] / den : 0.0;
   }
   return SWC_OK;
 }
@@ -2880,11 +2953,10 @@ int swc_logdet(swc_handle* h, double* logdet) {
   hipLaunchKernelGGL(k_logdet_partial, dim3(kRedBlocks), dim3(kThreads), 0, st, (const double*)h->dL,
                      (const int64_t*)h->dDiagPos, h->n, h->dNormPart);
   hipLaunchKernelGGL(k_reduce_final, dim3(1), dim3(kThreads), 0, st, (const double*)h->dNormPart, 1,
-                     h->dNorm + 1);
-  double v = 0;
-  SWC_HIP(hipMemcpyAsync(&v, h->dNorm + 1, sizeof(double), hipMemcpyDeviceToHost, st));
+                     &h->rec->logdet);
+  SWC_HIP(hipGetLastError());
   SWC_HIP(hipStreamSynchronize(st));
-  *logdet = 2.0 * v;
+  *logdet = 2.0 * h->rec->logdet;
   return SWC_OK;
 }
 

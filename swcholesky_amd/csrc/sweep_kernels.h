@@ -797,11 +797,19 @@ k_sweep_small(SweepRun a, int s0, int ns) {
   else small_backward<Q>(a, s, r0, min(Q, a.nrhs - r0), lane);
 }
 
-// Marks every entry a sweep waits for as pending and resets the two tickets.
+// Marks every entry a sweep waits for as pending and resets the two tickets; with `in`
+// given, out = P in (n x nrhs, factor order) in the same launch.
 __global__ void __launch_bounds__(kThreads)
 k_sweep_init(double* __restrict__ Y, int64_t ny, double* __restrict__ V, int64_t nv,
-             double* __restrict__ P, int64_t np, int* __restrict__ sync) {
+             double* __restrict__ P, int64_t np, int* __restrict__ sync,
+             const double* __restrict__ in, int64_t ldin, double* __restrict__ out, int64_t ldout,
+             const int* __restrict__ perm, int n, int nrhs) {
   const int64_t i0 = (int64_t)blockIdx.x * kThreads + threadIdx.x, st = (int64_t)gridDim.x * kThreads;
+  if (in)
+    for (int64_t e = i0; e < (int64_t)n * nrhs; e += st) {
+      const int k = (int)(e % n), r = (int)(e / n);
+      out[r * ldout + k] = in[r * ldin + perm[k]];
+    }
   for (int64_t i = i0; i < ny; i += st) mark_pending(Y + i);
   for (int64_t i = i0; i < nv; i += st) mark_pending(V + i);
   for (int64_t i = i0; i < np; i += st) mark_pending(P + i);
