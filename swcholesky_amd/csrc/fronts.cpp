@@ -4,6 +4,7 @@
 #include <algorithm>
 #include <map>
 #include <memory>
+#include <tuple>
 
 namespace swc {
 
@@ -50,6 +51,53 @@ class Arena {
 };
 
 }  // namespace
+
+// Orders a launch's tiles (sorted by k) so that workgroups of one XCD, which share an L2
+// and get every eighth workgroup, work on square groups of neighbouring tiles: side * side
+// tiles read 2 side operand blocks, a run down a column of tiles 1 + side^2.  A group goes
+// to the XCD with the least work so far.  Groups of 8 x 8 tiles need 16 blocks of 64 rows,
+// up to 4 MB at k = 512, what an L2 holds; a launch of few tiles gets smaller groups, so
+// that every XCD has several, and keeps its order below 4 x 64 tiles.
+static void order_for_xcds(std::vector<FrontTile>& tiles) {
+  constexpr int kXcds = 8;
+  const int n = (int)tiles.size();
+  int side = 1;
+  while (side < 8 && (side + 1) * (side + 1) * 64 <= n) ++side;
+  if (side == 1) return;
+  struct Group {
+    int k;
+    std::vector<int> tiles;
+  };
+  std::vector<Group> groups;
+  std::map<std::tuple<int64_t, int, int, int>, int> index;
+  for (int i = 0; i < n; ++i) {
+    const FrontTile& u = tiles[i];
+    const int col = u.row - (int)((u.asrc - u.bsrc) / T);
+    // supernode, step and kind have one source offset of tile row 0
+    const auto key = std::make_tuple(u.asrc - (int64_t)T * u.row, u.k, u.row / side, col / side);
+    const auto it = index.emplace(key, (int)groups.size());
+    if (it.second) groups.push_back({u.k, {}});
+    groups[it.first->second].tiles.push_back(i);
+  }
+  std::vector<int> queue[kXcds];
+  int64_t load[kXcds] = {};
+  for (const Group& g : groups) {  // in order of decreasing k
+    const int x = (int)(std::min_element(load, load + kXcds) - load);
+    load[x] += (int64_t)g.tiles.size() * (g.k + 32);
+    queue[x].insert(queue[x].end(), g.tiles.begin(), g.tiles.end());
+  }
+  std::vector<FrontTile> out;
+  out.reserve(n);
+  size_t at[kXcds] = {};
+  for (int i = 0; (int)out.size() < n; ++i) {
+    int x = i % kXcds;
+    if (at[x] == queue[x].size())  // its queue has run out: from the longest
+      for (int y = 0; y < kXcds; ++y)
+        if (queue[y].size() - at[y] > queue[x].size() - at[x]) x = y;
+    out.push_back(tiles[queue[x][at[x]++]]);
+  }
+  tiles.swap(out);
+}
 
 bool build_fronts(int n, int nsuper, const int* super, const int64_t* pi, const int64_t* px,
                   int64_t xsize, const int* Ls, const int* prunePtr, const int* pruneSet,
@@ -323,6 +371,7 @@ bool build_fronts(int n, int nsuper, const int* super, const int64_t* pi, const 
             u.nr = std::min(T, R - T * (q + t));
             u.nc = std::min(T, w - T * q);
             u.diag = t == 0;
+            u.row = q + t;
             u.slot = -1;
             // the panels of the first block are first touched by panel 0, the later
             // ones by the whole first block
@@ -350,6 +399,7 @@ bool build_fronts(int n, int nsuper, const int* super, const int64_t* pi, const 
               u.nr = std::min(T, m - T * a);
               u.nc = std::min(T, m - T * b);
               u.diag = a == b;
+              u.row = a;
               u.upd = 1;
               u.slot = -1;
               u.first = q0 == 0;
@@ -402,6 +452,7 @@ bool build_fronts(int n, int nsuper, const int* super, const int64_t* pi, const 
     auto heavier = [](const FrontTile& a, const FrontTile& b) { return a.k > b.k; };
     std::stable_sort(L.uc.begin(), L.uc.end(), heavier);
     std::stable_sort(L.ud.begin(), L.ud.end(), heavier);
+    order_for_xcds(L.uc);
     // diagonal copies: made by U_l, read by F_{l+1}
     int64_t off = 0;
     std::vector<std::pair<int64_t, int>> slots;  // panel's value offset -> slot

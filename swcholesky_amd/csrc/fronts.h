@@ -59,7 +59,7 @@ struct FrontTile {
   int g0, g1;     // [g0, g1) gathers, first touch only
   int a0, a1;     // [a0, a1) entries of A, first touch only
   int slot;       // >= 0: a copy of the diagonal block for the next factor launch goes here
-  int pad;
+  int row;        // tile row it is (its column: row - (asrc - bsrc) / 64), for the order of a launch
 };
 
 // One tile of a panel being factored (F launch); fields named as in Tile.
