@@ -125,7 +125,104 @@ __device__ inline void front_products(const T* __restrict__ src, const swc::Fron
   }
 }
 
-template <int MODE>
+// Operands through LDS in steps of 16 columns, two buffers: a thread loads four
+// consecutive rows of one column of each operand (the rows behind the tile's last are
+// read, not used), two steps ahead of their use, so an element comes from L1 once a
+// workgroup instead of twice and in 16-byte loads: straight from global memory L1's
+// lookups are taken 75% of the time and the matrix cores 44%.  Same sums in the same
+// order as front_products, bitwise.
+// Levels with a tile of kStageMin columns or more stage all their tiles; below that the
+// barriers cost more than L1 does.  Straight -> staged from 128 columns on: vector 48^3
+// with FP32 updates 50.6 -> 46.6 ms (update launches 33.2 -> 28.9), 64^3 in FP64 17.55 ->
+// 17.49; from 300 on 46.7 and 17.53; staging every level 46.4 and 17.47, but a mesh of
+// 20,000 points 0.88 -> 0.98.
+constexpr int kStageK = 16;
+constexpr int kStageMin = 128;
+template <typename T>
+constexpr int kStageLd = swc::TM + 16 / (int)sizeof(T);
+constexpr int kUpdateLds = 4 * kStageK * kStageLd<double>;  // doubles; >= PW * kTileLd
+static_assert(kUpdateLds >= swc::PW * kTileLd);
+typedef int i4 __attribute__((ext_vector_type(4)));
+
+template <typename T>
+__device__ inline void front_products_staged(const T* __restrict__ src, const swc::FrontTile& u, int wr,
+                                             int wc, bool active, int tid, double* lds,
+                                             d4 (&acc)[2][2]) {
+  constexpr bool kF32 = sizeof(T) == 4;
+  constexpr int ld = kStageLd<T>, NV = kF32 ? 1 : 2;
+  const int lane = tid & 63, lr = lane & 15, lk = lane >> 4;
+  const int cr = kF32 ? (lr >> 2) + 4 * (lr & 3) : lr;  // f32 output order (task_update)
+  const int kk = tid >> 4, r4 = 4 * (tid & 15);
+  const unsigned at = ((unsigned)kk * (unsigned)u.sld + (unsigned)r4) * (unsigned)sizeof(T);
+  T* stage = reinterpret_cast<T*>(lds);
+  i4 ra[NV], rb[NV];
+  auto load = [&](int kb) {
+    const int64_t base = (int64_t)min(kb, u.k) * u.sld;
+    const __amdgpu_buffer_rsrc_t qa = make_rsrc(src + u.asrc + base, 0x3fffffff);
+    const __amdgpu_buffer_rsrc_t qb = make_rsrc(src + u.bsrc + base, 0x3fffffff);
+    const bool in = kb + kk < u.k;
+    const unsigned oa = in && r4 < u.nr ? at : kNoLand, ob = in && r4 < u.nc ? at : kNoLand;
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+      ra[v] = __builtin_bit_cast(i4, __builtin_amdgcn_raw_buffer_load_b128(qa, (int)(oa + 16 * v), 0, 0));
+      rb[v] = __builtin_bit_cast(i4, __builtin_amdgcn_raw_buffer_load_b128(qb, (int)(ob + 16 * v), 0, 0));
+    }
+  };
+  auto store = [&](int buf) {
+    i4* a = reinterpret_cast<i4*>(stage + (2 * buf) * kStageK * ld + kk * ld + r4);
+    i4* b = reinterpret_cast<i4*>(stage + (2 * buf + 1) * kStageK * ld + kk * ld + r4);
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+      a[v] = ra[v];
+      b[v] = rb[v];
+    }
+  };
+  const bool skip01 = u.diag && wr == wc;  // the block of rows 0..15, columns 16..31
+  auto multiply = [&](int buf) {
+    const T* A = stage + (2 * buf) * kStageK * ld + lk * ld + 32 * wr + lr;
+    const T* B = stage + (2 * buf + 1) * kStageK * ld + lk * ld + 32 * wc + cr;
+    T a[2][4], b[2][4];
+#pragma unroll
+    for (int x = 0; x < 4; ++x)
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        a[q][x] = A[4 * x * ld + 16 * q];
+        b[q][x] = B[4 * x * ld + 16 * q];
+      }
+#pragma unroll
+    for (int bj = 0; bj < 2; ++bj)
+#pragma unroll
+      for (int bi = 0; bi < 2; ++bi) {
+        if (bj == 1 && bi == 0 && skip01) continue;
+        if constexpr (!kF32) {
+#pragma unroll
+          for (int x = 0; x < 4; ++x)
+            acc[bj][bi] = __builtin_amdgcn_mfma_f64_16x16x4f64(b[bj][x], a[bi][x], acc[bj][bi], 0, 0, 0);
+        } else {
+          f4 c = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int x = 0; x < 4; ++x)
+            c = __builtin_amdgcn_mfma_f32_16x16x4f32(b[bj][x], a[bi][x], c, 0, 0, 0);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) acc[bj][bi][r] += (double)c[r];
+        }
+      }
+  };
+  load(0);
+  store(0);
+  load(kStageK);
+  lds_barrier();
+  for (int kb = 0, buf = 0; kb < u.k; kb += kStageK, buf ^= 1) {
+    if (active) multiply(buf);
+    if (kb + kStageK < u.k) {
+      store(buf ^ 1);
+      load(kb + 2 * kStageK);
+    }
+    lds_barrier();
+  }
+}
+
+template <int MODE, bool STAGED>
 __device__ inline void front_update_body(double* __restrict__ L, const float* __restrict__ Lf,
                                          const swc::FrontTile& u, const FrontIn& in,
                                          double* __restrict__ dscratch, double* lds, int tid) {
@@ -141,15 +238,17 @@ __device__ inline void front_update_body(double* __restrict__ L, const float* __
     }
     lds_barrier();
   }
-  if ((diag && wr < wc) || 32 * wr >= u.nr || 32 * wc >= u.nc) return;  // nothing of the tile
+  // a wave with nothing of the tile only loads operands
+  const bool active = !((diag && wr < wc) || 32 * wr >= u.nr || 32 * wc >= u.nc);
   double* tgt = L + u.vbase;
   // this lane's elements: row 32 wr + 16 bi + l % 16, column 32 wc + 16 bj + l / 16 + 4 r
   auto row_of = [&](int l, int bi) { return 32 * wr + 16 * bi + (l & 15); };
   auto col_of = [&](int l, int bj, int r) { return 32 * wc + 16 * bj + (l >> 4) + 4 * r; };
-  auto inside = [&](int i, int j) { return i < u.nr && j < u.nc && !(diag && i < j); };
+  auto inside = [&](int i, int j) { return active && i < u.nr && j < u.nc && !(diag && i < j); };
   const __amdgpu_buffer_rsrc_t rt = land_rsrc(tgt);
   d4 cur[2][2];
-  if (!u.first) {
+  if (!active) {
+  } else if (!u.first) {
 #pragma unroll
     for (int bj = 0; bj < 2; ++bj)
 #pragma unroll
@@ -203,8 +302,16 @@ __device__ inline void front_update_body(double* __restrict__ L, const float* __
 #pragma unroll
     for (int bi = 0; bi < 2; ++bi) acc[bj][bi] = d4{0.0, 0.0, 0.0, 0.0};
   const bool f32 = MODE == 2 || (MODE == 1 && u.upd);
-  if (f32) front_products<float>(Lf, u, wr, wc, lane, acc);
-  else front_products<double>(L, u, wr, wc, lane, acc);
+  if constexpr (STAGED) {
+    if (u.a1 > u.a0) lds_barrier();  // the entries have been read
+    if (f32) front_products_staged<float>(Lf, u, wr, wc, active, tid, lds, acc);
+    else front_products_staged<double>(L, u, wr, wc, active, tid, lds, acc);
+  } else {
+    if (!active) return;
+    if (f32) front_products<float>(Lf, u, wr, wc, lane, acc);
+    else front_products<double>(L, u, wr, wc, lane, acc);
+  }
+  if (!active) return;
   // element addresses are formed again from an opaque lane index: kept from the loads
   // above they would hold 16 registers through the products
   int l2 = lane;
@@ -224,13 +331,13 @@ __device__ inline void front_update_body(double* __restrict__ L, const float* __
       }
 }
 
-template <int MODE>
-__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3)))
+template <int MODE, bool STAGED>
+__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(STAGED ? 4 : 3)))
 k_front_update(double* __restrict__ L, const swc::FrontTile* __restrict__ tiles, int tile0,
                FrontIn in, double* __restrict__ dscratch, const float* __restrict__ Lf) {
-  __shared__ double lds[swc::PW * kTileLd];
+  __shared__ __align__(16) double lds[kUpdateLds];
   const swc::FrontTile u = tiles[tile0 + blockIdx.x];
-  front_update_body<MODE>(L, Lf, u, in, dscratch, lds, threadIdx.x);
+  front_update_body<MODE, STAGED>(L, Lf, u, in, dscratch, lds, threadIdx.x);
 }
 
 // ---- F launch ----------------------------------------------------------------
@@ -541,7 +648,7 @@ k_front_factor(double* __restrict__ L, const swc::SmallFront* __restrict__ small
                const swc::FrontTile* __restrict__ utiles, int u0, FrontIn in,
                const double* __restrict__ dscratch, double* __restrict__ dscratch_u,
                int* __restrict__ info_out, float* Lf_factor, const float* __restrict__ Lf_update) {
-  extern __shared__ double lds[];  // front_factor_lds() doubles
+  extern __shared__ __align__(16) double lds[];  // front_factor_lds() doubles
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   int b = blockIdx.x;
   const int bs = (nsmall + 3) >> 2, bn = (nn + 3) >> 2;
@@ -568,7 +675,7 @@ k_front_factor(double* __restrict__ L, const swc::SmallFront* __restrict__ small
     panel_factor_blk_body(L, tl, dscratch, info_out, Lf_factor, lds, tid, in);
   } else {
     const swc::FrontTile u = utiles[u0 + (b - nw)];
-    front_update_body<MODE>(L, Lf_update, u, in, dscratch_u, lds, tid);
+    front_update_body<MODE, false>(L, Lf_update, u, in, dscratch_u, lds, tid);
   }
 }
 
@@ -580,6 +687,6 @@ inline size_t front_factor_lds(int nwave_items, int widest, int ndefer) {
   size_t d = 0;
   if (nwave_items) d = 4 * kSmallLds;
   if (widest) d = std::max(d, (size_t)((widest + 15) / 16 * 16 * kWld));
-  if (ndefer) d = std::max(d, (size_t)swc::PW * kTileLd);
+  if (ndefer) d = std::max(d, (size_t)kUpdateLds);
   return d * sizeof(double);
 }

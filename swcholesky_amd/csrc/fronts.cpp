@@ -421,6 +421,7 @@ bool build_fronts(int n, int nsuper, const int* super, const int64_t* pi, const 
   F.lvl_u.assign(F.nlevel + 1, 0);
   F.lvl_ud.assign(F.nlevel, 0);
   F.lvl_flops.assign(F.nlevel, 0.0);
+  F.lvl_kmax.assign(F.nlevel, 0);
   auto flops = [](const FrontTile& u) {
     const double pairs = u.diag ? u.nc * (u.nc + 1) / 2.0 + (double)(u.nr - u.nc) * u.nc
                                 : (double)u.nr * u.nc;
@@ -452,6 +453,7 @@ bool build_fronts(int n, int nsuper, const int* super, const int64_t* pi, const 
     auto heavier = [](const FrontTile& a, const FrontTile& b) { return a.k > b.k; };
     std::stable_sort(L.uc.begin(), L.uc.end(), heavier);
     std::stable_sort(L.ud.begin(), L.ud.end(), heavier);
+    if (!L.uc.empty()) F.lvl_kmax[l] = L.uc.front().k;
     order_for_xcds(L.uc);
     // diagonal copies: made by U_l, read by F_{l+1}
     int64_t off = 0;

@@ -95,6 +95,7 @@ struct FrontPlan {
   std::vector<int> lvl_u;           // nlevel+1
   std::vector<int> lvl_ud;          // nlevel: deferred tiles, last in their level: they run in the
                                     // next level's F launch
+  std::vector<int> lvl_kmax;        // nlevel: most source columns of a tile of U_l
   std::vector<double> lvl_flops;    // useful flops of U_l
   double update_flops = 0, factor_flops = 0;
 };

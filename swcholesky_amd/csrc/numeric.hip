@@ -1147,6 +1147,9 @@ __global__ void k_permute(const double* __restrict__ in, double* __restrict__ ou
 
 constexpr int kRedBlocks = 512;
 constexpr int kSetupBlocks = 2048;
+// Elements behind L and its FP32 copy: an update tile's staged loads read up to three rows
+// past its last.
+constexpr int kLoadPad = 16;
 
 // Workspace of swc_solve_noalloc, the entry point that allocates nothing: one
 // copy of this array per GPU, held from the library's load until the process
@@ -1674,8 +1677,9 @@ void enqueue_fronts(swc_handle* h, bool profile) {
     if (pe) (void)hipEventRecord(pe[2], st);
     const int u0 = F.lvl_u[l], nu = F.lvl_u[l + 1] - u0 - (profile ? 0 : F.lvl_ud[l]);
     if (nu > 0)
-      hipLaunchKernelGGL(k_front_update<MODE>, dim3(nu), dim3(kThreads), 0, st, h->dL, ut, u0, in,
-                         h->dDiag, (const float*)h->dLf);
+      hipLaunchKernelGGL((F.lvl_kmax[l] >= kStageMin ? k_front_update<MODE, true> : k_front_update<MODE, false>),
+                         dim3(nu), dim3(kThreads), 0, st, h->dL, ut, u0, in, h->dDiag,
+                         (const float*)h->dLf);
     if (pe) (void)hipEventRecord(pe[3], st);
   }
 }
@@ -2407,7 +2411,7 @@ int upload_structure(swc_handle* h, int n, const int* blockSet, int supNo, const
     plan(factor && !h->multifrontal);
     if (h->multifrontal) {
       // the arena follows L in one allocation
-      rc = upload(&h->dL, (const double*)nullptr, (size_t)(h->plan.xsize + h->fronts.usize), st);
+      rc = upload(&h->dL, (const double*)nullptr, (size_t)(h->plan.xsize + h->fronts.usize + kLoadPad), st);
       if (rc && h->fronts.usize > 0) {
         (void)hipGetLastError();
         h->multifrontal = false;
@@ -2440,7 +2444,7 @@ int upload_structure(swc_handle* h, int n, const int* blockSet, int supNo, const
   h->dLf = nullptr;
   h->lf_cap = 0;
   if (!rc && h->precision > 0 && factor) {
-    rc = upload(&h->dLf, (const float*)nullptr, (size_t)P.xsize, st);
+    rc = upload(&h->dLf, (const float*)nullptr, (size_t)(P.xsize + kLoadPad), st);
     if (!rc) h->lf_cap = P.xsize;
   }
   if (!rc) rc = upload(&h->dLs, h->Ls.data(), h->Ls.size(), st);
@@ -2925,7 +2929,7 @@ int swc_set_precision(swc_handle* h, int mode) {
     (void)hipFree(h->dLf);
     h->dLf = nullptr;
     h->lf_cap = 0;
-    SWC_HIP(hipMalloc((void**)&h->dLf, sizeof(float) * (size_t)h->plan.xsize));
+    SWC_HIP(hipMalloc((void**)&h->dLf, sizeof(float) * (size_t)(h->plan.xsize + kLoadPad)));
     h->lf_cap = h->plan.xsize;
   }
   h->precision = mode;

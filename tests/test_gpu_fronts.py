@@ -89,3 +89,31 @@ def test_left_looking_narrow_kernels(fuse, mode):
     else:
         L32, _ = O.factor(b, a2x, fp32_updates=True)
         assert relF(f.L_values(), L32) < 10 * max(relF(L32, Lo), 1e-7)
+
+
+@pytest.mark.parametrize("make", [lambda: P.dense_spd(600, seed=2), lambda: P.dense_spd(641, seed=2),
+                                  lambda: P.laplacian3d_var(13, shift=1.0), lambda: P.vector3d_var(11)],
+                         ids=["dense_600", "dense_641", "lap3d_13", "vec3d_11"])
+@pytest.mark.parametrize("mode", [0, 2])
+def test_updates_of_many_columns_match_dense_cholesky(make, mode):
+    """Supernodes of 128 columns and more (operands by way of LDS), remainders in every
+    dimension; FP64 updates, and FP32 ones whose products carry 2^-24 each."""
+    prob = make()
+    b = S.analyze_p2(prob.n, prob.colptr, prob.rowidx, prob.perm)
+    assert np.diff(b.super).max() >= 128
+    f = S.Factor(b)
+    f.set_precision(mode)
+    assert f.factor(prob.values) == 0
+    Ap = prob.scipy_full().toarray()[np.ix_(b.Perm, b.Perm)]
+    L = f.L_values()
+    ref = np.linalg.cholesky(Ap)
+    err = 0.0
+    for s in range(b.nsuper):
+        c0, c1 = b.super[s], b.super[s + 1]
+        rows = b.s[b.pi[s]:b.pi[s + 1]]
+        blk = L[b.p[c0]:b.p[c0] + len(rows) * (c1 - c0)].reshape(c1 - c0, len(rows)).T
+        low = rows[:, None] >= np.arange(c0, c1)[None, :]
+        err = max(err, np.abs(np.where(low, blk - ref[np.ix_(rows, np.arange(c0, c1))], 0.0)).max())
+    eps = np.finfo(float).eps if mode == 0 else 2.0 ** -24
+    # backward error n eps |A| at most, and cond(A) between it and L
+    assert err <= 10 * np.sqrt(prob.n) * eps * np.linalg.cond(Ap) * np.abs(ref).max()
