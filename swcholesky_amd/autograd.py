@@ -28,8 +28,15 @@ class _LogdetQuad(torch.autograd.Function):
         info = factor.factor(vals if vals.is_cuda else vals.numpy())
         if info:
             raise RuntimeError(f"matrix is not positive definite (column {info - 1})")
-        x = torch.from_numpy(factor.solve(rhs.cpu().numpy())).to(dev)
-        out = alpha * factor.logdet() + beta * float(torch.dot(rhs.cpu(), x.cpu()))
+        if rhs.is_cuda and rhs.device == dev and rhs.shape == (factor.n,):
+            # solved where it is: the vectors do not travel to the host and back
+            x = rhs.clone()
+            _sync()  # the solve runs on the factor's own stream
+            quad = float(torch.dot(rhs, factor.solve_device(x)))
+        else:
+            x = torch.from_numpy(factor.solve(rhs.cpu().numpy())).to(dev)
+            quad = float(torch.dot(rhs.cpu(), x.cpu()))
+        out = alpha * factor.logdet() + beta * quad
         ctx.factor, ctx.alpha, ctx.beta = factor, alpha, beta
         ctx.save_for_backward(x)
         return torch.tensor(out, dtype=torch.float64, device=dev)
