@@ -1505,6 +1505,7 @@ struct swc_handle {
   // (buffer, nrhs, ld); rebuilt when the structure changes
   bool use_graphs = true;
   hipGraphExec_t fgraph[3] = {nullptr, nullptr, nullptr};
+  bool factor_seen[3] = {};  // a factorization of this structure in that mode has run
   struct SolveGraph {
     const double* x;
     int nrhs;
@@ -1531,6 +1532,7 @@ struct swc_handle {
     for (auto& g : fgraph)
       if (g) (void)hipGraphExecDestroy(g);
     for (auto& g : fgraph) g = nullptr;
+    for (auto& s : factor_seen) s = false;
     for (auto& g : sgraphs) (void)hipGraphExecDestroy(g.exec);
     sgraphs.clear();
   }
@@ -1819,7 +1821,11 @@ int factor_device(swc_handle* h, const double* dvals) {
     h->pev.assign((size_t)4 * nlevel, nullptr);
     for (auto& e : h->pev) SWC_HIP(hipEventCreate(&e));
   }
-  const bool graph = h->use_graphs && !h->profile;
+  // the first factorization is launched kernel by kernel: capturing and instantiating
+  // its graph costs a call that is not repeated more than the graph saves it
+  bool& again = h->factor_seen[h->precision];
+  const bool graph = h->use_graphs && !h->profile && again;
+  again = true;
   hipGraphExec_t& gx = h->fgraph[h->precision];
   if (graph && !gx) {
     hipGraph_t g = nullptr;
