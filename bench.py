@@ -247,7 +247,7 @@ def main():
         log(f"large front: level {r['level']} {r['gflop']:.1f} GFLOP in {r['ms']:.2f} ms = "
             f"{r['tflops']:.1f} TFLOP/s ({100 * r['frac_fp64_peak']:.0f}% of FP64 MFMA peak)")
     traffic, traffic_src = None, None
-    pmc = os.path.join(ROOT, "profiles", "k_tile_update_lap3d64_pmc.json")
+    pmc = os.path.join(ROOT, "profiles", "k_front_update_lap3d64_pmc.json")
     if args.side == 64 and os.path.exists(pmc):
         with open(pmc) as fh:
             rec = json.load(fh)
@@ -284,7 +284,7 @@ def main():
         "time_to_1e-12_ms": {k: v["ms"] for k, v in paths.items()},
         "mixed_speedup_vs_fp64": paths["fp64"]["ms"] / min(paths["mixed"]["ms"], paths["mixed_all"]["ms"]),
         "paths": paths,
-        "roofline": {"bound": "mfma", "kernel": "k_tile_update", "achieved": achieved,
+        "roofline": {"bound": "mfma", "kernel": "k_front_update", "achieved": achieved,
                      "peak": PEAK_FP64_TFLOPS, "unit": "TFLOP/s",
                      "frac": achieved / PEAK_FP64_TFLOPS, "traffic": traffic,
                      "traffic_source": traffic_src,

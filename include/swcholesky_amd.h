@@ -139,8 +139,9 @@ int swc_set_perm(swc_handle* h, const int* perm);
 /* Shape parameters of the plan built by the next structure upload (swc_upload,
  * swc_upload_symbolic), as {rlb, spw, narrow_min_tiles, narrow_max_k, fuse_narrow,
  * dag} (count <= 6, leading entries; NULL restores the defaults {8, 128, 1024, 256,
- * 1, 0}): rlb panels per block of a wide supernode's right-looking steps, spw = 64
- * or 128 columns per solve panel, the one-wave tile kernel for levels with at least
+ * 1, 0}): rlb panels per block of a wide supernode's right-looking steps; the others shape
+ * the left-looking plan and its exports: spw = 64 or 128 columns per exported solve
+ * panel, the one-wave tile kernel for levels with at least
  * narrow_min_tiles tiles of panels <= 16 columns whose inner dimensions sum to
  * <= narrow_max_k, with fuse_narrow = 1 such panels (all tiles narrow) updated
  * and factored by one wave each in one persistent launch per level.  dag must be
@@ -234,8 +235,9 @@ int swc_plan_stats(const swc_handle* h, int64_t* out, double* flops);
  * launch's useful (lower-triangle) update flops; *nlevel = number of levels.
  * No counterpart in the reference: instrumentation of the GPU schedule. */
 int swc_level_timings(const swc_handle* h, double* out, int cap, int* nlevel);
-/* With graphs on (default), swc_factor and the solves replay launch sequences
- * captured once per structure (hipGraph) instead of launching level by level. */
+/* With graphs on (default), swc_factor (from its second call on a structure) and the
+ * solves replay launch sequences captured once per structure (hipGraph) instead of
+ * launching level by level. */
 int swc_set_graphs(swc_handle* h, int on);
 /* With profiling on, every kernel launch of swc_factor is bracketed by HIP events
  * on the handle's stream (for measurement runs; adds launch gaps). */

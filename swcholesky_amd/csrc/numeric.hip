@@ -1,12 +1,11 @@
-// MI355X (gfx950) numeric phase: supernodal left-looking Cholesky, triangular
-// solves, residual and refinement, behind the C ABI of include/swcholesky_amd.h.
+// MI355X (gfx950) numeric phase: supernodal Cholesky, triangular solves, residual,
+// refinement and adjoint, behind the C ABI of include/swcholesky_amd.h.
 //
-// Work is organised by the plan of plan.h: panels of <= 64 columns, tiles of
-// <= 64 rows, each tile's accumulator held in MFMA registers.  One level of the
-// panel DAG is one launch of the tile kernel (every update of every tile of
-// the level) followed by the panel factor launches (POTRF of the diagonal
-// block of each panel the level completes and TRSM of its tiles).  The solves
-// walk solve panels of <= SPW columns, level by level, forward then backward.
+// The factor is multifrontal (fronts.h, front_kernels.h): two launches per level of the
+// supernode tree.  The left-looking path (plan.h and the tile and panel kernels here)
+// serves structures without a front tree, arenas that do not fit and H-level schedules.
+// The solves are one persistent launch per sweep (sweeps.h, sweep_kernels.h); the selected
+// inverse is in selinv.h and selinv_kernels.h.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
