@@ -1916,7 +1916,10 @@ template <bool FORWARD>
 void launch_small(swc_handle* h, const SweepRun& a, int level) {
   const std::vector<int>& ls = h->plan.sweeps.lvl_small;
   const int s0 = ls[level], ns = ls[level + 1] - s0;
-  if (a.nrhs == 1)
+  if (a.nrhs == 1 && h->plan.sweeps.lvl_small_m[level] <= 16)
+    hipLaunchKernelGGL((k_sweep_small16<FORWARD>), dim3((ns + 15) / 16), dim3(kThreads), 0, h->stream, a,
+                       s0, ns);
+  else if (a.nrhs == 1)
     hipLaunchKernelGGL((k_sweep_small<FORWARD, 1>), dim3((ns + 3) / 4, 1), dim3(kThreads), 0,
                        h->stream, a, s0, ns);
   else

@@ -797,6 +797,85 @@ k_sweep_small(SweepRun a, int s0, int ns) {
   else small_backward<Q>(a, s, r0, min(Q, a.nrhs - r0), lane);
 }
 
+// A level's launch when none of its supernodes has more than 16 rows below, one right-hand
+// side: 16 lanes each, four to a wave.  The leaves of large forests: a wave a supernode
+// leaves three lanes of four idle and pays its chain of 16 columns once a supernode (a
+// solve of 4096 2D instances: 8.4 ms in its six leaf launches, 4.8 with two of them this).  Same
+// sums in the same order as small_forward and small_backward, bitwise.  What it reads has
+// been published by earlier launches, so nothing is waited for.
+template <bool FORWARD>
+__global__ void __launch_bounds__(kThreads)
+k_sweep_small16(SweepRun a, int s0, int ns) {
+  const int i = threadIdx.x & 15, lane = threadIdx.x & 63;
+  const int k0 = (int)blockIdx.x * (kThreads / 16) + ((int)threadIdx.x >> 4);
+  const bool have = k0 < ns;
+  const swc::SweepSmall s = a.small[s0 + min(k0, ns - 1)];
+  const int w = s.w, m = s.R - w;
+  const double* D = a.L + s.vbase;
+  int wmax = max(w, __shfl_xor(w, 16));
+  wmax = __builtin_amdgcn_readfirstlane(max(wmax, __shfl_xor(wmax, 32)));
+  const int ic = min(i, w - 1), c = s.c0 + ic;
+  const double rinv = i < w ? 1.0 / D[(int64_t)ic * (s.R + 1)] : 1.0;
+  double tri[16], lv[16];  // forward: row i of the triangle, backward: its column i
+  const int below = min(w + i, s.R - 1);
+#pragma unroll
+  for (int g = 0; g < 16; g += 4) {
+#pragma unroll
+    for (int k = g; k < g + 4; ++k) tri[k] = lv[k] = 0.0;
+    if (g < wmax) {
+#pragma unroll
+      for (int k = g; k < g + 4; ++k) {
+        const int kc = min(k, w - 1);
+        const double* col = D + (int64_t)kc * s.R;
+        const double v = FORWARD ? col[ic] : D[(int64_t)ic * s.R + kc], b = col[below];
+        tri[k] = (FORWARD ? i < w && k < i : i < w && k > i && k < w) ? v * rinv : 0.0;
+        lv[k] = k < w && (FORWARD || i < m) ? b : 0.0;
+      }
+    }
+  }
+  if constexpr (FORWARD) {
+    const int64_t e0 = a.gptr[c], e1 = i < w ? a.gptr[c + 1] : e0;
+    double p[4] = {0.0, 0.0, 0.0, 0.0};
+    for (int64_t e = e0; __builtin_amdgcn_ballot_w64(e < e1) != 0; e += 8) {
+      int64_t at[8];
+#pragma unroll
+      for (int q = 0; q < 8; ++q) at[q] = e + q < e1 ? a.gidx[e + q] : -1;
+#pragma unroll
+      for (int q = 0; q < 8; ++q) p[q & 3] += at[q] >= 0 ? entry_value(load_entry(a.V + at[q])) : 0.0;
+    }
+    double t = i < w ? (a.X[c] - ((p[0] + p[1]) + (p[2] + p[3]))) * rinv : 0.0;
+    unrolled<0, 15>([&](auto J) {
+      constexpr int j = decltype(J)::value;
+      if (j + 1 < wmax) t = fma(-tri[j], group_bcast<j>(t), t);
+    });
+    if (have && i < w) {
+      publish(a.Y + c, t);
+      mark_pending(a.X + c);  // the backward sweep's entry
+    }
+    double acc = 0.0;
+    unrolled<0, 16>([&](auto K) {
+      constexpr int k = decltype(K)::value;
+      if (k < wmax) acc = fma(lv[k], group_bcast<k>(t), acc);
+    });
+    if (have && i < m) publish(a.V + s.voff + i, acc);
+  } else {
+    const double x = i < m ? entry_value(load_entry(a.X + a.Ls[s.rows_off + below])) : 0.0;
+    LaneSums<1> acc;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) acc.v[k] = lv[k] * x;
+    fold_half<1, 8>(acc, lane);
+    fold_half<1, 4>(acc, lane);
+    fold_half<1, 2>(acc, lane);
+    fold_half<1, 1>(acc, lane);
+    double t = i < w ? (a.Y[c] - acc.v[0]) * rinv : 0.0;
+    unrolled<0, 15>([&](auto J) {
+      constexpr int j = 15 - decltype(J)::value;
+      if (j < wmax) t = fma(-tri[j], group_bcast<j>(t), t);
+    });
+    if (have && i < w) publish(a.X + c, t);
+  }
+}
+
 // Marks every entry a sweep waits for as pending and resets the two tickets; with `in`
 // given, out = P in (n x nrhs, factor order) in the same launch.
 __global__ void __launch_bounds__(kThreads)

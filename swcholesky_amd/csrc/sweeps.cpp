@@ -46,6 +46,11 @@ void build_sweeps(int nsuper, const int* super, const int64_t* pi, const int64_t
   }
   W.lvl_small.assign(first_small.begin(), first_small.begin() + plain);
   W.lvl_small.push_back(plain < nlev ? first_small[plain] : (int)W.small.size());
+  for (int l = 0; l + 1 < (int)W.lvl_small.size(); ++l) {
+    int m = 0;
+    for (int i = W.lvl_small[l]; i < W.lvl_small[l + 1]; ++i) m = std::max(m, W.small[i].R - W.small[i].w);
+    W.lvl_small_m.push_back(m);
+  }
   // rows below per backward partial: doubled until the partials fit
   int chunk = 512;
   auto parts = [&](int s) {
