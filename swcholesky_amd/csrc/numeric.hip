@@ -1916,14 +1916,16 @@ template <bool FORWARD>
 void launch_small(swc_handle* h, const SweepRun& a, int level) {
   const std::vector<int>& ls = h->plan.sweeps.lvl_small;
   const int s0 = ls[level], ns = ls[level + 1] - s0;
-  if (a.nrhs == 1 && h->plan.sweeps.lvl_small_m[level] <= 16)
-    hipLaunchKernelGGL((k_sweep_small16<FORWARD>), dim3((ns + 15) / 16), dim3(kThreads), 0, h->stream, a,
-                       s0, ns);
-  else if (a.nrhs == 1)
-    hipLaunchKernelGGL((k_sweep_small<FORWARD, 1>), dim3((ns + 3) / 4, 1), dim3(kThreads), 0,
-                       h->stream, a, s0, ns);
-  else
-    hipLaunchKernelGGL((k_sweep_small<FORWARD, 4>), dim3((ns + 3) / 4, (a.nrhs + 3) / 4),
+  // the packed ones and the others wait for nothing of the level: any order
+  const int n16 = a.nrhs == 1 ? h->plan.sweeps.lvl_small16[level] : 0, nw = ns - n16;
+  if (n16 > 0)
+    hipLaunchKernelGGL((k_sweep_small16<FORWARD>), dim3((n16 + 15) / 16), dim3(kThreads), 0, h->stream,
+                       a, s0, n16);
+  if (nw > 0 && a.nrhs == 1)
+    hipLaunchKernelGGL((k_sweep_small<FORWARD, 1>), dim3((nw + 3) / 4, 1), dim3(kThreads), 0,
+                       h->stream, a, s0 + n16, nw);
+  else if (nw > 0)
+    hipLaunchKernelGGL((k_sweep_small<FORWARD, 4>), dim3((nw + 3) / 4, (a.nrhs + 3) / 4),
                        dim3(kThreads), 0, h->stream, a, s0, ns);
 }
 

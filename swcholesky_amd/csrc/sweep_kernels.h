@@ -797,10 +797,10 @@ k_sweep_small(SweepRun a, int s0, int ns) {
   else small_backward<Q>(a, s, r0, min(Q, a.nrhs - r0), lane);
 }
 
-// A level's launch when none of its supernodes has more than 16 rows below, one right-hand
+// A leading level's supernodes with at most 16 rows below (lvl_small16), one right-hand
 // side: 16 lanes each, four to a wave.  The leaves of large forests: a wave a supernode
 // leaves three lanes of four idle and pays its chain of 16 columns once a supernode (a
-// solve of 4096 2D instances: 8.4 ms in its six leaf launches, 4.8 with two of them this).  Same
+// solve of 4096 2D instances: 8.4 ms in its six leaf launches, 4.6 with this).  Same
 // sums in the same order as small_forward and small_backward, bitwise.  What it reads has
 // been published by earlier launches, so nothing is waited for.
 template <bool FORWARD>

@@ -46,10 +46,13 @@ void build_sweeps(int nsuper, const int* super, const int64_t* pi, const int64_t
   }
   W.lvl_small.assign(first_small.begin(), first_small.begin() + plain);
   W.lvl_small.push_back(plain < nlev ? first_small[plain] : (int)W.small.size());
+  // Of a leading level, the supernodes with at most 16 rows below come first: 16 lanes each
+  // in a launch of their own, where they are all or again 2048.
   for (int l = 0; l + 1 < (int)W.lvl_small.size(); ++l) {
-    int m = 0;
-    for (int i = W.lvl_small[l]; i < W.lvl_small[l + 1]; ++i) m = std::max(m, W.small[i].R - W.small[i].w);
-    W.lvl_small_m.push_back(m);
+    const auto b = W.small.begin() + W.lvl_small[l], e = W.small.begin() + W.lvl_small[l + 1];
+    const auto few = [](const SweepSmall& s) { return s.R - s.w <= 16; };
+    const int n16 = (int)(std::stable_partition(b, e, few) - b);
+    W.lvl_small16.push_back(n16 == e - b || n16 >= 2048 ? n16 : 0);
   }
   // rows below per backward partial: doubled until the partials fit
   int chunk = 512;

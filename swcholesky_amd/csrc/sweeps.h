@@ -58,7 +58,7 @@ struct SweepItem {
 
 struct SweepPlan {
   std::vector<SweepSmall> small;   // by level, ascending
-  std::vector<int> lvl_small_m;    // most rows below of a small one, for those launches
+  std::vector<int> lvl_small16;    // of those, first in their level: the ones taken 16 lanes each
   std::vector<int> lvl_small;      // small ones of the launches before the persistent one:
                                    // level l holds [lvl_small[l], lvl_small[l + 1])
   std::vector<SweepItem> fwd, bwd;
