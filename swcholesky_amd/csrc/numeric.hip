@@ -2216,8 +2216,7 @@ int refine_device(swc_handle* h, const double* Bt, double* Xt, int nrhs, double 
 int selinv_setup(swc_handle* h) {
   if (h->dNodes) return SWC_OK;
   hipStream_t st = h->stream;
-  h->sel = swc::build_selinv(h->n, h->nsuper, h->super.data(), h->pi.data(), h->px.data(), h->Ls.data(),
-                             h->pruneptr.data(), h->pruneset.data());
+  h->sel = swc::build_selinv(h->n, h->nsuper, h->super.data(), h->pi.data(), h->px.data(), h->Ls.data());
   swc::SelPlan& S = h->sel;
   int rc = SWC_OK;
   if (!rc) rc = upload(&h->dSelRuns, S.runs.data(), S.runs.size(), st);

@@ -611,8 +611,8 @@ void build_plan(int n, int nsuper, const int* super, const int64_t* pi, const in
 
   // the backward partials take the place (and at most the room) that the row blocks'
   // partial sums of one solve level would
-  build_sweeps(nsuper, super, pi, px, voff.data(), prunePtr, pruneSet,
-               (int64_t)std::max(P.max_lvl_fblk, 1) * SPW, P.sweeps);
+  build_sweeps(nsuper, super, pi, px, Ls, voff.data(), (int64_t)std::max(P.max_lvl_fblk, 1) * SPW,
+               P.sweeps);
 
   // ---- flatten: tiles by level (stable), tasks, TRSM lists ----
   // Within a level the most expensive tiles go first (longest-processing-time

@@ -2,15 +2,17 @@
 
 #include <algorithm>
 
+#include "sweeps.h"
+
 namespace swc {
 
 SelPlan build_selinv(int n, int ns, const int* super, const int64_t* pi, const int64_t* px,
-                     const int* Ls, const int* pptr, const int* pset) {
+                     const int* Ls) {
   SelPlan P;
-  std::vector<int> lev(ns, 0), col2sup(n);
+  const std::vector<int> lev = supernode_levels(ns, super, pi, Ls);
+  std::vector<int> col2sup(n);
   int nlev = 0;
   for (int s = 0; s < ns; ++s) {
-    for (int t = pptr[s]; t < pptr[s + 1]; ++t) lev[s] = std::max(lev[s], lev[pset[t]] + 1);
     nlev = std::max(nlev, lev[s] + 1);
     for (int c = super[s]; c < super[s + 1]; ++c) col2sup[c] = s;
   }

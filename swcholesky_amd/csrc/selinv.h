@@ -65,8 +65,8 @@ struct SelPlan {
 };
 
 // ns supernodes: super (first columns, ns + 1), pi (row list offsets), px (value offsets),
-// rows Ls, descendants of s in pset[pptr[s] .. pptr[s + 1]).
+// rows Ls.
 SelPlan build_selinv(int n, int ns, const int* super, const int64_t* pi, const int64_t* px,
-                     const int* Ls, const int* pptr, const int* pset);
+                     const int* Ls);
 
 }  // namespace swc

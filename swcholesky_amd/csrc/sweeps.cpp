@@ -5,20 +5,31 @@
 
 namespace swc {
 
-void build_sweeps(int nsuper, const int* super, const int64_t* pi, const int64_t* px,
-                  const int64_t* voff, const int* prunePtr, const int* pruneSet, int64_t maxpart,
-                  SweepPlan& W) {
+std::vector<int> supernode_levels(int nsuper, const int* super, const int64_t* pi, const int* Ls) {
+  std::vector<int> lev(nsuper, 0), col2sup(nsuper ? super[nsuper] : 0);
+  for (int s = 0; s < nsuper; ++s)
+    for (int c = super[s]; c < super[s + 1]; ++c) col2sup[c] = s;
+  for (int s = 0; s < nsuper; ++s) {  // rows below belong to later supernodes
+    const int* r = Ls + pi[s] + (super[s + 1] - super[s]);
+    const int* end = Ls + pi[s + 1];
+    while (r < end) {
+      const int t = col2sup[*r];
+      lev[t] = std::max(lev[t], lev[s] + 1);
+      while (r < end && *r < super[t + 1]) ++r;
+    }
+  }
+  return lev;
+}
+
+void build_sweeps(int nsuper, const int* super, const int64_t* pi, const int64_t* px, const int* Ls,
+                  const int64_t* voff, int64_t maxpart, SweepPlan& W) {
   W = SweepPlan();
   auto width = [&](int s) { return super[s + 1] - super[s]; };
   auto nrows = [&](int s) { return (int)(pi[s + 1] - pi[s]); };
   auto small = [&](int s) { return width(s) <= 16 && nrows(s) - width(s) <= kSmallRows; };
-  std::vector<int> lev(nsuper, 0);
+  const std::vector<int> lev = supernode_levels(nsuper, super, pi, Ls);
   int nlev = 0;
-  for (int s = 0; s < nsuper; ++s) {
-    for (int t = prunePtr[s]; t < prunePtr[s + 1]; ++t)
-      lev[s] = std::max(lev[s], lev[pruneSet[t]] + 1);
-    nlev = std::max(nlev, lev[s] + 1);
-  }
+  for (int s = 0; s < nsuper; ++s) nlev = std::max(nlev, lev[s] + 1);
   std::vector<int> lptr(nlev + 1, 0), order(nsuper), nsmall(nlev, 0);
   for (int s = 0; s < nsuper; ++s) {
     lptr[lev[s] + 1]++;

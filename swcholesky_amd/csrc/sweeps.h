@@ -65,9 +65,13 @@ struct SweepPlan {
   int64_t psize = 0;               // doubles of backward partials per right-hand side
 };
 
+// Level of every supernode: one above the highest of those whose rows below meet its
+// columns.  From the row lists, which say what the sweeps (and the selected inverse) read and
+// wait for; a caller's descendant sets may leave out a supernode whose rows hold only zeros.
+std::vector<int> supernode_levels(int nsuper, const int* super, const int64_t* pi, const int* Ls);
+
 // voff[s]: offset of the contribution vector of s.  maxpart: most doubles of partials.
-void build_sweeps(int nsuper, const int* super, const int64_t* pi, const int64_t* px,
-                  const int64_t* voff, const int* prunePtr, const int* pruneSet, int64_t maxpart,
-                  SweepPlan& W);
+void build_sweeps(int nsuper, const int* super, const int64_t* pi, const int64_t* px, const int* Ls,
+                  const int64_t* voff, int64_t maxpart, SweepPlan& W);
 
 }  // namespace swc
