@@ -235,6 +235,11 @@ int swc_plan_stats(const swc_handle* h, int64_t* out, double* flops);
  * launch's useful (lower-triangle) update flops; *nlevel = number of levels.
  * No counterpart in the reference: instrumentation of the GPU schedule. */
 int swc_level_timings(const swc_handle* h, double* out, int cap, int* nlevel);
+/* For tests of what a full device does: the nth device allocation that a handle makes on
+ * the calling thread from now on is refused as if there were no room (0: none).  A handle
+ * that is refused memory first gives back the factorization's update matrices, about as
+ * much as L, and its factorizations then run left-looking until the next upload. */
+int swc_refuse_allocation(int nth);
 /* With graphs on (default), swc_factor (from its second call on a structure) and the
  * solves replay launch sequences captured once per structure (hipGraph) instead of
  * launching level by level. */

@@ -48,6 +48,7 @@ SIGNATURES = {
     "swc_plan_stats": (c_int, [c_vp, c_vp, ctypes.POINTER(c_dbl)]),
     "swc_level_timings": (c_int, [c_vp, c_vp, c_int, c_vp]),
     "swc_set_profiling": (c_int, [c_vp, c_int]),
+    "swc_refuse_allocation": (c_int, [c_int]),
     "swc_set_graphs": (c_int, [c_vp, c_int]),
     "swc_selected_inverse": (c_int, [c_vp, c_vp, c_int]),
     "swc_logdet": (c_int, [c_vp, ctypes.POINTER(c_dbl)]),

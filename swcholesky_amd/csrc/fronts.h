@@ -3,7 +3,7 @@
 //
 // Every supernode s (w columns, R rows, m = R - w rows below) has, beside its
 // block of L, a frontal update matrix U_s (m x m, lower triangle, column-major) in
-// an arena behind L in the same allocation:
+// an arena, whose offsets count on behind L's (rounded up to 32 values):
 //   U_s = (sum over children c of U_c at their landing positions) - L21 L21^T,
 // and a supernode's own columns start from A plus the children's U_c.  So every
 // product is a dense block of one supernode (rows consecutive, inner dimension the
@@ -15,7 +15,8 @@
 // left-looking -> multifrontal (ms, same solve): 64^3 26.6 -> 21.4, 32^3 mixed 6.01 ->
 // 4.94, 2D 100^2 1.04 -> 0.68, a mesh of 20,000 points 2.11 -> 1.41, 256 uneven 2D
 // instances 4.69 -> 2.81.  The arena takes about as much memory as L (1.5 GB beside
-// 1.6 GB at 64^3).
+// 1.6 GB at 64^3) and holds nothing between factorizations, so the handle gives it up first
+// when the device has no room.
 //
 // A supernode is cut into panels of at most 64 columns, its rows into tiles of at
 // most 64.  Level l runs two launches: F_l factors the panels of level l (a first

@@ -12,6 +12,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <initializer_list>
 #include <memory>
 #include <mutex>
 #include <new>
@@ -1422,6 +1423,9 @@ struct swc_handle {
   swc::HLevelSchedule hlevel;  // non-empty: factor levels follow this schedule
   bool multifrontal = false;   // the factor runs the front plan, else the left-looking one
   swc::FrontPlan fronts;
+  swc::PlanParams up_params;   // the parameters of the uploaded structure's plan
+  bool uploading = false;      // an upload is under way: it sees to a refused allocation itself
+  bool no_room = false;        // one was refused in it
   int n = 0, nsuper = 0;
   int64_t nvals = 0;  // number of values swc_factor expects
   std::vector<int> super, Ls;
@@ -1430,6 +1434,7 @@ struct swc_handle {
   std::vector<int> pruneptr, pruneset;
   // device buffers
   double* dL = nullptr;
+  double* dU = nullptr;  // the front plan's arena
   float* dLf = nullptr;  // FP32 shadow of L, written with it when FP32 updates are on
   int64_t lf_cap = 0;    // elements allocated at dLf
   int* dLs = nullptr;
@@ -1537,7 +1542,7 @@ struct swc_handle {
   }
   void release() {
     drop_graphs();
-    (void)hipFree(dL); (void)hipFree(dLf); (void)hipFree(dLs); (void)hipFree(dTiles); (void)hipFree(dTasks);
+    (void)hipFree(dL); (void)hipFree(dU); (void)hipFree(dLf); (void)hipFree(dLs); (void)hipFree(dTiles); (void)hipFree(dTasks);
     (void)hipFree(dGptr); (void)hipFree(dGidx); (void)hipFree(dSweepSmall); (void)hipFree(dSweepFwd); (void)hipFree(dSweepBwd); (void)hipFree(dSweepSync); (void)hipFree(dV); (void)hipFree(dPb); (void)hipFree(dY); (void)hipFree(dFtiles); (void)hipFree(dFused);
     (void)hipFree(dGathers); (void)hipFree(dAents); (void)hipFree(dFactorTiles); (void)hipFree(dSmall); (void)hipFree(dFrontTiles);
     (void)hipFree(dCounters); (void)hipFree(dDagItems); (void)hipFree(dDagDeps); (void)hipFree(dDagSync); (void)hipFree(dDiag); (void)hipFree(dAmap); (void)hipFree(dPerm);
@@ -1546,7 +1551,7 @@ struct swc_handle {
     (void)hipFree(dRef);
     (void)hipFree(dZ); (void)hipFree(dArena); (void)hipFree(dNodes); (void)hipFree(dSelM); (void)hipFree(dSelRuns);
     (void)hipFree(dSelJrun); (void)hipFree(dSelRel); (void)hipFree(dSelItems); (void)hipFree(dDiagPos); (void)hipFree(dQi); (void)hipFree(dQj);
-    dL = nullptr; dLf = nullptr; dLs = nullptr; dTiles = nullptr; dTasks = nullptr;
+    dL = nullptr; dU = nullptr; dLf = nullptr; dLs = nullptr; dTiles = nullptr; dTasks = nullptr;
     dGptr = nullptr; dGidx = nullptr; dSweepSmall = nullptr; dSweepFwd = nullptr; dSweepBwd = nullptr; dSweepSync = nullptr; dV = nullptr; dPb = nullptr; dY = nullptr; dFtiles = nullptr; dFused = nullptr; dGathers = nullptr; dAents = nullptr; dFactorTiles = nullptr; dSmall = nullptr; dFrontTiles = nullptr; dCounters = nullptr; dDagItems = nullptr; dDagDeps = nullptr; dDagSync = nullptr; dDiag = nullptr; dAmap = nullptr; dPerm = nullptr;
     dVals = nullptr; dWork = nullptr; dInfo = nullptr;
     dRp = nullptr; dCi = nullptr; dVmap = nullptr; dAf = nullptr; dScal = nullptr; dPart = nullptr; dNormPart = nullptr;
@@ -1565,13 +1570,39 @@ struct swc_handle {
 
 namespace {
 
+// Device allocations of the calling thread until one is refused (0: none is); for tests.
+thread_local int refuse_allocation = 0;
+
+bool give_up_arena(swc_handle* h);
+
+// Device memory for a handle.  The front plan's arena is as large as L, and only
+// factorizations use it: where there is no room beside it, it is given back, and the
+// handle's later factorizations run left-looking.
+template <class Alloc>
+hipError_t with_room(swc_handle* h, Alloc&& alloc) {
+  auto attempt = [&] {
+    if (refuse_allocation > 0 && --refuse_allocation == 0) return hipErrorOutOfMemory;
+    return alloc();
+  };
+  hipError_t e = attempt();
+  if (e != hipErrorOutOfMemory) return e;
+  (void)hipGetLastError();
+  if (h->uploading) h->no_room = true;
+  else if (give_up_arena(h)) e = attempt();
+  return e;
+}
+hipError_t device_malloc(swc_handle* h, void** p, size_t bytes) {
+  return with_room(h, [&] { return hipMalloc(p, bytes); });
+}
+
 template <class T>
-int upload(T** dst, const T* src, size_t count, hipStream_t s) {
+int upload(T** dst, const T* src, size_t count, swc_handle* h) {
   (void)hipFree(*dst);
   *dst = nullptr;
   const size_t alloc = count == 0 ? 1 : count;
-  SWC_HIP(hipMalloc((void**)dst, alloc * sizeof(T)));
-  if (src && count) SWC_HIP(hipMemcpyAsync(*dst, src, count * sizeof(T), hipMemcpyHostToDevice, s));
+  SWC_HIP(device_malloc(h, (void**)dst, alloc * sizeof(T)));
+  if (src && count)
+    SWC_HIP(hipMemcpyAsync(*dst, src, count * sizeof(T), hipMemcpyHostToDevice, h->stream));
   return SWC_OK;
 }
 
@@ -1633,15 +1664,15 @@ int ensure_work(swc_handle* h, int cols) {
   h->dWork = h->dV = h->dY = h->dPb = h->dPart = h->dRef = nullptr;
   h->work_cols = 0;
   const Plan& P = h->plan;
-  SWC_HIP(hipMalloc((void**)&h->dPart, sizeof(double) * (size_t)kRedBlocks * cols));
+  SWC_HIP(device_malloc(h, (void**)&h->dPart, sizeof(double) * (size_t)kRedBlocks * cols));
   (void)hipFree(h->dScal);
   h->dScal = nullptr;
-  SWC_HIP(hipMalloc((void**)&h->dScal, sizeof(double) * (size_t)(64 + 4 * cols)));
-  SWC_HIP(hipMalloc((void**)&h->dRef, sizeof(double) * (size_t)5 * h->n * cols));
-  SWC_HIP(hipMalloc((void**)&h->dWork, sizeof(double) * (size_t)h->n * cols));
-  SWC_HIP(hipMalloc((void**)&h->dV, sizeof(double) * (size_t)std::max<int64_t>(P.vsize, 1) * cols));
-  SWC_HIP(hipMalloc((void**)&h->dY, sizeof(double) * (size_t)h->n * cols));
-  SWC_HIP(hipMalloc((void**)&h->dPb, sizeof(double) * (size_t)std::max(P.max_lvl_fblk, 1) * swc::SPW * cols));
+  SWC_HIP(device_malloc(h, (void**)&h->dScal, sizeof(double) * (size_t)(64 + 4 * cols)));
+  SWC_HIP(device_malloc(h, (void**)&h->dRef, sizeof(double) * (size_t)5 * h->n * cols));
+  SWC_HIP(device_malloc(h, (void**)&h->dWork, sizeof(double) * (size_t)h->n * cols));
+  SWC_HIP(device_malloc(h, (void**)&h->dV, sizeof(double) * (size_t)std::max<int64_t>(P.vsize, 1) * cols));
+  SWC_HIP(device_malloc(h, (void**)&h->dY, sizeof(double) * (size_t)h->n * cols));
+  SWC_HIP(device_malloc(h, (void**)&h->dPb, sizeof(double) * (size_t)std::max(P.max_lvl_fblk, 1) * swc::SPW * cols));
   h->work_cols = cols;
   return SWC_OK;
 }
@@ -2219,9 +2250,9 @@ int selinv_setup(swc_handle* h) {
   h->sel = swc::build_selinv(h->n, h->nsuper, h->super.data(), h->pi.data(), h->px.data(), h->Ls.data());
   swc::SelPlan& S = h->sel;
   int rc = SWC_OK;
-  if (!rc) rc = upload(&h->dSelRuns, S.runs.data(), S.runs.size(), st);
-  if (!rc) rc = upload(&h->dSelJrun, S.jrun.data(), S.jrun.size(), st);
-  if (!rc) rc = upload(&h->dSelRel, (const int*)nullptr, (size_t)S.nrel, st);
+  if (!rc) rc = upload(&h->dSelRuns, S.runs.data(), S.runs.size(), h);
+  if (!rc) rc = upload(&h->dSelJrun, S.jrun.data(), S.jrun.size(), h);
+  if (!rc) rc = upload(&h->dSelRel, (const int*)nullptr, (size_t)S.nrel, h);
   // the item lists, one after the other
   std::vector<swc::SelItem> items;
   const std::vector<swc::SelItem>* lists[kSelLists] = {&S.diag,   &S.cols,  &S.u,   &S.gather,
@@ -2233,11 +2264,11 @@ int selinv_setup(swc_handle* h) {
     h->sel_items[q] = items.size();
     items.insert(items.end(), lists[q]->begin(), lists[q]->end());
   }
-  if (!rc) rc = upload(&h->dSelItems, items.data(), items.size(), st);
-  if (!rc) rc = upload(&h->dSelM, (const double*)nullptr, (size_t)S.msize, st);
-  if (!rc) rc = upload(&h->dArena, (const double*)nullptr, (size_t)S.zsize, st);
-  if (!rc) rc = upload(&h->dZ, (const double*)nullptr, (size_t)h->plan.xsize, st);
-  if (!rc) rc = upload(&h->dNodes, S.nodes.data(), S.nodes.size(), st);
+  if (!rc) rc = upload(&h->dSelItems, items.data(), items.size(), h);
+  if (!rc) rc = upload(&h->dSelM, (const double*)nullptr, (size_t)S.msize, h);
+  if (!rc) rc = upload(&h->dArena, (const double*)nullptr, (size_t)S.zsize, h);
+  if (!rc) rc = upload(&h->dZ, (const double*)nullptr, (size_t)h->plan.xsize, h);
+  if (!rc) rc = upload(&h->dNodes, S.nodes.data(), S.nodes.size(), h);
   if (rc) {
     (void)hipStreamSynchronize(st);  // the uploads read vectors of this frame
     return rc;
@@ -2363,111 +2394,119 @@ bool covers_values(const A2Pattern& a, int n) {
   return true;
 }
 
-// Structure part of an upload: the plan (solve part only without A2), L and its FP32
-// copy, the row lists and the plan arrays on the device.  The factorization runs the
-// multifrontal plan (fronts.h) where the structure has one and its arena fits the
-// device, else, and for an H-level schedule, the left-looking one (plan.h).
-int upload_structure(swc_handle* h, int n, const int* blockSet, int supNo, const size_t* lC,
-                     const int* Ls, const size_t* Li_ptr, const int* prunePtr,
-                     const int* pruneSet, A2Pattern* a2) {
-  const bool factor = a2 != nullptr;
-  if (int rc = validate_structure(n, blockSet, supNo, lC, Ls, Li_ptr)) return rc;
-  // pruneSet may be null when it is empty (no supernode has descendants)
-  if (!prunePtr || (!pruneSet && prunePtr[supNo] != 0) || prunePtr[0] != 0)
-    return swc_set_error(SWC_EINVAL, "structure: bad descendant sets");
-  for (int s = 0; s < supNo; ++s)
-    if (prunePtr[s + 1] < prunePtr[s]) return swc_set_error(SWC_EINVAL, "structure: bad descendant sets");
-  h->factored = false;
-  h->has_values = false;
-  h->drop_graphs();
-  h->work_cols = 0;  // the solve buffers are sized by the structure: rebuilt on next use
-  // the old structure's L goes first: if this upload fails part way, no buffer
-  // sized for the old structure is left beside the new plan, and swc_factor
-  // refuses to run until an upload completes
-  (void)hipFree(h->dL);
-  h->dL = nullptr;
-  h->n = n;
-  h->nsuper = supNo;
-  h->nvals = 0;
-  h->super.assign(blockSet, blockSet + supNo + 1);
-  h->pi.resize(supNo + 1);
-  h->px.resize(supNo);
-  for (int s = 0; s <= supNo; ++s) h->pi[s] = (int64_t)Li_ptr[blockSet[s]];
-  for (int s = 0; s < supNo; ++s) h->px[s] = (int64_t)lC[blockSet[s]];
-  const int64_t ssize = h->pi[supNo];
-  h->Ls.assign(Ls, Ls + ssize);
-  h->pruneptr.assign(prunePtr, prunePtr + supNo + 1);
-  h->pruneset.assign(pruneSet, pruneSet + prunePtr[supNo]);
+// The plan counts the arena's offsets as if it followed L (rounded up); it is an allocation
+// of its own, `shift` values further on.
+void place_arena(swc::FrontPlan& F, int64_t shift) {
+  for (swc::Gather& g : F.gathers) g.src += shift;
+  for (swc::SmallFront& f : F.small)
+    if (f.R > f.w) f.ubase += shift;
+  for (swc::FrontTile& u : F.utiles)
+    if (u.upd) u.vbase += shift;
+}
+
+void free_all(std::initializer_list<void**> ps) {
+  for (void** p : ps) {
+    (void)hipFree(*p);
+    *p = nullptr;
+  }
+}
+
+// Work lists of the left-looking factorization.
+int upload_left_looking(swc_handle* h) {
+  const Plan& P = h->plan;
+  int rc = upload(&h->dTiles, P.tiles.data(), P.tiles.size(), h);
+  if (!rc) rc = upload(&h->dTasks, P.tasks.data(), P.tasks.size(), h);
+  if (!rc) rc = upload(&h->dFtiles, P.ftiles.data(), P.ftiles.size(), h);
+  if (!rc) rc = upload(&h->dFused, P.fused.data(), P.fused.size(), h);
+  if (!rc) rc = upload(&h->dCounters, (const int*)nullptr, (size_t)std::max(P.nlevel, 1), h);
+  if (!rc) rc = upload(&h->dDagItems, P.dag_items.data(), P.dag_items.size(), h);
+  if (!rc) rc = upload(&h->dDagDeps, P.dag_deps.data(), P.dag_deps.size(), h);
+  if (!rc)
+    rc = upload(&h->dDagSync, (const int*)nullptr, 2 + P.dag_items.size() + (size_t)P.npanel, h);
+  return rc;
+}
+
+// Leaves the multifrontal plan: its lists and arena are freed.
+void drop_fronts(swc_handle* h) {
+  (void)hipStreamSynchronize(h->stream);  // uploads read the lists
+  free_all({(void**)&h->dU, (void**)&h->dGathers, (void**)&h->dAents, (void**)&h->dFactorTiles,
+            (void**)&h->dSmall, (void**)&h->dFrontTiles});
   h->multifrontal = false;
   h->fronts = swc::FrontPlan();
-  auto plan = [&](bool left_looking) {
-    swc::build_plan(n, supNo, h->super.data(), h->pi.data(), h->px.data(), h->Ls.data(),
-                    prunePtr, pruneSet, h->plan, left_looking, h->params,
-                    h->hlevel.level_ptr.empty() ? nullptr : &h->hlevel);
-  };
-  hipStream_t st = h->stream;
-  int rc = SWC_OK;
-  try {
-    if (factor) a2->ok = a2_positions(h, a2->p, a2->i, a2->pos);
-    int64_t xsize = 0;
-    for (int s = 0; s < supNo; ++s)
-      xsize = std::max(xsize, h->px[s] + (h->pi[s + 1] - h->pi[s]) * (h->super[s + 1] - h->super[s]));
-    h->multifrontal =
-        factor && a2->ok && h->hlevel.level_ptr.empty() && covers_values(*a2, n) &&
-        swc::build_fronts(n, supNo, h->super.data(), h->pi.data(), h->px.data(), xsize,
-                          h->Ls.data(), prunePtr, pruneSet, a2->p, a2->src, a2->pos.data(),
-                          h->params.rlb, h->fronts);
-    plan(factor && !h->multifrontal);
-    if (h->multifrontal) {
-      // the arena follows L in one allocation
-      rc = upload(&h->dL, (const double*)nullptr, (size_t)(h->plan.xsize + h->fronts.usize + kLoadPad), st);
-      if (rc && h->fronts.usize > 0) {
-        (void)hipGetLastError();
-        h->multifrontal = false;
-        plan(true);
-      } else if (!rc) {
-        // above the diagonal blocks' diagonals L is never written
-        hipLaunchKernelGGL(k_fill, dim3(grid_for(h->plan.xsize)), dim3(kThreads), 0, st, h->dL,
-                           h->plan.xsize, 0.0);
-      }
-    }
-    if (!h->multifrontal) {
-      h->fronts = swc::FrontPlan();
-      rc = upload(&h->dL, (const double*)nullptr, (size_t)h->plan.xsize, st);
-    }
-  } catch (const std::bad_alloc&) {
-    return swc_set_error(SWC_ENOMEM, "upload: out of host memory");
-  } catch (const std::exception& e) {
-    return swc_set_error(SWC_EINVAL, std::string("upload: ") + e.what());
+}
+
+void plan_structure(swc_handle* h, bool left_looking) {
+  swc::build_plan(h->n, h->nsuper, h->super.data(), h->pi.data(), h->px.data(), h->Ls.data(),
+                  h->pruneptr.data(), h->pruneset.data(), h->plan, left_looking, h->up_params,
+                  h->hlevel.level_ptr.empty() ? nullptr : &h->hlevel);
+}
+
+// After an upload: gives the arena's memory back and prepares the left-looking
+// factorization.  The factor in L and the solves stay as they are.  False where there is
+// no arena or no room even so; swc_factor then refuses until the next upload.
+bool give_up_arena(swc_handle* h) {
+  if (!h->multifrontal || !h->dU) return false;
+  for (auto& g : h->fgraph) {
+    if (g) (void)hipGraphExecDestroy(g);
+    g = nullptr;
   }
+  for (auto& f : h->factor_seen) f = false;
+  drop_fronts(h);
+  h->lvl_tile_ms.clear();
+  int rc = SWC_ENOMEM;
+  try {
+    swc::Plan left;
+    // an H-level schedule set since the upload belongs to the next one
+    swc::build_plan(h->n, h->nsuper, h->super.data(), h->pi.data(), h->px.data(), h->Ls.data(),
+                    h->pruneptr.data(), h->pruneset.data(), left, true, h->up_params, nullptr);
+    h->plan = std::move(left);
+    rc = upload_left_looking(h);
+    if (!rc)
+      rc = upload(&h->dDiag, (const double*)nullptr, (size_t)std::max<int64_t>(h->plan.diag_scratch, 1), h);
+  } catch (const std::exception&) {
+  }
+  if (rc) h->has_values = false;
+  return rc == SWC_OK && hipStreamSynchronize(h->stream) == hipSuccess;
+}
+
+// L, its FP32 copy, the row lists and the plans' arrays on the device.
+int upload_arrays(swc_handle* h, bool factor) {
+  hipStream_t st = h->stream;
   const Plan& P = h->plan;
-  const swc::FrontPlan& F = h->fronts;
-  if (!rc) rc = upload(&h->dGathers, F.gathers.data(), F.gathers.size(), st);
-  if (!rc) rc = upload(&h->dAents, F.aents.data(), F.aents.size(), st);
-  if (!rc) rc = upload(&h->dFactorTiles, F.ftiles.data(), F.ftiles.size(), st);
-  if (!rc) rc = upload(&h->dSmall, F.small.data(), F.small.size(), st);
-  if (!rc) rc = upload(&h->dFrontTiles, F.utiles.data(), F.utiles.size(), st);
+  swc::FrontPlan& F = h->fronts;
+  int rc = upload(&h->dL, (const double*)nullptr, (size_t)(P.xsize + kLoadPad), h);
+  if (!rc && h->multifrontal) {
+    // above the diagonal blocks' diagonals L is never written
+    hipLaunchKernelGGL(k_fill, dim3(grid_for(P.xsize)), dim3(kThreads), 0, st, h->dL, P.xsize, 0.0);
+    const int64_t ubase = (P.xsize + 31) & ~(int64_t)31;  // where the plan has the arena
+    if (F.usize > 0) rc = upload(&h->dU, (const double*)nullptr, (size_t)(P.xsize + F.usize - ubase), h);
+    if (!rc && F.usize > 0) place_arena(F, ((intptr_t)h->dU - (intptr_t)h->dL) / (intptr_t)sizeof(double) - ubase);
+  }
+  if (h->multifrontal) {
+    if (!rc) rc = upload(&h->dGathers, F.gathers.data(), F.gathers.size(), h);
+    if (!rc) rc = upload(&h->dAents, F.aents.data(), F.aents.size(), h);
+    if (!rc) rc = upload(&h->dFactorTiles, F.ftiles.data(), F.ftiles.size(), h);
+    if (!rc) rc = upload(&h->dSmall, F.small.data(), F.small.size(), h);
+    if (!rc) rc = upload(&h->dFrontTiles, F.utiles.data(), F.utiles.size(), h);
+  } else if (!rc) {
+    rc = upload_left_looking(h);
+  }
   // the FP32 shadow follows the structure's size whatever the current mode: a
   // later switch to a mixed mode finds it sized for this structure
   (void)hipFree(h->dLf);
   h->dLf = nullptr;
   h->lf_cap = 0;
   if (!rc && h->precision > 0 && factor) {
-    rc = upload(&h->dLf, (const float*)nullptr, (size_t)(P.xsize + kLoadPad), st);
+    rc = upload(&h->dLf, (const float*)nullptr, (size_t)(P.xsize + kLoadPad), h);
     if (!rc) h->lf_cap = P.xsize;
   }
-  if (!rc) rc = upload(&h->dLs, h->Ls.data(), h->Ls.size(), st);
-  if (!rc) rc = upload(&h->dTiles, P.tiles.data(), P.tiles.size(), st);
-  if (!rc) rc = upload(&h->dTasks, P.tasks.data(), P.tasks.size(), st);
-  if (!rc) rc = upload(&h->dGptr, P.gptr.data(), P.gptr.size(), st);
-  if (!rc) rc = upload(&h->dGidx, P.gidx.data(), P.gidx.size(), st);
-  if (!rc) rc = upload(&h->dSweepSmall, P.sweeps.small.data(), P.sweeps.small.size(), st);
-  if (!rc) rc = upload(&h->dSweepFwd, P.sweeps.fwd.data(), P.sweeps.fwd.size(), st);
-  if (!rc) rc = upload(&h->dSweepBwd, P.sweeps.bwd.data(), P.sweeps.bwd.size(), st);
-  if (!rc) rc = upload(&h->dSweepSync, (const int*)nullptr, 4, st);
-  if (!rc) rc = upload(&h->dFtiles, P.ftiles.data(), P.ftiles.size(), st);
-  if (!rc) rc = upload(&h->dFused, P.fused.data(), P.fused.size(), st);
-  if (!rc) rc = upload(&h->dCounters, (const int*)nullptr, (size_t)std::max(P.nlevel, 1), st);
+  if (!rc) rc = upload(&h->dLs, h->Ls.data(), h->Ls.size(), h);
+  if (!rc) rc = upload(&h->dGptr, P.gptr.data(), P.gptr.size(), h);
+  if (!rc) rc = upload(&h->dGidx, P.gidx.data(), P.gidx.size(), h);
+  if (!rc) rc = upload(&h->dSweepSmall, P.sweeps.small.data(), P.sweeps.small.size(), h);
+  if (!rc) rc = upload(&h->dSweepFwd, P.sweeps.fwd.data(), P.sweeps.fwd.size(), h);
+  if (!rc) rc = upload(&h->dSweepBwd, P.sweeps.bwd.data(), P.sweeps.bwd.size(), h);
+  if (!rc) rc = upload(&h->dSweepSync, (const int*)nullptr, 4, h);
   if (!rc && h->sweep_cap == 0) {
     // two workgroups to a CU (what the sweeps' registers allow); any number is safe
     int ncu = 0;
@@ -2489,10 +2528,6 @@ int upload_structure(swc_handle* h, int n, const int* blockSet, int supNo, const
     else
       for (int m = 0; m < 3; ++m) h->fused_cap[m] = std::max(1, per[m]) * std::max(ncu, 1);
   }
-  if (!rc) rc = upload(&h->dDagItems, P.dag_items.data(), P.dag_items.size(), st);
-  if (!rc) rc = upload(&h->dDagDeps, P.dag_deps.data(), P.dag_deps.size(), st);
-  if (!rc)
-    rc = upload(&h->dDagSync, (const int*)nullptr, 2 + P.dag_items.size() + (size_t)P.npanel, st);
   if (!rc && h->dag_cap[0] == 0) {
     int ncu = 0, per[3] = {0, 0, 0};
     hipError_t e = hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, h->device);
@@ -2506,8 +2541,79 @@ int upload_structure(swc_handle* h, int n, const int* blockSet, int supNo, const
   }
   if (!rc)
     rc = upload(&h->dDiag, (const double*)nullptr,
-                (size_t)std::max(P.diag_scratch, F.diag_scratch), st);
-  if (!rc) rc = upload(&h->dNormPart, (const double*)nullptr, kSetupBlocks, st);
+                (size_t)std::max(P.diag_scratch, F.diag_scratch), h);
+  if (!rc) rc = upload(&h->dNormPart, (const double*)nullptr, kSetupBlocks, h);
+  return rc;
+}
+
+// Structure part of an upload: the plan (solve part only without A2), L and its FP32
+// copy, the row lists and the plan arrays on the device.  The factorization runs the
+// multifrontal plan (fronts.h) where the structure has one and its arena fits the
+// device beside everything else, else, and for an H-level schedule, the left-looking one
+// (plan.h).
+int upload_structure(swc_handle* h, int n, const int* blockSet, int supNo, const size_t* lC,
+                     const int* Ls, const size_t* Li_ptr, const int* prunePtr,
+                     const int* pruneSet, A2Pattern* a2) {
+  const bool factor = a2 != nullptr;
+  if (int rc = validate_structure(n, blockSet, supNo, lC, Ls, Li_ptr)) return rc;
+  // pruneSet may be null when it is empty (no supernode has descendants)
+  if (!prunePtr || (!pruneSet && prunePtr[supNo] != 0) || prunePtr[0] != 0)
+    return swc_set_error(SWC_EINVAL, "structure: bad descendant sets");
+  for (int s = 0; s < supNo; ++s)
+    if (prunePtr[s + 1] < prunePtr[s]) return swc_set_error(SWC_EINVAL, "structure: bad descendant sets");
+  h->factored = false;
+  h->has_values = false;
+  h->drop_graphs();
+  h->work_cols = 0;  // the solve buffers are sized by the structure: rebuilt on next use
+  // the old structure's L goes first: if this upload fails part way, no buffer
+  // sized for the old structure is left beside the new plan, and swc_factor
+  // refuses to run until an upload completes
+  (void)hipFree(h->dL);
+  h->dL = nullptr;
+  drop_fronts(h);
+  free_all({(void**)&h->dTiles, (void**)&h->dTasks, (void**)&h->dFtiles, (void**)&h->dFused, (void**)&h->dCounters,
+            (void**)&h->dDagItems, (void**)&h->dDagDeps, (void**)&h->dDagSync});
+  h->up_params = h->params;
+  h->n = n;
+  h->nsuper = supNo;
+  h->nvals = 0;
+  h->super.assign(blockSet, blockSet + supNo + 1);
+  h->pi.resize(supNo + 1);
+  h->px.resize(supNo);
+  for (int s = 0; s <= supNo; ++s) h->pi[s] = (int64_t)Li_ptr[blockSet[s]];
+  for (int s = 0; s < supNo; ++s) h->px[s] = (int64_t)lC[blockSet[s]];
+  const int64_t ssize = h->pi[supNo];
+  h->Ls.assign(Ls, Ls + ssize);
+  h->pruneptr.assign(prunePtr, prunePtr + supNo + 1);
+  h->pruneset.assign(pruneSet, pruneSet + prunePtr[supNo]);
+  h->uploading = true;
+  h->no_room = false;
+  hipStream_t st = h->stream;
+  int rc = SWC_OK;
+  try {
+    if (factor) a2->ok = a2_positions(h, a2->p, a2->i, a2->pos);
+    int64_t xsize = 0;
+    for (int s = 0; s < supNo; ++s)
+      xsize = std::max(xsize, h->px[s] + (h->pi[s + 1] - h->pi[s]) * (h->super[s + 1] - h->super[s]));
+    h->multifrontal =
+        factor && a2->ok && h->hlevel.level_ptr.empty() && covers_values(*a2, n) &&
+        swc::build_fronts(n, supNo, h->super.data(), h->pi.data(), h->px.data(), xsize,
+                          h->Ls.data(), prunePtr, pruneSet, a2->p, a2->src, a2->pos.data(),
+                          h->params.rlb, h->fronts);
+    if (!h->multifrontal) h->fronts = swc::FrontPlan();
+    plan_structure(h, factor && !h->multifrontal);
+    rc = upload_arrays(h, factor);
+    if (rc && h->fronts.usize > 0 && h->no_room) {
+      drop_fronts(h);
+      plan_structure(h, true);
+      rc = upload_arrays(h, factor);
+    }
+  } catch (const std::bad_alloc&) {
+    rc = swc_set_error(SWC_ENOMEM, "upload: out of host memory");
+  } catch (const std::exception& e) {
+    rc = swc_set_error(SWC_EINVAL, std::string("upload: ") + e.what());
+  }
+  h->uploading = false;
   h->zvalid = false;
   (void)hipFree(h->dZ);
   (void)hipFree(h->dArena);
@@ -2618,15 +2724,15 @@ int swc_upload(swc_handle* h, int n, const int* blockSet, int supNo, const size_
   }
   hipStream_t st = h->stream;
   int rc = SWC_OK;
-  if (!rc) rc = upload(&h->dAmap, amap.data(), amap.size(), st);
-  if (!rc) rc = upload(&h->dVals, (const double*)nullptr, (size_t)h->nvals, st);
-  if (!rc) rc = upload(&h->dRp, frp.data(), frp.size(), st);
-  if (!rc) rc = upload(&h->dCi, fci.data(), fci.size(), st);
-  if (!rc) rc = upload(&h->dVmap, fvm.data(), fvm.size(), st);
-  if (!rc) rc = upload(&h->dAf, (const double*)nullptr, fci.size(), st);
-  if (!rc) rc = upload(&h->dQi, qi.data(), qi.size(), st);
-  if (!rc) rc = upload(&h->dQj, qj.data(), qj.size(), st);
-  if (!rc) rc = upload(&h->dDiagPos, dpos.data(), dpos.size(), st);
+  if (!rc) rc = upload(&h->dAmap, amap.data(), amap.size(), h);
+  if (!rc) rc = upload(&h->dVals, (const double*)nullptr, (size_t)h->nvals, h);
+  if (!rc) rc = upload(&h->dRp, frp.data(), frp.size(), h);
+  if (!rc) rc = upload(&h->dCi, fci.data(), fci.size(), h);
+  if (!rc) rc = upload(&h->dVmap, fvm.data(), fvm.size(), h);
+  if (!rc) rc = upload(&h->dAf, (const double*)nullptr, fci.size(), h);
+  if (!rc) rc = upload(&h->dQi, qi.data(), qi.size(), h);
+  if (!rc) rc = upload(&h->dQj, qj.data(), qj.size(), h);
+  if (!rc) rc = upload(&h->dDiagPos, dpos.data(), dpos.size(), h);
   // the copies above read this frame's vectors: wait for them on every path
   const hipError_t se = hipStreamSynchronize(st);
   if (rc) {
@@ -2679,7 +2785,7 @@ int swc_set_perm(swc_handle* h, const int* perm) {
     seen[perm[k]] = 1;
   }
   h->perm.assign(perm, perm + h->n);
-  return upload(&h->dPerm, h->perm.data(), h->perm.size(), h->stream);
+  return upload(&h->dPerm, h->perm.data(), h->perm.size(), h);
 }
 
 int swc_factor(swc_handle* h, const double* values, int values_on_device, int* info) {
@@ -2859,10 +2965,10 @@ int swc_factor_csc(swc_handle* h, int64_t* Cp, int* Ci, double* Cx, int on_devic
   int64_t* dCp = on_device ? Cp : nullptr;
   int* dCi = on_device ? Ci : nullptr;
   double* dCx = on_device ? Cx : nullptr;
-  hipError_t e = hipMalloc((void**)&dcol, sizeof(CscColumn) * cols.size());
-  if (e == hipSuccess && !on_device) e = hipMalloc((void**)&dCp, sizeof(int64_t) * (h->n + 1));
-  if (e == hipSuccess && !on_device) e = hipMalloc((void**)&dCi, sizeof(int) * std::max<int64_t>(nnz, 1));
-  if (e == hipSuccess && !on_device) e = hipMalloc((void**)&dCx, sizeof(double) * std::max<int64_t>(nnz, 1));
+  hipError_t e = device_malloc(h, (void**)&dcol, sizeof(CscColumn) * cols.size());
+  if (e == hipSuccess && !on_device) e = device_malloc(h, (void**)&dCp, sizeof(int64_t) * (h->n + 1));
+  if (e == hipSuccess && !on_device) e = device_malloc(h, (void**)&dCi, sizeof(int) * std::max<int64_t>(nnz, 1));
+  if (e == hipSuccess && !on_device) e = device_malloc(h, (void**)&dCx, sizeof(double) * std::max<int64_t>(nnz, 1));
   if (e == hipSuccess)
     e = hipMemcpyAsync(dcol, cols.data(), sizeof(CscColumn) * cols.size(), hipMemcpyHostToDevice, st);
   if (e == hipSuccess) {
@@ -2938,7 +3044,7 @@ int swc_set_precision(swc_handle* h, int mode) {
     (void)hipFree(h->dLf);
     h->dLf = nullptr;
     h->lf_cap = 0;
-    SWC_HIP(hipMalloc((void**)&h->dLf, sizeof(float) * (size_t)(h->plan.xsize + kLoadPad)));
+    SWC_HIP(device_malloc(h, (void**)&h->dLf, sizeof(float) * (size_t)(h->plan.xsize + kLoadPad)));
     h->lf_cap = h->plan.xsize;
   }
   h->precision = mode;
@@ -2988,7 +3094,9 @@ int swc_gradient(swc_handle* h, const double* x, int x_on_device, double alpha, 
   double* g = grad_on_device ? grad : h->dRef + h->n;  // dRef holds >= 5 n doubles
   double* gbuf = nullptr;
   if (!grad_on_device) {
-    SWC_HIP(hipMallocAsync((void**)&gbuf, sizeof(double) * std::max<int64_t>(h->nvals, 1), st));
+    SWC_HIP(with_room(h, [&] {
+      return hipMallocAsync((void**)&gbuf, sizeof(double) * std::max<int64_t>(h->nvals, 1), st);
+    }));
     g = gbuf;
   }
   hipLaunchKernelGGL(k_grad_values, dim3(grid_for(h->nvals)), dim3(kThreads), 0, st,
@@ -3000,6 +3108,12 @@ int swc_gradient(swc_handle* h, const double* x, int x_on_device, double alpha, 
     SWC_HIP(hipFreeAsync(gbuf, st));
   }
   SWC_HIP(hipStreamSynchronize(st));
+  return SWC_OK;
+}
+
+int swc_refuse_allocation(int nth) {
+  if (nth < 0) return swc_set_error(SWC_EINVAL, "swc_refuse_allocation: negative count");
+  refuse_allocation = nth;
   return SWC_OK;
 }
 
