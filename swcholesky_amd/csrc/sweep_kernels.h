@@ -8,10 +8,8 @@
 // L^T x = y: column panel by column panel, t = y - L21^T x - (later panels), then the
 // transposed triangle.  Every sum has a fixed order, so results do not depend on timing.
 
-// Bits of an entry not yet computed: a signalling NaN that arithmetic does not return
-// (it returns quiet ones); publish() keeps any result away from it.
-constexpr unsigned long long kPending = 0x7ff4a5c35a3c4b21ull;
-constexpr unsigned long long kQuietNan = 0x7ff8000000000000ull;
+#include "sweep_entries.h"
+
 constexpr uint64_t kSweepTicks = 1000000000ull;  // 10 s of the 100 MHz clock
 
 struct SweepRun {
@@ -32,25 +30,6 @@ struct SweepRun {
   int64_t ldx, ldy, ldv, ldp;
   int nrhs;
 };
-
-// Entries pass between workgroups as relaxed agent-scope atomics: each is coherent by
-// itself (written through to, and read from, memory beyond the XCDs' caches), and its own
-// readiness, so no order between entries is needed.
-__device__ inline unsigned long long load_entry(const double* p) {
-  return __hip_atomic_load(reinterpret_cast<const unsigned long long*>(p), __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ inline void publish(double* p, double v) {
-  unsigned long long b = __builtin_bit_cast(unsigned long long, v);
-  if (b == kPending) b = kQuietNan;
-  __hip_atomic_store(reinterpret_cast<unsigned long long*>(p), b, __ATOMIC_RELAXED,
-                     __HIP_MEMORY_SCOPE_AGENT);
-}
-
-// (For a later launch: a plain store.)
-__device__ inline void mark_pending(double* p) {
-  *reinterpret_cast<unsigned long long*>(p) = kPending;
-}
 
 // Called by a whole wave: true while the wait may go on.
 __device__ inline bool keep_waiting(const SweepRun& a, unsigned& spins, uint64_t& t0) {
