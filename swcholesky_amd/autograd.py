@@ -13,9 +13,13 @@ import torch
 from .api import Factor
 
 
-def _sync():
+def _sync(*tensors):
+    """Waits until the tensors hold their values: the factor works on a stream of its own, and
+    a tensor's work is on its own device's stream, whichever device is current (a host
+    tensor's, say a copy under way, on the current one's)."""
     if torch.cuda.is_available():
-        torch.cuda.current_stream().synchronize()
+        for device in {t.device if t.is_cuda else None for t in tensors}:
+            torch.cuda.current_stream(device).synchronize()
 
 
 class _LogdetQuad(torch.autograd.Function):
@@ -24,14 +28,14 @@ class _LogdetQuad(torch.autograd.Function):
         vals = values.detach().to(torch.float64).contiguous()
         rhs = b.detach().to(torch.float64).contiguous()
         dev = vals.device
-        _sync()
+        _sync(vals, rhs)
         info = factor.factor(vals if vals.is_cuda else vals.numpy())
         if info:
             raise RuntimeError(f"matrix is not positive definite (column {info - 1})")
         if rhs.is_cuda and rhs.device == dev and rhs.shape == (factor.n,):
             # solved where it is: the vectors do not travel to the host and back
             x = rhs.clone()
-            _sync()  # the solve runs on the factor's own stream
+            _sync(x)
             quad = float(torch.dot(rhs, factor.solve_device(x)))
         else:
             x = torch.from_numpy(factor.solve(rhs.cpu().numpy())).to(dev)
@@ -45,11 +49,12 @@ class _LogdetQuad(torch.autograd.Function):
     def backward(ctx, g):
         (x,) = ctx.saved_tensors
         f = ctx.factor
-        _sync()
         if x.is_cuda:
             gv = torch.empty(f.bcsc.nnz, dtype=torch.float64, device=x.device)
+            _sync(x)  # what used gv's memory before has run too
             f.gradient(x, alpha=ctx.alpha, beta=ctx.beta, out=gv)
         else:
+            _sync(x)
             gv = torch.from_numpy(f.gradient(x.numpy(), alpha=ctx.alpha, beta=ctx.beta))
         return g * gv, g * 2.0 * ctx.beta * x, None, None, None
 
