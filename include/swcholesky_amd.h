@@ -247,7 +247,8 @@ int swc_set_graphs(swc_handle* h, int on);
 /* With profiling on, every kernel launch of swc_factor is bracketed by HIP events
  * on the handle's stream (for measurement runs; adds launch gaps). */
 int swc_set_profiling(swc_handle* h, int on);
-/* out[8] = {last factor ms, last solve ms (device events), tile-kernel total ms,
+/* out[8] = {last factor ms, last solve ms (device events; from the launch that prepares
+ * the work vectors, and with an ordering brings B into it, to the last sweep), tile-kernel total ms,
  * tile-kernel launches, trsm-kernel total ms, trsm launches (profiling only),
  * tile-kernel algorithmic flops, trsm-kernel algorithmic flops}. */
 int swc_get_timings(const swc_handle* h, double* out);

@@ -2037,7 +2037,7 @@ void enqueue_solve(swc_handle* h, double* dX, int nrhs, int64_t ldx, bool marked
 }
 
 // In-place solve of L L^T X = B on device columns X (factor ordering); needs
-// ensure_work(h, nrhs).
+// ensure_work(h, nrhs).  marked: enqueue_marks has been launched, after ev[2].
 int solve_device(swc_handle* h, double* dX, int nrhs, int64_t ldx, bool marked) {
   hipStream_t st = h->stream;
   hipGraphExec_t gx = nullptr;
@@ -2059,7 +2059,7 @@ int solve_device(swc_handle* h, double* dX, int nrhs, int64_t ldx, bool marked) 
       h->sgraphs.push_back({dX, nrhs, ldx, marked, gx});
     }
   }
-  SWC_HIP(hipEventRecord(h->ev[2], st));
+  if (!marked) SWC_HIP(hipEventRecord(h->ev[2], st));
   if (gx) SWC_HIP(hipGraphLaunch(gx, st));
   else enqueue_solve(h, dX, nrhs, ldx, marked);
   SWC_HIP(hipEventRecord(h->ev[3], st));
@@ -2832,6 +2832,7 @@ int swc_solve(swc_handle* h, double* B, int nrhs, int64_t ldb, int on_device) {
                                sizeof(double) * h->n, nrhs, hipMemcpyHostToDevice, h->stream));
       src = h->dWork;
     }
+    SWC_HIP(hipEventRecord(h->ev[2], h->stream));  // the marks are part of the solve
     enqueue_marks(h, sweep_run(h, dY, nrhs, h->n, h->dY, h->dV, h->dPb), src, on_device ? ldb : h->n);
   } else if (int rc = to_factor(h, B, on_device, ldb, dY, nrhs)) {
     return rc;
