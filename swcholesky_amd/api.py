@@ -423,6 +423,9 @@ def build_plan(bcsc: BCSC, derive_sets=False, params=None, schedule=None):
             out[name] = np.zeros(int(cnt), dtype=dt)
             check(lib.swc_plan_export(h, which, ptr(out[name])))
         out["sweep_psize"] = int(sw[4])
+        most = np.zeros(1, dtype=np.int64)
+        check(lib.swc_plan_export(h, 28, ptr(most)))
+        out["sweep_one_each"] = int(most[0])
         out.update(nlevel=nlevel, nslevel=nslevel, xsize=xsize, update_flops=fl[0],
                    factor_flops=fl[1], vsize=vsize, diag_scratch=dscr, dag_level0=dag_level0,
                    dag_flops=fl[2], dag_sim_us=fl[3], lvl_sim_us=fl[4])

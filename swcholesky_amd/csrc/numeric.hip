@@ -1923,9 +1923,6 @@ int factor_device(swc_handle* h, const double* dvals) {
   return SWC_OK;
 }
 
-// Right-hand sides from which the sweeps take them 16 to an item (MFMA) instead of one.
-constexpr int kSweepGroupMin = 2;
-
 // One persistent launch of a sweep; the ticket was cleared before.
 template <bool FORWARD, int GROUP>
 void launch_sweep(swc_handle* h, const SweepRun& a) {
@@ -1948,16 +1945,16 @@ void launch_small(swc_handle* h, const SweepRun& a, int level) {
   const std::vector<int>& ls = h->plan.sweeps.lvl_small;
   const int s0 = ls[level], ns = ls[level + 1] - s0;
   // the packed ones and the others wait for nothing of the level: any order
-  const int n16 = a.nrhs == 1 ? h->plan.sweeps.lvl_small16[level] : 0, nw = ns - n16;
+  const int n16 = h->plan.sweeps.lvl_small16[level], nw = ns - n16;
   if (n16 > 0)
-    hipLaunchKernelGGL((k_sweep_small16<FORWARD>), dim3((n16 + 15) / 16), dim3(kThreads), 0, h->stream,
-                       a, s0, n16);
+    hipLaunchKernelGGL((k_sweep_small16<FORWARD>), dim3((n16 + 15) / 16, a.nrhs), dim3(kThreads), 0,
+                       h->stream, a, s0, n16);
   if (nw > 0 && a.nrhs == 1)
     hipLaunchKernelGGL((k_sweep_small<FORWARD, 1>), dim3((nw + 3) / 4, 1), dim3(kThreads), 0,
                        h->stream, a, s0 + n16, nw);
   else if (nw > 0)
     hipLaunchKernelGGL((k_sweep_small<FORWARD, 4>), dim3((nw + 3) / 4, (a.nrhs + 3) / 4),
-                       dim3(kThreads), 0, h->stream, a, s0, ns);
+                       dim3(kThreads), 0, h->stream, a, s0 + n16, nw);
 }
 
 SweepRun sweep_run(swc_handle* h, double* dX, int nrhs, int64_t ldx, double* dY, double* dV,
@@ -2000,7 +1997,7 @@ void enqueue_forward(swc_handle* h, SweepRun a, bool marked = false) {
   a.items = h->dSweepFwd;
   a.nitems = (int)W.fwd.size();
   a.ticket = h->dSweepSync;
-  if (a.nrhs < kSweepGroupMin) launch_sweep<true, 1>(h, a);
+  if (!swc::sweep_by_16(W, a.nrhs)) launch_sweep<true, 1>(h, a);
   else launch_sweep<true, 16>(h, a);
 }
 
@@ -2010,7 +2007,7 @@ void enqueue_backward(swc_handle* h, SweepRun a) {
   a.items = h->dSweepBwd;
   a.nitems = (int)W.bwd.size();
   a.ticket = h->dSweepSync + 1;
-  if (a.nrhs < kSweepGroupMin) launch_sweep<false, 1>(h, a);
+  if (!swc::sweep_by_16(W, a.nrhs)) launch_sweep<false, 1>(h, a);
   else launch_sweep<false, 16>(h, a);
   for (int l = (int)W.lvl_small.size() - 2; l >= 0; --l) launch_small<false>(h, a, l);
 }

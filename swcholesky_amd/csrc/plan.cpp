@@ -611,7 +611,7 @@ void build_plan(int n, int nsuper, const int* super, const int64_t* pi, const in
 
   // the backward partials take the place (and at most the room) that the row blocks'
   // partial sums of one solve level would
-  build_sweeps(nsuper, super, pi, px, Ls, voff.data(), (int64_t)std::max(P.max_lvl_fblk, 1) * SPW,
+  build_sweeps(nsuper, super, pi, px, Ls, voff.data(), P.gptr.data(), (int64_t)std::max(P.max_lvl_fblk, 1) * SPW,
                P.sweeps);
 
   // ---- flatten: tiles by level (stable), tasks, TRSM lists ----
@@ -1003,6 +1003,7 @@ int swc_plan_export(const swc_plan* p, int which, void* dst) {
     case 25: return cp(P.sweeps.lvl_small);
     case 26: return cp(P.sweeps.fwd);
     case 27: return cp(P.sweeps.bwd);
+    case 28: return cp(std::vector<int64_t>{P.sweeps.one_each});
     default: return swc_set_error(SWC_EINVAL, "swc_plan_export: unknown array id");
   }
 }

@@ -68,11 +68,10 @@ __device__ inline double entry_value(unsigned long long b) {
 }
 
 // Sums of this lane's list V[q][gidx[e]], e = e0, e0 + step, ... < e1, in that order, for Q
-// right-hand sides at once, eight entries of each in flight.
-template <int Q>
+// right-hand sides at once, N entries of each in flight.
+template <int Q, int N>
 __device__ inline void gather_sums(const SweepRun& a, const double* const (&V)[Q], int64_t e0,
                                    int64_t e1, int step, double (&sum)[Q]) {
-  constexpr int N = 8;
 #pragma unroll
   for (int q = 0; q < Q; ++q) sum[q] = 0.0;
   for (int64_t e = e0; __builtin_amdgcn_ballot_w64(e < e1) != 0; e += N * step) {
@@ -182,28 +181,34 @@ __device__ inline void small_forward(const SweepRun& a, const swc::SweepSmall& s
   const int64_t e0 = a.gptr[c], e1 = i < w ? a.gptr[c + 1] : e0;
 #pragma unroll
   for (int k = 0; k < 16; ++k) row[k] *= rinv;
-  double x[Q];
+  // right-hand sides past nq repeat the last one's entries; all of a supernode's are
+  // gathered and substituted together, so that their waits and chains overlap
+  double b[Q], x[Q];
+  const double* V[Q];
 #pragma unroll
   for (int q = 0; q < Q; ++q) {
-    x[q] = 0.0;
-    if (q >= nq) continue;  // uniform
-    double* X = a.X + (int64_t)(r0 + q) * a.ldx;
-    const double b = X[c];
-    // four lanes share a column's list
-    const double* V[1] = {a.V + (int64_t)(r0 + q) * a.ldv};
-    double sum[1];
-    gather_sums<1>(a, V, e0 + g, e1, 4, sum);
-    sum[0] += __shfl_xor(sum[0], 16);
-    sum[0] += __shfl_xor(sum[0], 32);
-    double t = i < w ? (b - sum[0]) * rinv : 0.0;
-#pragma unroll
-    for (int j = 0; j < 15; ++j) t = fma(-row[j], bcast(t, j), t);
-    x[q] = t;
-    if (lane < w) {
-      publish(a.Y + (int64_t)(r0 + q) * a.ldy + c, t);
-      mark_pending(X + c);  // the backward sweep's entry
-    }
+    const int64_t r = r0 + min(q, nq - 1);
+    b[q] = a.X[r * a.ldx + c];
+    V[q] = a.V + r * a.ldv;
   }
+  // four lanes share a column's list
+  gather_sums<Q, Q == 1 ? 8 : 4>(a, V, e0 + g, e1, 4, x);
+#pragma unroll
+  for (int q = 0; q < Q; ++q) {
+    x[q] += __shfl_xor(x[q], 16);
+    x[q] += __shfl_xor(x[q], 32);
+    x[q] = i < w ? (b[q] - x[q]) * rinv : 0.0;
+  }
+#pragma unroll
+  for (int j = 0; j < 15; ++j)
+#pragma unroll
+    for (int q = 0; q < Q; ++q) x[q] = fma(-row[j], bcast(x[q], j), x[q]);
+#pragma unroll
+  for (int q = 0; q < Q; ++q)
+    if (q < nq && lane < w) {
+      publish(a.Y + (int64_t)(r0 + q) * a.ldy + c, x[q]);
+      mark_pending(a.X + (int64_t)(r0 + q) * a.ldx + c);  // the backward sweep's entry
+    }
   for (int r = 0; r < m; r += 64) {
     if (r > 0) {
 #pragma unroll
@@ -295,15 +300,19 @@ __device__ inline void small_backward(const SweepRun& a, const swc::SweepSmall& 
     }
   }
   fold16<Q>(acc, lane);
+  double t[Q];
 #pragma unroll
   for (int q = 0; q < Q; ++q) {
-    const double sum = acc.v[q];
     const double y = a.Y[(int64_t)(r0 + min(q, nq - 1)) * a.ldy + c];
-    double t = i < w ? (y - sum) * rinv : 0.0;
-#pragma unroll
-    for (int j = 15; j >= 1; --j) t = fma(-col[j], bcast(t, j), t);
-    if (lane < w && q < nq) publish(a.X + (int64_t)(r0 + q) * a.ldx + c, t);
+    t[q] = i < w ? (y - acc.v[q]) * rinv : 0.0;
   }
+#pragma unroll
+  for (int j = 15; j >= 1; --j)
+#pragma unroll
+    for (int q = 0; q < Q; ++q) t[q] = fma(-col[j], bcast(t[q], j), t[q]);
+#pragma unroll
+  for (int q = 0; q < Q; ++q)
+    if (lane < w && q < nq) publish(a.X + (int64_t)(r0 + q) * a.ldx + c, t[q]);
 }
 
 // ---- one right-hand side, a workgroup of four waves per item --------------------
@@ -347,7 +356,7 @@ __device__ inline void forward_item(const SweepRun& a, const swc::SweepItem& it,
     rinv = stage_triangle<true>(D + (int64_t)it.row0 * it.ld, it.ld, it.nr, lds, wave, lane);
     const double* V[1] = {a.V};
     double sum[1];
-    gather_sums<1>(a, V, e0 + wave, e1, 4, sum);
+    gather_sums<1, 8>(a, V, e0 + wave, e1, 4, sum);
     acc = sum[0];
   }
   if (it.nq > 0) {
@@ -561,7 +570,7 @@ __device__ inline void forward_item16(const SweepRun& a, const swc::SweepItem& i
       V[q] = a.V + rhs(q) * a.ldv;
     }
     rinv = stage_triangle<true>(D + (int64_t)it.row0 * it.ld, it.ld, it.nr, lds, wave, lane);
-    if (nw > 0) gather_sums<4>(a, V, e0, e1, 1, g);
+    if (nw > 0) gather_sums<4, 8>(a, V, e0, e1, 1, g);
   }
   double f0[16], f1[16];
   Unknowns u0, u1;
@@ -738,12 +747,13 @@ k_sweep(SweepRun a, int g0, int ngroups) {
           else small_backward<1>(a, s, r0, 1, lane);
         }
       } else {
-        const int nw = min(4, nq - 4 * wave);
-        for (int i = 0; i < it.count; ++i) {
+        // four right-hand sides to a wave; waves that are left over take other supernodes
+        const int quads = (nq + 3) >> 2, side = 4 / quads;
+        const int q0 = 4 * (wave % quads);
+        for (int i = wave / quads; i < it.count && wave < quads * side; i += side) {
           const swc::SweepSmall s = a.small[it.first + i];
-          if (nw <= 0) continue;
-          if constexpr (FORWARD) small_forward<4>(a, s, r0 + 4 * wave, nw, lane);
-          else small_backward<4>(a, s, r0 + 4 * wave, nw, lane);
+          if constexpr (FORWARD) small_forward<4>(a, s, r0 + q0, min(4, nq - q0), lane);
+          else small_backward<4>(a, s, r0 + q0, min(4, nq - q0), lane);
         }
       }
     } else if constexpr (GROUP == 1) {
@@ -785,6 +795,9 @@ k_sweep_small(SweepRun a, int s0, int ns) {
 template <bool FORWARD>
 __global__ void __launch_bounds__(kThreads)
 k_sweep_small16(SweepRun a, int s0, int ns) {
+  a.X += (int64_t)blockIdx.y * a.ldx;
+  a.Y += (int64_t)blockIdx.y * a.ldy;
+  a.V += (int64_t)blockIdx.y * a.ldv;
   const int i = threadIdx.x & 15, lane = threadIdx.x & 63;
   const int k0 = (int)blockIdx.x * (kThreads / 16) + ((int)threadIdx.x >> 4);
   const bool have = k0 < ns;

@@ -22,7 +22,7 @@ std::vector<int> supernode_levels(int nsuper, const int* super, const int64_t* p
 }
 
 void build_sweeps(int nsuper, const int* super, const int64_t* pi, const int64_t* px, const int* Ls,
-                  const int64_t* voff, int64_t maxpart, SweepPlan& W) {
+                  const int64_t* voff, const int64_t* gptr, int64_t maxpart, SweepPlan& W) {
   W = SweepPlan();
   auto width = [&](int s) { return super[s + 1] - super[s]; };
   auto nrows = [&](int s) { return (int)(pi[s + 1] - pi[s]); };
@@ -197,6 +197,25 @@ void build_sweeps(int nsuper, const int* super, const int64_t* pi, const int64_t
       }
     add_small(W.bwd, l);
   }
+  // one right-hand side to an item or 16 (sweep_by_16)
+  std::vector<int64_t> steps(nsuper, 0);  // of the longest chain up to a supernode
+  std::vector<int> col2sup(nsuper ? super[nsuper] : 0);
+  int64_t bytes = 1, longest = 1;
+  for (int s = 0; s < nsuper; ++s)
+    for (int c = super[s]; c < super[s + 1]; ++c) col2sup[c] = s;
+  for (int s = 0; s < nsuper; ++s) {
+    int64_t list = 0;
+    for (int c = super[s]; c < super[s + 1]; ++c) list = std::max(list, gptr[c + 1] - gptr[c]);
+    steps[s] += np_of(s) + list / 64;
+    longest = std::max(longest, steps[s]);
+    bytes += (int64_t)sizeof(double) * width(s) * nrows(s);
+    if (nrows(s) > width(s)) {
+      int64_t& up = steps[col2sup[Ls[pi[s] + width(s)]]];
+      up = std::max(up, steps[s]);
+    }
+  }
+  const int64_t items = std::max<int64_t>(std::min<int64_t>(W.fwd.size(), longest), 1);
+  W.one_each = std::min(kStepBytes * longest / bytes, kChains * longest / items);
 }
 
 }  // namespace swc

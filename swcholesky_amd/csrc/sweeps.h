@@ -63,15 +63,30 @@ struct SweepPlan {
                                    // level l holds [lvl_small[l], lvl_small[l + 1])
   std::vector<SweepItem> fwd, bwd;
   int64_t psize = 0;               // doubles of backward partials per right-hand side
+  int64_t one_each = 1;            // most right-hand sides that go one to an item
 };
+
+// Several right-hand sides go one to an item, or 16 to an item with L read once for them.
+// The chain of an item with one is the shorter one, so that is better while the longest chain
+// is what takes the time: while the right-hand sides together read no more of L per step of it
+// (a 64-column panel, or 64 entries of a column's list of contributions, about 3 us) than comes
+// from memory meanwhile, 12 MB, and their chains, where a step is an item of its own, are no
+// more than 300, beyond which they wait for each other's places on the device.  One against
+// 16 to an item (ms): 24^3 with 16 right-hand sides 0.46 and 0.54, with 33 0.76 and 0.58; 48^3
+// with 2 0.92 and 1.35, with 8 2.04 and 1.63; 600 2D instances with 2 0.94 and 0.97, with 3 1.23
+// and 1.08; tridiagonal 20,000 in natural order with 300 8.6 and 9.5, with 400 11.5 and 9.6; an
+// arrow with a border of 30 with 2 0.93 and 4.8.
+constexpr int64_t kStepBytes = 12000000, kChains = 300;
+inline bool sweep_by_16(const SweepPlan& W, int nrhs) { return nrhs > 1 && nrhs > W.one_each; }
 
 // Level of every supernode: one above the highest of those whose rows below meet its
 // columns.  From the row lists, which say what the sweeps (and the selected inverse) read and
 // wait for; a caller's descendant sets may leave out a supernode whose rows hold only zeros.
 std::vector<int> supernode_levels(int nsuper, const int* super, const int64_t* pi, const int* Ls);
 
-// voff[s]: offset of the contribution vector of s.  maxpart: most doubles of partials.
+// voff[s]: offset of the contribution vector of s; gptr: offsets of the columns' lists of
+// contributions.  maxpart: most doubles of partials.
 void build_sweeps(int nsuper, const int* super, const int64_t* pi, const int64_t* px, const int* Ls,
-                  const int64_t* voff, int64_t maxpart, SweepPlan& W);
+                  const int64_t* voff, const int64_t* gptr, int64_t maxpart, SweepPlan& W);
 
 }  // namespace swc
