@@ -234,20 +234,22 @@ bool build_fronts(int n, int nsuper, const int* super, const int64_t* pi, const 
   std::vector<int> aptr((size_t)tbase[nsuper] + 1, 0);
   F.aents.resize((size_t)nnz);
   {
-    std::vector<int64_t> tid((size_t)nnz);
-    for (int j = 0; j < n; ++j) {
+    // the first tile of column j's panel, less its row tile
+    auto base = [&](int j) {
       const int s = col2sup[j], p = (j - super[s]) / T;
-      for (int e = A2p[j]; e < A2p[j + 1]; ++e) {
-        tid[e] = tile_id(s, p, (pos[e] - T * p) / T);
-        aptr[tid[e] + 1]++;
-      }
+      return tile_id(s, p, 0) - p;
+    };
+    for (int j = 0; j < n; ++j) {
+      int* cnt = aptr.data() + base(j) + 1;
+      for (int e = A2p[j]; e < A2p[j + 1]; ++e) cnt[pos[e] / T]++;
     }
     for (size_t i = 1; i < aptr.size(); ++i) aptr[i] += aptr[i - 1];
     std::vector<int> fill(aptr.begin(), aptr.end() - 1);
     for (int j = 0; j < n; ++j) {
-      const int s = col2sup[j], jj = j - super[s];
+      const int col = T * ((j - super[col2sup[j]]) % T);
+      int* at = fill.data() + base(j);
       for (int e = A2p[j]; e < A2p[j + 1]; ++e)
-        F.aents[fill[tid[e]]++] = {(int)(src ? src[e] : e), pos[e] % T + T * (jj % T)};
+        F.aents[at[pos[e] / T]++] = {(int)(src ? src[e] : e), pos[e] % T + col};
     }
   }
 

@@ -1618,12 +1618,19 @@ bool a2_positions(const swc_handle* h, const int* a2p, const int* a2i, std::vect
   for (int s = 0; s < h->nsuper; ++s) {
     const int* rows = h->Ls.data() + h->pi[s];
     const int len = (int)(h->pi[s + 1] - h->pi[s]);
-    for (int j = h->super[s]; j < h->super[s + 1]; ++j)
+    for (int j = h->super[s]; j < h->super[s + 1]; ++j) {
+      int k = j - h->super[s];  // row j
       for (int64_t q = a2p[j]; q < a2p[j + 1]; ++q) {
-        const int k = int(std::lower_bound(rows, rows + len, a2i[q]) - rows);
-        if (a2i[q] < j || k >= len || rows[k] != a2i[q]) return false;
+        const int v = a2i[q];
+        if (v < j) return false;
+        // the row after the last entry's, for most of a dense column, else a search
+        if (rows[k] != v && !(k + 1 < len && rows[++k] == v)) {
+          k = int(std::lower_bound(rows, rows + len, v) - rows);
+          if (k >= len || rows[k] != v) return false;
+        }
         pos[q] = k;
       }
+    }
   }
   return true;
 }
