@@ -296,7 +296,8 @@ int swc_plan_export(const swc_plan* p, int which, void* dst);
  * array 25, forward items, backward items, doubles of backward partials, byte sizes of
  * SweepSmall and SweepItem}; swc_plan_export 24 narrow supernodes, 25 offsets of the
  * leading levels that get launches of their own, 26 forward items, 27 backward items, 28 the
- * most right-hand sides that are solved one to an item instead of 16 (int64, 1). */
+ * most right-hand sides that are solved one to an item instead of 16 (int64, 1), 29 per
+ * leading level: its supernodes that are taken 16 lanes each, first in the level. */
 int swc_plan_sweep_sizes(const swc_plan* p, int64_t* sizes);
 /* Byte sizes of the exported structs {Panel, Tile, Task, SolveBlock}. */
 int swc_plan_struct_sizes(int64_t* out);

@@ -426,6 +426,8 @@ def build_plan(bcsc: BCSC, derive_sets=False, params=None, schedule=None):
         most = np.zeros(1, dtype=np.int64)
         check(lib.swc_plan_export(h, 28, ptr(most)))
         out["sweep_one_each"] = int(most[0])
+        out["sweep_lvl_small16"] = np.zeros(max(int(sw[1]) - 1, 0), dtype=np.int32)
+        check(lib.swc_plan_export(h, 29, ptr(out["sweep_lvl_small16"])))
         out.update(nlevel=nlevel, nslevel=nslevel, xsize=xsize, update_flops=fl[0],
                    factor_flops=fl[1], vsize=vsize, diag_scratch=dscr, dag_level0=dag_level0,
                    dag_flops=fl[2], dag_sim_us=fl[3], lvl_sim_us=fl[4])
