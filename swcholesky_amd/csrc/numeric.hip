@@ -1167,22 +1167,27 @@ struct HostRecord {
   int info;       // of the factor
   double norm;    // ||A||_inf
   double logdet;  // sum of log L_jj
-  double pad;
+  HostRecord* next;  // of the free ones
 };
 std::mutex g_record_mu;
-std::vector<HostRecord*> g_record_free;
+HostRecord* g_record_free = nullptr;
 
+// Free records are linked through themselves: handles come and go without an allocation
+// that could fail.
 HostRecord* take_record() {
   std::lock_guard<std::mutex> lock(g_record_mu);
-  if (g_record_free.empty()) {
+  if (!g_record_free) {
     constexpr int kRecords = 256;
     HostRecord* block = nullptr;
     if (hipHostMalloc((void**)&block, kRecords * sizeof(HostRecord), hipHostMallocPortable) != hipSuccess)
       return nullptr;
-    for (int i = 0; i < kRecords; ++i) g_record_free.push_back(block + i);
+    for (int i = 0; i < kRecords; ++i) {
+      block[i].next = g_record_free;
+      g_record_free = block + i;
+    }
   }
-  HostRecord* r = g_record_free.back();
-  g_record_free.pop_back();
+  HostRecord* r = g_record_free;
+  g_record_free = r->next;
   *r = HostRecord{};
   return r;
 }
@@ -1190,7 +1195,8 @@ HostRecord* take_record() {
 void give_record(HostRecord* r) {
   if (!r) return;
   std::lock_guard<std::mutex> lock(g_record_mu);
-  g_record_free.push_back(r);
+  r->next = g_record_free;
+  g_record_free = r;
 }
 
 // Per-device address of `scratch`, looked up once per device with that device
@@ -2248,15 +2254,10 @@ int refine_device(swc_handle* h, const double* Bt, double* Xt, int nrhs, double 
 
 // ---- adjoint ---------------------------------------------------------------
 
-int selinv_setup(swc_handle* h) {
-  if (h->dNodes) return SWC_OK;
+int build_selinv_arrays(swc_handle* h) {
   hipStream_t st = h->stream;
   h->sel = swc::build_selinv(h->n, h->nsuper, h->super.data(), h->pi.data(), h->px.data(), h->Ls.data());
   swc::SelPlan& S = h->sel;
-  int rc = SWC_OK;
-  if (!rc) rc = upload(&h->dSelRuns, S.runs.data(), S.runs.size(), h);
-  if (!rc) rc = upload(&h->dSelJrun, S.jrun.data(), S.jrun.size(), h);
-  if (!rc) rc = upload(&h->dSelRel, (const int*)nullptr, (size_t)S.nrel, h);
   // the item lists, one after the other
   std::vector<swc::SelItem> items;
   const std::vector<swc::SelItem>* lists[kSelLists] = {&S.diag,   &S.cols,  &S.u,   &S.gather,
@@ -2268,6 +2269,9 @@ int selinv_setup(swc_handle* h) {
     h->sel_items[q] = items.size();
     items.insert(items.end(), lists[q]->begin(), lists[q]->end());
   }
+  int rc = upload(&h->dSelRuns, S.runs.data(), S.runs.size(), h);
+  if (!rc) rc = upload(&h->dSelJrun, S.jrun.data(), S.jrun.size(), h);
+  if (!rc) rc = upload(&h->dSelRel, (const int*)nullptr, (size_t)S.nrel, h);
   if (!rc) rc = upload(&h->dSelItems, items.data(), items.size(), h);
   if (!rc) rc = upload(&h->dSelM, (const double*)nullptr, (size_t)S.msize, h);
   if (!rc) rc = upload(&h->dArena, (const double*)nullptr, (size_t)S.zsize, h);
@@ -2299,6 +2303,15 @@ int selinv_setup(swc_handle* h) {
   std::vector<swc::SelRun>().swap(S.runs);
   std::vector<int>().swap(S.jrun);
   return SWC_OK;
+}
+
+int selinv_setup(swc_handle* h) {
+  if (h->dNodes) return SWC_OK;
+  try {
+    return build_selinv_arrays(h);
+  } catch (const std::bad_alloc&) {  // thrown before anything is uploaded
+    return swc_set_error(SWC_ENOMEM, "selected inverse: out of host memory");
+  }
 }
 
 int selinv_device(swc_handle* h) {

@@ -1003,7 +1003,7 @@ int swc_plan_export(const swc_plan* p, int which, void* dst) {
     case 25: return cp(P.sweeps.lvl_small);
     case 26: return cp(P.sweeps.fwd);
     case 27: return cp(P.sweeps.bwd);
-    case 28: return cp(std::vector<int64_t>{P.sweeps.one_each});
+    case 28: std::memcpy(dst, &P.sweeps.one_each, sizeof(int64_t)); return SWC_OK;
     case 29: return cp(P.sweeps.lvl_small16);
     default: return swc_set_error(SWC_EINVAL, "swc_plan_export: unknown array id");
   }
