@@ -2632,12 +2632,8 @@ int upload_structure(swc_handle* h, int n, const int* blockSet, int supNo, const
   }
   h->uploading = false;
   h->zvalid = false;
-  (void)hipFree(h->dZ);
-  (void)hipFree(h->dArena);
-  (void)hipFree(h->dNodes);
-  h->dZ = nullptr;
-  h->dArena = nullptr;
-  h->dNodes = nullptr;
+  free_all({(void**)&h->dZ, (void**)&h->dArena, (void**)&h->dNodes, (void**)&h->dSelM, (void**)&h->dSelRuns,
+            (void**)&h->dSelJrun, (void**)&h->dSelRel, (void**)&h->dSelItems});
   const hipError_t se = hipStreamSynchronize(st);
   if (rc) {
     (void)hipFree(h->dL);
