@@ -99,6 +99,23 @@ static void order_for_xcds(std::vector<FrontTile>& tiles) {
   tiles.swap(out);
 }
 
+// The update matrices take about as much as L (1.2 times at most on grids, meshes and dense
+// matrices), but far more where many small supernodes lie below a wide border: every one of
+// them then writes the border's whole triangle and the border reads it (16 bytes an entry at
+// 4.3 TB/s), while the left-looking plan runs through the border's descendants one after
+// another, about 3 us each, but takes longer over the border itself.  Factorizations, left-
+// looking and multifrontal (ms), of single columns below a border: 300 x 600 (arena 199 times
+// L) 1.34 and 1.18, 300 x 1000 (230) 1.74 and 2.07, 300 x 2000 (260) 3.2 and 4.0, 1000 x 1000
+// (499) 3.6 and 5.8, 1500 x 2000 (30 GB) 5.7 and 13.8, but 30 x 4000 (29) 4.7 and 3.4, and by the
+// longer chain 3000 x 600 (443) 8.8 and 7.2.  More than 4 times L takes 32 GiB at most.
+static bool arena_pays(int64_t usize, int64_t xsize, int nsuper, const int* prunePtr) {
+  if (usize <= 4 * xsize) return true;
+  if (usize > (int64_t)1 << 32) return false;
+  int most = 0;  // descendants of one supernode
+  for (int s = 0; s < nsuper; ++s) most = std::max(most, prunePtr[s + 1] - prunePtr[s]);
+  return usize <= 200 * xsize || 16.0 * (double)usize / 4.3e6 <= 3.0 * most;
+}
+
 bool build_fronts(int n, int nsuper, const int* super, const int64_t* pi, const int64_t* px,
                   int64_t xsize, const int* Ls, const int* prunePtr, const int* pruneSet,
                   const int* A2p, const int64_t* src, const int* pos, int rlb, FrontPlan& F) {
@@ -217,6 +234,7 @@ bool build_fronts(int n, int nsuper, const int* super, const int64_t* pi, const 
       }
     }
     F.usize = ar.size() ? ubase - xsize + ar.size() : 0;
+    if (!arena_pays(F.usize, xsize, nsuper, prunePtr)) return false;
   }
 
   // ---- entries of A by tile of L: tile (panel p, row tile t) of s ----

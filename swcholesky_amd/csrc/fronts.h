@@ -105,7 +105,8 @@ struct FrontPlan {
 // value of each A2 entry (null: its own index).  Returns false (plan untouched
 // beyond use) for a structure whose supernodes do not pass their rows up one tree:
 // a supernode's rows below its columns that are not all rows of the supernode owning
-// the first of them, or descendant sets that are not those of the row lists.
+// the first of them, or descendant sets that are not those of the row lists; and for one
+// whose update matrices are not worth their size.
 bool build_fronts(int n, int nsuper, const int* super, const int64_t* pi, const int64_t* px,
                   int64_t xsize, const int* Ls, const int* prunePtr, const int* pruneSet,
                   const int* A2p, const int64_t* src, const int* pos, int rlb, FrontPlan& F);
