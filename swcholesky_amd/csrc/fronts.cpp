@@ -276,27 +276,43 @@ bool build_fronts(int n, int nsuper, const int* super, const int64_t* pi, const 
     int lo;
     uint64_t mask;
   };
-  std::vector<std::vector<Cut>> cl, cu;  // per child: by 64 rows from row 0, and from row w
-  auto cut = [&](int c, int from, int len, std::vector<Cut>& out) {
-    const int* r = rel.data() + roff[c];
-    const int m = (int)(roff[c + 1] - roff[c]);
-    out.clear();
-    int e = int(std::lower_bound(r, r + m, from) - r);
-    for (int x = 0; x < len; x += T) {
-      Cut k{e, 0};
-      for (; e < m && r[e] < from + x + T; ++e) k.mask |= 1ull << (r[e] - from - x);
-      out.push_back(k);
+  // The children's rows by blocks of 64 of the supernode's rows from one row on, and the
+  // children with rows in each block: a supernode of thousands of small children, each in
+  // few of its blocks, has a tile ask only those (the upload of a tree of 30,000 points whose
+  // root has 3434 columns: 15.0 ms with every child asked, 4.7 now).
+  struct Cuts {
+    std::vector<std::vector<Cut>> of;     // by child
+    std::vector<std::vector<int>> child;  // by block, ascending
+  };
+  Cuts cl, cu;  // from row 0, and from row w
+  auto cut = [&](int s, int from, int len, Cuts& out) {
+    const int nch = nchild[s + 1] - nchild[s], nb = (len + T - 1) / T;
+    if ((int)out.of.size() < nch) out.of.resize(nch);
+    if ((int)out.child.size() < nb) out.child.resize(nb);
+    for (int b = 0; b < nb; ++b) out.child[b].clear();
+    for (int k = 0; k < nch; ++k) {
+      const int c = child[nchild[s] + k];
+      const int* r = rel.data() + roff[c];
+      const int m = (int)(roff[c + 1] - roff[c]);
+      std::vector<Cut>& of = out.of[k];
+      of.assign(nb, Cut{});
+      for (int e = int(std::lower_bound(r, r + m, from) - r); e < m;) {
+        const int b = (r[e] - from) / T;
+        of[b].lo = e;
+        for (; e < m && r[e] < from + T * (b + 1); ++e) of[b].mask |= 1ull << (r[e] - from - T * b);
+        out.child[b].push_back(k);
+      }
     }
   };
-  auto add_gathers = [&](int s, const std::vector<std::vector<Cut>>& rc, int I,
-                         const std::vector<std::vector<Cut>>& cc, int J, int nc) {
+  auto add_gathers = [&](int s, const Cuts& cuts, int I, int J, int nc) {
     const uint64_t keep = nc >= 64 ? ~0ull : (1ull << nc) - 1;
-    for (int q = nchild[s]; q < nchild[s + 1]; ++q) {
-      const int c = child[q], k = q - nchild[s];
-      const uint64_t rm = rc[k][I].mask, cm = cc[k][J].mask & keep;
+    for (int k : cuts.child[cuts.child[I].size() <= cuts.child[J].size() ? I : J]) {
+      const int c = child[nchild[s] + k];
+      const Cut &rc = cuts.of[k][I], &cc = cuts.of[k][J];
+      const uint64_t rm = rc.mask, cm = cc.mask & keep;
       if (!rm || !cm) continue;
       const int ld = ldu_of(c);
-      F.gathers.push_back({ux[c] + rc[k][I].lo + (int64_t)cc[k][J].lo * ld, ld, 0, rm, cm});
+      F.gathers.push_back({ux[c] + rc.lo + (int64_t)cc.lo * ld, ld, 0, rm, cm});
     }
   };
 
@@ -311,15 +327,8 @@ bool build_fronts(int n, int nsuper, const int* super, const int64_t* pi, const 
     for (int bi = lvl_s[l0]; bi < lvl_s[l0 + 1]; ++bi) {
       const int s = by_start[bi], w = width(s), R = nrows(s), m = R - w, np = npan(s);
       const int nt = (R + T - 1) / T, ntu = (m + T - 1) / T, ldu = ldu_of(s);
-      const int nch = nchild[s + 1] - nchild[s];
-      if ((int)cl.size() < nch) {
-        cl.resize(nch);
-        cu.resize(nch);
-      }
-      for (int k = 0; k < nch; ++k) {
-        cut(child[nchild[s] + k], 0, R, cl[k]);
-        cut(child[nchild[s] + k], w, m, cu[k]);
-      }
+      cut(s, 0, R, cl);
+      cut(s, w, m, cu);
       F.npanel += np;
       const double dw = w, dm = m;
       F.factor_flops += dw * dw * dw / 3.0 + dm * dw * dw;
@@ -332,7 +341,7 @@ bool build_fronts(int n, int nsuper, const int* super, const int64_t* pi, const 
         f.ldu = ldu;
         f.c0 = super[s];
         f.g0 = (int)F.gathers.size();
-        add_gathers(s, cl, 0, cl, 0, 64);
+        add_gathers(s, cl, 0, 0, 64);
         f.g1 = (int)F.gathers.size();
         f.a0 = aptr[tbase[s]];
         f.a1 = aptr[tbase[s] + 1];
@@ -357,7 +366,7 @@ bool build_fronts(int n, int nsuper, const int* super, const int64_t* pi, const 
           f.first = p == 0;
           if (f.first) {
             f.g0 = (int)F.gathers.size();
-            add_gathers(s, cl, t, cl, 0, nc);
+            add_gathers(s, cl, t, 0, nc);
             f.g1 = (int)F.gathers.size();
             f.a0 = aptr[tile_id(s, 0, t)];
             f.a1 = aptr[tile_id(s, 0, t) + 1];
@@ -398,7 +407,7 @@ bool build_fronts(int n, int nsuper, const int* super, const int64_t* pi, const 
             u.first = first && (q < b1 ? p == 0 : true);
             if (u.first) {
               u.g0 = (int)F.gathers.size();
-              add_gathers(s, cl, q + t, cl, q, u.nc);
+              add_gathers(s, cl, q + t, q, u.nc);
               u.g1 = (int)F.gathers.size();
               u.a0 = aptr[tile_id(s, q, t)];
               u.a1 = aptr[tile_id(s, q, t) + 1];
@@ -425,7 +434,7 @@ bool build_fronts(int n, int nsuper, const int* super, const int64_t* pi, const 
               u.first = q0 == 0;
               if (u.first) {
                 u.g0 = (int)F.gathers.size();
-                add_gathers(s, cu, a, cu, b, u.nc);
+                add_gathers(s, cu, a, b, u.nc);
                 u.g1 = (int)F.gathers.size();
               }
               (p + 1 == np ? L.uc : L.ud).push_back(u);
