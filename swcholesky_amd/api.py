@@ -446,7 +446,7 @@ SMALL_FRONT_DT = np.dtype([("vbase", np.int64), ("ubase", np.int64)] + [(k, np.i
     "R", "w", "ldu", "c0", "g0", "g1", "a0", "a1")])
 FRONT_TILE_DT = np.dtype([("vbase", np.int64), ("asrc", np.int64), ("bsrc", np.int64)] + [
     (k, np.int32) for k in ("ld", "sld", "k", "nr", "nc", "diag", "first", "upd", "g0", "g1", "a0",
-                            "a1", "slot", "pad")])
+                            "a1", "slot", "row")])
 
 
 def build_fronts(bcsc: BCSC, rlb=8):

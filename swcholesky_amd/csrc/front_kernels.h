@@ -679,8 +679,8 @@ k_front_factor(double* __restrict__ L, const swc::SmallFront* __restrict__ small
   }
 }
 
-// LDS (doubles) of k_front_factor: the widest panel's working matrix (16-column blocks)
-// and multipliers, the one-wave items' buffers, the deferred tiles' entries of A.  A
+// LDS (doubles) of k_front_factor: the widest panel's working matrix (16-column blocks),
+// the one-wave items' buffers, the deferred tiles' entries of A, whichever takes most.  A
 // level of panels of at most 32 columns takes half of what 64 columns need, so twice
 // the workgroups fit on a CU.
 inline size_t front_factor_lds(int nwave_items, int widest, int ndefer) {

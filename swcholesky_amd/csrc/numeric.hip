@@ -670,7 +670,7 @@ __device__ inline d4 lds_block_update(const double* __restrict__ W, d4 acc, int 
 // pivot of column j + 1 is formed from column j's raw entries beside the others' updates,
 // and nothing is selected: a pivot that is not a positive finite number is noticed at the
 // end and the sweep done again with a test in every column (SAFE).  Cycles a column, the
-// kernel's own: multipliers through LDS and selects 328, by readlane 377, this 200.
+// kernel's own: multipliers through LDS and selects 328, by readlane 377, this 238.
 // Returns 1 + the first column whose pivot is not positive, else 0; such a pivot
 // continues as 1, so no NaNs spread.
 template <bool SAFE>
@@ -1482,11 +1482,10 @@ struct swc_handle {
   int64_t* dVmap = nullptr;
   double* dAf = nullptr;
   int64_t nnz_full = 0;
-  // small device scalars written by captured launch sequences ([0] ||A||_inf,
-  // [1] logdet): allocated with the structure and never moved while a graph
-  // that writes them exists
-  double* dScal = nullptr;   // refinement scalars, sized by ensure_work (eager launches only)
-  double* dNormPart = nullptr;  // kRedBlocks partial maxima of ||A||_inf
+  double* dScal = nullptr;   // reductions and coefficients of the refinement, 4 * work_cols
+                             // (eager launches only)
+  double* dNormPart = nullptr;  // kSetupBlocks partial maxima of ||A||_inf, kRedBlocks partial
+                                // sums of the log determinant
   double* dPart = nullptr;   // reduction partials, kRedBlocks * work_cols
   double* dRef = nullptr;    // refinement vectors, 5 * n * work_cols
   double normA = 0;
@@ -1680,7 +1679,7 @@ int ensure_work(swc_handle* h, int cols) {
   SWC_HIP(device_malloc(h, (void**)&h->dPart, sizeof(double) * (size_t)kRedBlocks * cols));
   (void)hipFree(h->dScal);
   h->dScal = nullptr;
-  SWC_HIP(device_malloc(h, (void**)&h->dScal, sizeof(double) * (size_t)(64 + 4 * cols)));
+  SWC_HIP(device_malloc(h, (void**)&h->dScal, sizeof(double) * (size_t)(4 * cols)));
   SWC_HIP(device_malloc(h, (void**)&h->dRef, sizeof(double) * (size_t)5 * h->n * cols));
   SWC_HIP(device_malloc(h, (void**)&h->dWork, sizeof(double) * (size_t)h->n * cols));
   SWC_HIP(device_malloc(h, (void**)&h->dV, sizeof(double) * (size_t)std::max<int64_t>(P.vsize, 1) * cols));
@@ -1706,7 +1705,9 @@ void enqueue_fronts(swc_handle* h, bool profile) {
     const int f0 = F.lvl_f[l], nf = F.lvl_f[l + 1] - f0, nn = F.lvl_fn[l], nw = nf - nn;
     const int nd = l > 0 && !profile ? F.lvl_ud[l - 1] : 0;
     if (pe) (void)hipEventRecord(pe[1], st);
-    // many one-wave items keep their own launch, where more of them fit on a CU
+    // many one-wave items keep their own launch, where more of them fit on a CU.  From 512 /
+    // 2048 / 8192 items on (ms): 500^2 GMRF 0.996 / 0.970 / 0.968, 600 2D instances 0.775 / 0.755 /
+    // 0.746, larger grids the same; in between, so that LDS does not bound larger levels
     const bool lean = nw + nd == 0 || ns + nn > 2048;
     if (lean && ns + nn > 0)
       hipLaunchKernelGGL(k_front_narrow<MODE>, dim3(ns + nn), dim3(64), 0, st, h->dL, sm, s0, ns,
@@ -2127,10 +2128,10 @@ void launch_reduce(swc_handle* h, const double* X, const double* Y, int ncol, in
   hipLaunchKernelGGL(k_reduce_partial, dim3(kRedBlocks, ncol), dim3(kThreads), 0, st, X, Y, h->n,
                      (int64_t)h->n, op, h->dPart);
   hipLaunchKernelGGL(k_reduce_final, dim3(ncol), dim3(kThreads), 0, st, (const double*)h->dPart, op,
-                     h->dScal + 64 + (int64_t)slot * ncol);
+                     h->dScal + (int64_t)slot * ncol);
 }
 int fetch_reduced(swc_handle* h, int ncol, int nslots, double* out) {
-  SWC_HIP(hipMemcpyAsync(out, h->dScal + 64, sizeof(double) * ncol * nslots, hipMemcpyDeviceToHost, h->stream));
+  SWC_HIP(hipMemcpyAsync(out, h->dScal, sizeof(double) * ncol * nslots, hipMemcpyDeviceToHost, h->stream));
   return sync_stream(h);
 }
 int reduce_cols(swc_handle* h, const double* X, const double* Y, int ncol, int op, double* out) {
@@ -2150,7 +2151,7 @@ void launch_csr_mv(swc_handle* h, const double* X, const double* B, double* Y, i
 }
 
 int put_coeffs(swc_handle* h, const std::vector<double>& c) {
-  SWC_HIP(hipMemcpyAsync(h->dScal + 64 + 2 * c.size(), c.data(), sizeof(double) * c.size(),
+  SWC_HIP(hipMemcpyAsync(h->dScal + 2 * c.size(), c.data(), sizeof(double) * c.size(),
                          hipMemcpyHostToDevice, h->stream));
   return SWC_OK;
 }
@@ -2204,7 +2205,7 @@ int refine_device(swc_handle* h, const double* Bt, double* Xt, int nrhs, double 
       for (int c = 0; c < nrhs; ++c) co[c] = conv[c] ? 0.0 : 1.0;
       if (int rc = put_coeffs(h, co)) return rc;
       hipLaunchKernelGGL(k_axpy_cols, g, dim3(kThreads), 0, st, Xt, (const double*)Z,
-                         (const double*)(h->dScal + 64 + 2 * nrhs), n, ld);
+                         (const double*)(h->dScal + 2 * nrhs), n, ld);
       if (int rc = evaluate(R, done)) return rc;
     }
   } else {
@@ -2224,11 +2225,11 @@ int refine_device(swc_handle* h, const double* Bt, double* Xt, int nrhs, double 
       }
       if (int rc = put_coeffs(h, co)) return rc;
       hipLaunchKernelGGL(k_axpy_cols, g, dim3(kThreads), 0, st, Xt, (const double*)Pv,
-                         (const double*)(h->dScal + 64 + 2 * nrhs), n, ld);
+                         (const double*)(h->dScal + 2 * nrhs), n, ld);
       for (int c = 0; c < nrhs; ++c) co[c] = -co[c];
       if (int rc = put_coeffs(h, co)) return rc;
       hipLaunchKernelGGL(k_axpy_cols, g, dim3(kThreads), 0, st, R, (const double*)Z,
-                         (const double*)(h->dScal + 64 + 2 * nrhs), n, ld);
+                         (const double*)(h->dScal + 2 * nrhs), n, ld);
       if (int rc = evaluate(Z, done)) return rc;  // true residual, for eta only
       if (done) {
         ++it;
@@ -2244,7 +2245,7 @@ int refine_device(swc_handle* h, const double* Bt, double* Xt, int nrhs, double 
       }
       if (int rc = put_coeffs(h, co)) return rc;
       hipLaunchKernelGGL(k_xpby_cols, g, dim3(kThreads), 0, st, Pv, (const double*)Z,
-                         (const double*)(h->dScal + 64 + 2 * nrhs), n, ld);
+                         (const double*)(h->dScal + 2 * nrhs), n, ld);
     }
   }
   SWC_HIP(hipGetLastError());
@@ -2863,7 +2864,7 @@ int swc_solve(swc_handle* h, double* B, int nrhs, int64_t ldb, int on_device) {
 // allocation, no captured graph (eager launches on the handle's stream).
 // Layout, each part starting on a 256-byte boundary: the permuted right-hand
 // sides (n x nrhs), the forward solutions (n x nrhs), the contribution vectors
-// (max(vsize,1) x nrhs, cleared by the forward sweep's fill kernel) and the
+// (max(vsize,1) x nrhs, marked pending before the forward sweep) and the
 // backward partials.  Calls on one GPU share the array: overlapping calls race.
 int swc_solve_noalloc(swc_handle* h, double* B, int nrhs, int64_t ldb) {
   if (int rc = check_handle(h)) return rc;

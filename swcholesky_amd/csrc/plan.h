@@ -152,8 +152,10 @@ struct Plan {
   std::vector<int> panel_level;     // per panel
   std::vector<int> lvl_panels;      // nlevel+1 offsets into panel_order
   std::vector<int> panel_order;     // panels grouped by level
-  // solves: solve panels of up to SPW columns of one supernode, with their own
-  // level structure (nslevel levels)
+  // solves by levels: solve panels of up to SPW columns of one supernode, with their own
+  // level structure (nslevel levels).  The library solves by the sweeps' work lists; it takes
+  // of these only gptr, gidx and max_lvl_fblk (which bounds the sweeps' partials), and gives
+  // the others out with the plan.
   std::vector<Panel> spanels;
   std::vector<int> sp_order;        // solve panels grouped by level
   std::vector<int> lvl_sp;          // nslevel+1

@@ -5,9 +5,10 @@
 //   T = L11^{-1},  U = L21 T               from L alone
 //   Z21 = -Z(R,R) U                        Z(R,R) read from the ancestors' Z
 //   Z11 = T^T T - U^T Z21
-// T and U wait for no other supernode: they are made for a whole chunk of levels in three
-// launches (64 x 64 diagonal blocks, columns of blocks below them, U), so that only the
-// last two steps follow the chain of levels, three launches a level.  A chunk holds as many
+// T and U wait for no other supernode: they are made for a whole chunk of levels in four
+// launches (64 x 64 diagonal blocks, those of at most 16 columns, columns of blocks below
+// them, U), so that only the last two steps follow the chain of levels, three launches a
+// level.  A chunk holds as many
 // levels as fit kSelChunk values (its T and U are read again soon, from the caches), and at
 // least one.  One thread per entry in four launches a level before, with every entry's own
 // serial sum, -> this: 3.9 -> 0.54 ms on a 256^2 GMRF (65,536 unknowns, 13 levels; 0.16 ms
